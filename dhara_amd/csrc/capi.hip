@@ -1279,12 +1279,15 @@ int dhara_create(const dhara_grid* grid, const dhara_params* params, dhara_ctx**
     g2.cy = params->dt / (grid->dy * grid->dy);
     for (int e = 0; e < 2; ++e) {
         c->tile[e] = default_tile(g);
-        c->cg1_tile[e] = dh::TileCfg{32, 8, g.nz, 0};
+        c->cg1_tile[e] = dh::TileCfg{32, 8, dh::cg1_default_planes(g), 0};
         if (dh::cg1_blocks(g, c->cg1_tile[e]) > dh::kMaxBlocks) c->cg1_tile[e].grid = dh::kMaxBlocks;   // blocks loop
         const int tkind = (e == 0 && mixed_column(params)) ? 2 : 0;
         for (const TuneEntry& te : g_tune_table) {
             if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, tkind}) c->tile[e] = te.cfg;
-            if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, 1}) c->cg1_tile[e] = te.cfg;
+            if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, 1}) {
+                c->cg1_tile[e] = te.cfg;
+                c->cg1_set[e] = true;
+            }
         }
     }
 
@@ -1588,6 +1591,7 @@ int dhara_set_krylov_tile(dhara_ctx* c, int32_t elem_bytes, int32_t tx, int32_t 
     if (!dh::cg1_tile_supported(t)) return set_err(c, DHARA_E_ARG, "unsupported one-kernel PCG tile");
     if (dh::cg1_blocks(c->g, t) > dh::kMaxBlocks) return set_err(c, DHARA_E_ARG, "tile grid too large; raise kc or cap the grid");
     c->cg1_tile[elem_bytes == 8 ? 0 : 1] = t;
+    c->cg1_set[elem_bytes == 8 ? 0 : 1] = true;
     return DHARA_OK;
 }
 
@@ -1774,6 +1778,7 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
                         if (us < 0.97f * best_t || best_t >= 1e29f) { best_t = us; best_cfg = t; }
                     }
             c->cg1_tile[e] = best_cfg;
+            c->cg1_set[e] = true;
             best[e] = best_t;
             remember_tile(TuneKey{c->g.nx, c->g.ny, c->g.nz, e == 0 ? 8 : 4, 1}, best_cfg);
         }

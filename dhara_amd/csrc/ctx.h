@@ -84,8 +84,9 @@ struct dhara_ctx {
     std::vector<void*> allocs;
     // SpMV tile shapes: [0] FP64 solves, [1] FP32 inner solves (tx = 0: untiled kernel)
     dh::TileCfg tile[2] = {{32, 8, 0}, {32, 8, 0}};
-    // one-kernel PCG tiles: [0] FP64, [1] FP32 (kc = 0: whole columns)
+    // one-kernel PCG tiles: [0] FP64, [1] FP32; cg1_set: chosen by the caller or the autotuner
     dh::TileCfg cg1_tile[2] = {{32, 8, 0, 0}, {32, 8, 0, 0}};
+    bool cg1_set[2] = {false, false};
     // kernel profiling (dhara_profile_enable)
     bool prof = false;
     std::vector<hipEvent_t> ev;

@@ -94,6 +94,7 @@ struct dhara_ensemble {
     void* a_c1 = nullptr;
     std::vector<dh::Cg1Args<double>> h_c1d;
     std::vector<dh::Cg1Args<float>> h_c1f;
+    bool c1_full = false;           // the members' whole-column tiles fill the chip together
     int kc_div = 0;                 // dhara_ensemble_autotune: planes per tile = ceil(nz / kc_div); 0: member's tile
     // column-preconditioned PCG (every member with DHARA_PRECOND_COLUMN): the column kernel's
     // block maps, one per register-array size (nz <= 16, 32, 64)
@@ -436,12 +437,17 @@ int upload_k3(dhara_ensemble* e)
                     : upload_args(e, (dh::KrylovArgs<double>*)e->a_k3, e->h_k3d);
 }
 
-// Tiles of a member in the batched one-kernel PCG: 32 x 8 columns; the member's own (tuned)
-// planes per tile when its tile is 32 x 8, whole columns otherwise.
+// Tiles of a member in the batched one-kernel PCG: 32 x 8 columns; the member's own planes per
+// tile when its tile is 32 x 8, whole columns otherwise.  The default planes of a small member split
+// its columns to fill the chip; members that fill it together (e->c1_full: more whole-column tiles
+// than kCg1FillTiles) keep whole columns unless their tile was set or tuned, since the chunks' halo
+// planes would then only add work (the solve is the same to rounding: other partial sums).
 void c1_tiles(const dhara_ensemble* e, const dhara_ctx* c, int& kc, int& ntx, int& nty, int& nkz, int kc_div)
 {
-    const dh::TileCfg& t = c->cg1_tile[e->mixed ? 1 : 0];
+    const int pr = e->mixed ? 1 : 0;
+    const dh::TileCfg& t = c->cg1_tile[pr];
     if (kc_div > 0) kc = (c->g.nz + kc_div - 1) / kc_div;
+    else if (e->c1_full && !c->cg1_set[pr]) kc = c->g.nz;
     else kc = (t.tx == dh::kCg1BatchTx && t.ty == dh::kCg1BatchTy && t.kc > 0) ? std::min(t.kc, c->g.nz) : c->g.nz;
     ntx = (c->g.nx + dh::kCg1BatchTx - 1) / dh::kCg1BatchTx;
     nty = (c->g.ny + dh::kCg1BatchTy - 1) / dh::kCg1BatchTy;
@@ -978,6 +984,11 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
     if (e->one) {
         e->h_c1d.resize(n);
         e->h_c1f.resize(n);
+        long tiles = 0;
+        for (dhara_ctx* c : e->mem)
+            tiles += (long)((c->g.nx + dh::kCg1BatchTx - 1) / dh::kCg1BatchTx) *
+                     ((c->g.ny + dh::kCg1BatchTy - 1) / dh::kCg1BatchTy);
+        e->c1_full = tiles > dh::kCg1FillTiles;
         // room for the finest policy the autotuner tries (a third of the planes per tile)
         std::vector<dh::BlkMap> finest;
         if (c1_map(e, 0, mc1) || c1_map(e, 3, finest)) {

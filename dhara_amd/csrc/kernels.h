@@ -341,6 +341,8 @@ void launch_pcg3_spmv_tiled_f32(hipStream_t s, const Geo& g, const TileCfg& t, c
 // (partials [rz, rr, bb, rr64] of the assembly or of a reliable update).
 bool cg1_tile_supported(const TileCfg& t);
 int cg1_blocks(const Geo& g, const TileCfg& t);
+constexpr int kCg1FillTiles = 400;   // blocks up to which a small surface's columns are split
+int cg1_default_planes(const Geo& g);   // planes per block of the 32 x 8 tile when none is set or tuned
 void launch_cg1_f64(hipStream_t s, const Geo& g, const TileCfg& t, const double* K, const double* D,
                     const double* r_in, double* r_out, const double* p_in, double* p_out, double* x,
                     const SolveCtl& sc, const LaunchEv& ev = LaunchEv{});

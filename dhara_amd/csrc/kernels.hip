@@ -3115,6 +3115,21 @@ bool cg1_tile_supported(const TileCfg& t)
             (t.tx == 64 && t.ty == 8));
 }
 
+// A block marches its planes one after the other (two barriers each), so a surface of few tiles
+// is bound by that chain, not by its bytes: 20 to 30 planes of a 32 x 32 or 64 x 64 surface took
+// 25 to 34 us a launch.  Splitting the columns adds four halo planes of arithmetic per chunk,
+// which idle CUs do for nothing: chunks are taken as long as the blocks stay at about 1.5 per CU.
+// Jacobi-PCG steps with whole columns / with this rule (FP64, MI355X, us): 32x32x20 1455 / 979,
+// 64x64x30 3470 / 1975, 150x97x40 2274 / 1632, 200x200x30 2813 / 2590; beyond the line (300x300x20,
+// 380 tiles) whole columns are within 2 % of the best split, and at 400x400x30 every split loses
+// (9689 whole, 10475 with two chunks).
+int cg1_default_planes(const Geo& g)
+{
+    const int nt = ((g.nx + 31) / 32) * ((g.ny + 7) / 8);
+    const int nkz = std::max(1, std::min(g.nz, kCg1FillTiles / nt));
+    return (g.nz + nkz - 1) / nkz;
+}
+
 int cg1_blocks(const Geo& g, const TileCfg& t)
 {
     const int nb = tile_blocks(g, t);
