@@ -231,15 +231,14 @@ def aa_pass_bytes(npass, depth, mixed):
     return total
 
 
-def mg_single_block_only(nx, ny, cells=3400):
+def mg_single_block_only(nx, ny, threads=1024):
     """True when every level of the overland multigrid fits the single-block kernel (the
     surface has no tiled level), as the library decides it."""
-    total = 0
-    while True:
-        total += nx * ny
-        if nx == 1 and ny == 1:
-            return total <= cells
+    total = 0   # the coarser levels' cells: one thread for each, down to the exact level
+    while nx * ny > 64:
         nx, ny = (nx + 1) // 2, (ny + 1) // 2
+        total += nx * ny
+    return total <= threads
 
 
 def counted_bytes(stats, n3, n2, mixed, olf_mg=True, one_kernel=False, column=False, aa_depth=0,

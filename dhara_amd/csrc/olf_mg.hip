@@ -14,12 +14,19 @@
 //     update multiplies by the reciprocal of the diagonal (held in LDS);
 //   * coarse correction scaled by 1.2 (over-correction for piecewise-constant interpolation;
 //     1.5 took 17 % more iterations on the 400 x 400 coupled run, 1.1 to 1.25 about the same);
+//   * a thread owns a 2 x 2 aggregate (two red and two black cells): its operator, right-hand
+//     side and iterate stay in registers and only the iterate is exchanged, through four LDS
+//     planes (one per cell of the aggregate, so every access is stride 1);
+//   * the first red half-sweep from x = 0 needs no neighbours, the residual of the cells smoothed
+//     last is zero, so the restriction sums the red residuals alone, and the post-smoothing starts
+//     by overwriting the black cells, so only red x and y are carried between the kernels;
 //   * large levels: one tiled kernel down (smooth, residual, restrict) and one up (prolong,
-//     smooth) per level; a tile of T x T cells works in LDS with a halo of 5 (down) or 4 (up)
-//     cells recomputed redundantly, so four half-sweeps need no grid-wide synchronisation and
-//     the tile interior equals a global sweep exactly;
-//   * the coarsest levels (as many as fit 3400 cells in LDS: 50 x 50 down to 7 x 7 on a 400 x 400
-//     surface): the rest of the V-cycle in one single-block kernel.
+//     smooth) per level; a tile of 32 x 32 cells works with a halo of 4 cells (6 where A z is
+//     formed too) recomputed redundantly, so the half-sweeps need no grid-wide synchronisation
+//     and the tile interior equals a global sweep exactly;
+//   * the coarsest levels (as many as give one aggregate to each of 1024 threads: 50 x 50 down to
+//     7 x 7 on a 400 x 400 surface): the rest of the V-cycle in one single-block kernel, every
+//     level's aggregates on threads of their own.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -27,21 +34,21 @@
 namespace dh {
 
 constexpr double kMgOver = 1.2;   // coarse-correction scaling
-constexpr int kMgT = 28;          // tile edge of the large-level kernels (even)
-constexpr int kMgHd = 5;          // halo: 4 half-sweeps + the residual
-constexpr int kMgHu = 4;          // halo: 4 half-sweeps
-constexpr int kMgThreads = 1024;   // one pass of a 38 x 38 tile's half-sweep per block
-constexpr int kMgCoarseCells = 3400;   // LDS capacity of the single-block kernel, in cells of its levels
+constexpr int kMgT = 32;          // tile edge of the large-level kernels (even)
+constexpr int kMgHalo = 2;        // halo in aggregates: the three half-sweeps after the first and the residual
+constexpr int kMgHaloA = 3;       // the four half-sweeps after the prolongation, and A z
+constexpr int kMgThreads = 1024;   // threads of the single-block kernels
+constexpr int kMgExactChunks = kMgThreads / kMgExactCells;   // threads per row of the exact solve
 
-// The first level handled by the single-block kernel: the finest whose cells, together with
-// those of every coarser level down to le, fit in its LDS (50 x 50 ... 7 x 7 on a 400 x 400
-// surface).  Host and device use the same rule.
+// The first level handled by the single-block kernel: the finest whose aggregates and those of
+// every coarser level (an aggregate of a level is a cell of the next) fit its threads (50 x 50 ...
+// 7 x 7 on a 400 x 400 surface).  Host and device use the same rule.
 __host__ __device__ inline int mg_first_single_block(const MgHier& h)
 {
-    int l = h.le, cells = h.lv[l].nx * h.lv[l].ny;
-    while (l > 0 && cells + h.lv[l - 1].nx * h.lv[l - 1].ny <= kMgCoarseCells) {
+    int l = h.le, aggs = 0;
+    while (l > 0 && aggs + h.lv[l].nx * h.lv[l].ny <= kMgThreads) {
+        aggs += h.lv[l].nx * h.lv[l].ny;
         --l;
-        cells += h.lv[l].nx * h.lv[l].ny;
     }
     return l;
 }
@@ -98,24 +105,160 @@ __global__ __launch_bounds__(kBlock) void k_mg_coarsen(MgLevel F, MgLevel C)
     mg_coarsen_cells(F, C, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
-// One red-black Gauss-Seidel half-sweep over an LDS grid of w x w cells (global origin ox, oy),
-// updating the cells of `color` ((gi + gj) & 1) that are not on the LDS border.
-// Threads are dealt only the cells of the colour: row lj holds the interior cells li = p, p+2, ...
-// with p fixed by the colour, so a half-sweep of a 38 x 38 tile is one pass of 648 threads.
-__device__ __forceinline__ void lds_half_sweep(int w, int ox, int oy, int color, const double* sb, const double* sdi,
-                                               const double* swe, const double* swn, double* sx)
+// A thread's 2 x 2 aggregate of a level: cells 0 (i, j), 1 (i + 1, j), 2 (i, j + 1), 3 (i + 1, j + 1)
+// with i and j even, so 0 and 3 are red and 1 and 2 black.  Cells outside the level have d = 1,
+// b = 0 and no couplings.
+struct MgAgg {
+    double b[4], d[4], di[4], x[4];
+    double h0, h1, v0, v1;                   // couplings inside: 0-1, 2-3, 0-2, 1-3
+    double w0, w2, e1, e3, s0, s1, n2, n3;   // and out: west, east, south (j - 1), north
+};
+
+struct MgIn {
+    bool c[4];   // cell inside the level
+};
+
+__device__ __forceinline__ MgIn agg_in(const MgLevel& L, int gi, int gj)
 {
-    const int hw = (w - 1) / 2;   // colour cells per interior row, at most
-    for (int u = threadIdx.x; u < (w - 2) * hw; u += blockDim.x) {
-        const int lj = 1 + u / hw;
-        const int p = ((color - ox - oy - lj) & 1) ? 1 : 2;   // first interior li of the colour
-        const int li = p + 2 * (u - (lj - 1) * hw);
-        if (li > w - 2) continue;
-        const int t = lj * w + li;
-        const double s = sb[t] + swe[t] * sx[t + 1] + swe[t - 1] * sx[t - 1] + swn[t] * sx[t + w] + swn[t - w] * sx[t - w];
-        sx[t] = s * sdi[t];
+    MgIn in;
+    in.c[0] = gi >= 0 && gj >= 0 && gi < L.nx && gj < L.ny;
+    in.c[1] = in.c[0] && gi + 1 < L.nx;
+    in.c[2] = in.c[0] && gj + 1 < L.ny;
+    in.c[3] = in.c[1] && in.c[2];
+    return in;
+}
+
+__device__ __forceinline__ double ld_if(bool in, const double* __restrict__ p, int g, double other)
+{
+    return in ? p[g] : other;
+}
+
+// The operator of the aggregate at (gi, gj).
+__device__ __forceinline__ void agg_load(const MgLevel& L, int gi, int gj, const MgIn& in, MgAgg& a)
+{
+    const int nx = L.nx, g = gj * nx + gi;
+    a.d[0] = ld_if(in.c[0], L.d, g, 1.0);
+    a.d[1] = ld_if(in.c[1], L.d, g + 1, 1.0);
+    a.d[2] = ld_if(in.c[2], L.d, g + nx, 1.0);
+    a.d[3] = ld_if(in.c[3], L.d, g + nx + 1, 1.0);
+    const bool we = gi > 0, ea = gi + 2 < nx, so = gj > 0, no = gj + 2 < L.ny;
+    a.h0 = ld_if(in.c[1], L.we, g, 0.0);
+    a.h1 = ld_if(in.c[3], L.we, g + nx, 0.0);
+    a.w0 = ld_if(in.c[0] && we, L.we, g - 1, 0.0);
+    a.w2 = ld_if(in.c[2] && we, L.we, g + nx - 1, 0.0);
+    a.e1 = ld_if(in.c[1] && ea, L.we, g + 1, 0.0);
+    a.e3 = ld_if(in.c[3] && ea, L.we, g + nx + 1, 0.0);
+    a.v0 = ld_if(in.c[2], L.wn, g, 0.0);
+    a.v1 = ld_if(in.c[3], L.wn, g + 1, 0.0);
+    a.s0 = ld_if(in.c[0] && so, L.wn, g - nx, 0.0);
+    a.s1 = ld_if(in.c[1] && so, L.wn, g - nx + 1, 0.0);
+    a.n2 = ld_if(in.c[2] && no, L.wn, g + nx, 0.0);
+    a.n3 = ld_if(in.c[3] && no, L.wn, g + nx + 1, 0.0);
+}
+
+__device__ __forceinline__ void agg_invert(MgAgg& a)
+{
+#pragma unroll
+    for (int c = 0; c < 4; ++c) a.di[c] = 1.0 / a.d[c];
+}
+
+// The LDS planes of a grid of aggregates: plane c holds cell c of every aggregate, with a border of
+// zeros; `q` is this thread's slot of plane 0, `pitch` the slots of a row, `plane` of a plane.
+struct MgPlanes {
+    double* q;
+    int pitch, plane;
+    __device__ __forceinline__ double at(int c, int off) const { return q[c * plane + off]; }
+    __device__ __forceinline__ void put(int c, double v) const { q[c * plane] = v; }
+};
+
+// Zeros around the planes (the border slots that a neighbour read can reach), by the edge threads.
+__device__ __forceinline__ void planes_border(const MgPlanes& s, bool west, bool east, bool south, bool north)
+{
+    if (west) { s.q[s.plane - 1] = 0.0; s.q[3 * s.plane - 1] = 0.0; }
+    if (east) { s.q[1] = 0.0; s.q[2 * s.plane + 1] = 0.0; }
+    if (south) { s.q[2 * s.plane - s.pitch] = 0.0; s.q[3 * s.plane - s.pitch] = 0.0; }
+    if (north) { s.q[s.pitch] = 0.0; s.q[s.plane + s.pitch] = 0.0; }
+}
+
+// Sums of the couplings times the neighbours' values of the red cells (0, 3) and of the black ones (1, 2).
+__device__ __forceinline__ void red_sums(const MgAgg& a, const MgPlanes& s, double& t0, double& t3)
+{
+    t0 = a.h0 * a.x[1] + a.w0 * s.at(1, -1) + a.v0 * a.x[2] + a.s0 * s.at(2, -s.pitch);
+    t3 = a.e3 * s.at(2, 1) + a.h1 * a.x[2] + a.n3 * s.at(1, s.pitch) + a.v1 * a.x[1];
+}
+__device__ __forceinline__ void black_sums(const MgAgg& a, const MgPlanes& s, double& t1, double& t2)
+{
+    t1 = a.e1 * s.at(0, 1) + a.h0 * a.x[0] + a.v1 * a.x[3] + a.s1 * s.at(3, -s.pitch);
+    t2 = a.h1 * a.x[3] + a.w2 * s.at(3, -1) + a.n2 * s.at(0, s.pitch) + a.v0 * a.x[0];
+}
+__device__ __forceinline__ void put_red(const MgAgg& a, const MgPlanes& s)
+{
+    s.put(0, a.x[0]);
+    s.put(3, a.x[3]);
+}
+__device__ __forceinline__ void red_sweep(MgAgg& a, const MgPlanes& s)
+{
+    double t0, t3;
+    red_sums(a, s, t0, t3);
+    a.x[0] = (a.b[0] + t0) * a.di[0];
+    a.x[3] = (a.b[3] + t3) * a.di[3];
+    put_red(a, s);
+}
+__device__ __forceinline__ void black_sweep(MgAgg& a, const MgPlanes& s)
+{
+    double t1, t2;
+    black_sums(a, s, t1, t2);
+    a.x[1] = (a.b[1] + t1) * a.di[1];
+    a.x[2] = (a.b[2] + t2) * a.di[2];
+    s.put(1, a.x[1]);
+    s.put(2, a.x[2]);
+}
+
+// Two forward sweeps from x = 0 and the restricted residual of the aggregate (returned).  Every
+// thread of the block calls it; `on`: this thread has an aggregate.
+__device__ __forceinline__ double agg_down(MgAgg& a, const MgPlanes& s, bool on)
+{
+    double u0 = 0.0, u3 = 0.0, t0 = 0.0, t3 = 0.0;
+    if (on) {
+        a.x[0] = a.b[0] * a.di[0];
+        a.x[3] = a.b[3] * a.di[3];
+        put_red(a, s);
     }
     __syncthreads();
+    if (on) black_sweep(a, s);
+    __syncthreads();
+    if (on) {
+        red_sums(a, s, u0, u3);
+        a.x[0] = (a.b[0] + u0) * a.di[0];
+        a.x[3] = (a.b[3] + u3) * a.di[3];
+        put_red(a, s);
+    }
+    __syncthreads();
+    if (on) black_sweep(a, s);
+    __syncthreads();
+    if (on) red_sums(a, s, t0, t3);   // d x + couplings changed by t - u since the red cells were set
+    return (t0 - u0) + (t3 - u3);
+}
+
+// Two backward sweeps on the prolonged iterate (its red cells, in a.x[0] and a.x[3]); the last
+// red values are in the registers and, if put, in the planes (no barrier after them).
+__device__ __forceinline__ void agg_up(MgAgg& a, const MgPlanes& s, bool on, bool put)
+{
+    if (on) put_red(a, s);
+    __syncthreads();
+    if (on) black_sweep(a, s);
+    __syncthreads();
+    if (on) red_sweep(a, s);
+    __syncthreads();
+    if (on) black_sweep(a, s);
+    __syncthreads();
+    if (on) {
+        double t0, t3;
+        red_sums(a, s, t0, t3);
+        a.x[0] = (a.b[0] + t0) * a.di[0];
+        a.x[3] = (a.b[3] + t3) * a.di[3];
+        if (put) put_red(a, s);
+    }
 }
 
 // Start of iteration sc.it of the single-reduction CG (MgCg1): the stopping test on (r, r)
@@ -175,267 +318,289 @@ __device__ __forceinline__ bool olf_cg1_begin(const SolveCtl& sc, double& alpha,
     return true;
 }
 
-// Down: x = 2 forward RBGS sweeps from 0 on b, r = b - A x, b_coarse = P^T r.  On level 0,
-// MODE 1: b is the CG residual after this iteration's update, done here (see MgUpd); MODE 2:
-// the same for the single-reduction CG (see MgCg1).
-template <int MODE>
-__global__ __launch_bounds__(kMgThreads) void k_mg_down(MgHier h, int l, const PcgState* st, MgUpd u, MgCg1 v)
+// Threads of a tile of kMgT x kMgT cells with a halo of H aggregates.
+constexpr int mg_tile_threads(int H)
 {
-    static_assert(kMgT * kMgT <= kMgThreads, "one tile-interior cell per thread");
-    constexpr int W = kMgT + 2 * kMgHd;
-    __shared__ double sb[W * W], sd[W * W], sdi[W * W], swe[W * W], swn[W * W], sx[W * W], sr[kMgT * kMgT];
-    __shared__ double ss[MODE == 2 ? W * W : 1];
-    const MgLevel L = h.lv[l], C = h.lv[l + 1];
-    const int ntx = (L.nx + kMgT - 1) / kMgT;
-    const int gx0 = (blockIdx.x % ntx) * kMgT, gy0 = (blockIdx.x / ntx) * kMgT;
-    const int ox = gx0 - kMgHd, oy = gy0 - kMgHd;
-    const bool first = v.sc.it == 0;
-    // MODE 2: z, p, x of this thread's tile-interior cell, loaded before the partial sums are
-    // reduced (they do not depend on alpha and beta), so that their latency overlaps it
-    int gint = -1;
-    double zi = 0.0, pold = 0.0, xi = 0.0;
-    if constexpr (MODE == 2) {
-        const int tj = threadIdx.x / kMgT, ti = threadIdx.x - tj * kMgT;
-        if (threadIdx.x < kMgT * kMgT && gx0 + ti < L.nx && gy0 + tj < L.ny) {
-            gint = (gy0 + tj) * L.nx + gx0 + ti;
-            zi = v.z[gint];
-            pold = first ? 0.0 : v.p[gint];
-            xi = v.x[gint];
-        }
-    }
-    double alpha = 0.0, beta = 0.0;
-    if constexpr (MODE == 1) {
-        if (!update_begin(u.sc, alpha, blockIdx.x)) return;
-    } else if constexpr (MODE == 2) {
-        if (!olf_cg1_begin(v.sc, alpha, beta, blockIdx.x)) return;
-    } else if (st && st->done) {
-        return;
-    }
-    for (int t = threadIdx.x; t < W * W; t += blockDim.x) {
-        const int lj = t / W, li = t - lj * W;
-        const int gi = ox + li, gj = oy + lj;
-        const bool in = gi >= 0 && gj >= 0 && gi < L.nx && gj < L.ny;
-        const int g = gj * L.nx + gi;
-        if constexpr (MODE == 1) {
-            sb[t] = in ? u.r_old[g] - alpha * u.q[g] : 0.0;
-        } else if constexpr (MODE == 2) {
-            const double wg = in ? v.w[g] : 0.0, sg = (in && !first) ? v.s_old[g] : 0.0;
-            const double rg = in ? v.r_old[g] : 0.0;
-            const double sn = wg + beta * sg;
-            ss[t] = sn;
-            sb[t] = rg - alpha * sn;
-        } else {
-            sb[t] = in ? L.b[g] : 0.0;
-        }
-        const double dg = in ? L.d[g] : 1.0;
-        sd[t] = dg;
-        sdi[t] = 1.0 / dg;
-        swe[t] = in ? L.we[g] : 0.0;
-        swn[t] = in ? L.wn[g] : 0.0;
-        sx[t] = 0.0;
-    }
-    __syncthreads();
-    lds_half_sweep(W, ox, oy, 0, sb, sdi, swe, swn, sx);
-    lds_half_sweep(W, ox, oy, 1, sb, sdi, swe, swn, sx);
-    lds_half_sweep(W, ox, oy, 0, sb, sdi, swe, swn, sx);
-    lds_half_sweep(W, ox, oy, 1, sb, sdi, swe, swn, sx);
-    // residual of the tile interior (exact: the halo absorbed the four half-sweeps)
-    for (int t = threadIdx.x; t < kMgT * kMgT; t += blockDim.x) {
-        const int tj = t / kMgT, ti = t - tj * kMgT;
-        const int q = (tj + kMgHd) * W + ti + kMgHd;
-        const double Ax = sd[q] * sx[q] - swe[q] * sx[q + 1] - swe[q - 1] * sx[q - 1] - swn[q] * sx[q + W] -
-                          swn[q - W] * sx[q - W];
-        const int gi = gx0 + ti, gj = gy0 + tj;
-        if (gi < L.nx && gj < L.ny) {
-            const int g = gj * L.nx + gi;
-            L.x[g] = sx[q];
-            if constexpr (MODE == 1) {
-                u.r_new[g] = sb[q];
-                u.x[g] = u.x[g] + alpha * u.p[g];
-            }
-            if constexpr (MODE == 2) {   // g == gint: the cell whose z, p, x this thread loaded
-                v.s_new[g] = ss[q];
-                v.r_new[g] = sb[q];
-                const double pn = zi + beta * pold;
-                v.p[g] = pn;
-                v.x[g] = xi + alpha * pn;
-            }
-        }
-        sr[t] = sb[q] - Ax;
-    }
-    __syncthreads();
-    constexpr int TC = kMgT / 2;
-    for (int t = threadIdx.x; t < TC * TC; t += blockDim.x) {
-        const int cj = t / TC, ci = t - cj * TC;
-        const int I = gx0 / 2 + ci, J = gy0 / 2 + cj;
-        if (I >= C.nx || J >= C.ny) continue;
-        const int q = 2 * cj * kMgT + 2 * ci;
-        C.b[J * C.nx + I] = sr[q] + sr[q + 1] + sr[q + kMgT] + sr[q + kMgT + 1];
-    }
+    const int n = (kMgT / 2 + 2 * H) * (kMgT / 2 + 2 * H);
+    return (n + kWave - 1) / kWave * kWave;
 }
 
-// Up: x = x_l + 1.2 P y_{l+1}, 2 backward RBGS sweeps, written to out.  On level 0 also the
-// partial sums (b, x), (b, b), (bb_src, bb_src), (b, b) the CG kernels read; CG1 (level 0 of
-// the single-reduction CG): a halo of 5, so that x is exact one cell beyond the tile and
-// w = A x can be formed on the tile, written to w_out, and the partial sums
-// (b, x), (b, b), (w, x), (bb_src, bb_src).
+// The aggregate of this thread in the tile of this block.
+template <int H>
+struct MgTile {
+    static constexpr int NB = kMgT / 2 + 2 * H, P = NB + 2;
+    int I, J, gi, gj;
+    bool on, interior;
+    __device__ __forceinline__ explicit MgTile(const MgLevel& L)
+    {
+        const int ntx = (L.nx + kMgT - 1) / kMgT;
+        const int t = threadIdx.x;
+        J = t / NB;
+        I = t - J * NB;
+        on = t < NB * NB;
+        gi = (int)(blockIdx.x % ntx) * kMgT + 2 * (I - H);
+        gj = (int)(blockIdx.x / ntx) * kMgT + 2 * (J - H);
+        interior = on && I >= H && J >= H && I < NB - H && J < NB - H;
+    }
+    __device__ __forceinline__ MgPlanes planes(double* sx) const
+    {
+        return MgPlanes{sx + (on ? (J + 1) * P + I + 1 : P + 1), P, P * P};
+    }
+    __device__ __forceinline__ void border(const MgPlanes& s) const
+    {
+        if (on) planes_border(s, I == 0, I == NB - 1, J == 0, J == NB - 1);
+    }
+};
+
+// Down: x = 2 forward RBGS sweeps from 0 on b, b_coarse = P^T (b - A x).  CG1 (level 0 of the
+// single-reduction CG): b is the CG residual after this iteration's update, done here (see MgCg1).
+// Every load is issued before the partial sums are reduced, so that their latency overlaps it.
+// Bound by latency (one tile is ~8 us of dependent steps, a surface of 400 x 400 169 tiles on 256
+// CUs).  With the operator in LDS (ten LDS reads per cell and half-sweep, 80 KB a tile) these
+// kernels took 12.9 us (CG1) and 5.7 us.
 template <bool CG1>
-__global__ __launch_bounds__(kMgThreads) void k_mg_up(MgHier h, int l, double* out, const PcgState* st,
-                                                      double* part, const double* bb_src, double* w_out)
+__global__ __launch_bounds__(mg_tile_threads(kMgHalo)) void k_mg_down(MgLevel L, MgLevel C, const PcgState* st, MgCg1 v)
 {
-    if (st && st->done) return;
-    constexpr int HU = CG1 ? kMgHu + 1 : kMgHu;
-    constexpr int W = kMgT + 2 * HU;
-    __shared__ double sb[W * W], sdi[W * W], swe[W * W], swn[W * W], sx[W * W];
-    __shared__ double sd[CG1 ? W * W : 1];
-    const MgLevel L = h.lv[l], C = h.lv[l + 1];
-    const int ntx = (L.nx + kMgT - 1) / kMgT;
-    const int gx0 = (blockIdx.x % ntx) * kMgT, gy0 = (blockIdx.x / ntx) * kMgT;
-    const int ox = gx0 - HU, oy = gy0 - HU;
-    for (int t = threadIdx.x; t < W * W; t += blockDim.x) {
-        const int lj = t / W, li = t - lj * W;
-        const int gi = ox + li, gj = oy + lj;
-        const bool in = gi >= 0 && gj >= 0 && gi < L.nx && gj < L.ny;
-        const int g = gj * L.nx + gi;
-        sb[t] = in ? L.b[g] : 0.0;
-        const double dg = in ? L.d[g] : 1.0;
-        if constexpr (CG1) sd[t] = dg;
-        sdi[t] = 1.0 / dg;
-        swe[t] = in ? L.we[g] : 0.0;
-        swn[t] = in ? L.wn[g] : 0.0;
-        sx[t] = in ? L.x[g] + kMgOver * C.y[(gj >> 1) * C.nx + (gi >> 1)] : 0.0;
-    }
-    __syncthreads();
-    lds_half_sweep(W, ox, oy, 1, sb, sdi, swe, swn, sx);
-    lds_half_sweep(W, ox, oy, 0, sb, sdi, swe, swn, sx);
-    lds_half_sweep(W, ox, oy, 1, sb, sdi, swe, swn, sx);
-    lds_half_sweep(W, ox, oy, 0, sb, sdi, swe, swn, sx);
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int t = threadIdx.x; t < kMgT * kMgT; t += blockDim.x) {
-        const int tj = t / kMgT, ti = t - tj * kMgT;
-        const int gi = gx0 + ti, gj = gy0 + tj;
-        if (gi >= L.nx || gj >= L.ny) continue;
-        const int q = (tj + HU) * W + ti + HU;
-        const int g = gj * L.nx + gi;
-        out[g] = sx[q];
-        acc[0] += sb[q] * sx[q];
-        acc[1] += sb[q] * sb[q];
-        if constexpr (CG1) {
-            const double wq = sd[q] * sx[q] - swe[q] * sx[q + 1] - swe[q - 1] * sx[q - 1] - swn[q] * sx[q + W] -
-                              swn[q - W] * sx[q - W];
-            w_out[g] = wq;
-            acc[2] += wq * sx[q];
-            if (bb_src) acc[3] += bb_src[g] * bb_src[g];
-        } else if (bb_src) {
-            acc[2] += bb_src[g] * bb_src[g];
+    using Tile = MgTile<kMgHalo>;
+    __shared__ double sx[4 * Tile::P * Tile::P];
+    const Tile t(L);
+    const MgPlanes s = t.planes(sx);
+    const MgIn in = agg_in(L, t.gi, t.gj);
+    const bool on = t.on;
+    const int nx = L.nx, g = t.gj * nx + t.gi;
+    const int off[4] = {0, 1, nx, nx + 1};
+    MgAgg a;
+    if constexpr (CG1) {
+        const bool first = v.sc.it == 0;
+        double w[4], so[4], ro[4], z[4], p[4], x[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bool i = on && in.c[c], ii = t.interior && in.c[c];
+            w[c] = ld_if(i, v.w, g + off[c], 0.0);
+            so[c] = ld_if(i && !first, v.s_old, g + off[c], 0.0);
+            ro[c] = ld_if(i, v.r_old, g + off[c], 0.0);
+            z[c] = ld_if(ii, v.z, g + off[c], 0.0);
+            p[c] = ld_if(ii && !first, v.p, g + off[c], 0.0);
+            x[c] = ld_if(ii, v.x, g + off[c], 0.0);
         }
+        if (on) agg_load(L, t.gi, t.gj, in, a);
+        double alpha, beta;
+        if (!olf_cg1_begin(v.sc, alpha, beta, blockIdx.x)) return;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const double sn = w[c] + beta * so[c];
+            a.b[c] = ro[c] - alpha * sn;
+            if (t.interior && in.c[c]) {
+                v.s_new[g + off[c]] = sn;
+                v.r_new[g + off[c]] = a.b[c];
+                const double pn = z[c] + beta * p[c];
+                v.p[g + off[c]] = pn;
+                v.x[g + off[c]] = x[c] + alpha * pn;
+            }
+        }
+    } else {
+        const int done = st ? st->done : 0;
+        if (on) {
+            agg_load(L, t.gi, t.gj, in, a);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) a.b[c] = ld_if(in.c[c], L.b, g + off[c], 0.0);
+        }
+        if (done) return;
     }
-    if constexpr (!CG1) acc[3] = acc[1];
-    if (part) block_partials<4, false>(acc, part);
+    if (on) agg_invert(a);
+    t.border(s);
+    const double rc = agg_down(a, s, on);
+    if (t.interior && in.c[0]) {
+        C.b[(t.gj >> 1) * C.nx + (t.gi >> 1)] = rc;
+        L.x[g] = a.x[0];
+        if (in.c[3]) L.x[g + nx + 1] = a.x[3];
+    }
 }
 
-// The V-cycle from level lc (<= 32 x 32) down to 1 x 1 and back, in one block, in LDS:
-// reads b of level lc, writes y of level lc (and on level 0 the CG partial sums).  The levels
-// are small, so a phase is one pass of a few waves followed by a barrier, and its cost is the
-// latency of one cell: the four neighbour terms read their LDS operands without branches (a
-// neighbour outside the level reads the cell itself with a zero weight) so that the reads issue
-// together, the smoother multiplies by the reciprocal diagonal kept in LDS, and the restriction
-// sums the residuals of each aggregate as it computes them.
+// Up: x = x_l + 1.2 P y_{l+1}, 2 backward RBGS sweeps, written to out.  CG1 (level 0 of the
+// single-reduction CG): also w = A x on the tile, written to w_out, and the partial sums
+// (b, x), (b, b), (w, x), (bb_src, bb_src).  (With the operator in LDS: 9.9 us (CG1) and 5.4 us.)
+template <bool CG1>
+__global__ __launch_bounds__(mg_tile_threads(CG1 ? kMgHaloA : kMgHalo)) void k_mg_up(MgLevel L, MgLevel C, double* out,
+                                                                                  const PcgState* st, double* part,
+                                                                                  const double* bb_src, double* w_out)
+{
+    using Tile = MgTile<CG1 ? kMgHaloA : kMgHalo>;
+    __shared__ double sx[4 * Tile::P * Tile::P];
+    const int done = st ? st->done : 0;
+    const Tile t(L);
+    const MgPlanes s = t.planes(sx);
+    const MgIn in = agg_in(L, t.gi, t.gj);
+    const bool on = t.on;
+    const int nx = L.nx, g = t.gj * nx + t.gi;
+    const int off[4] = {0, 1, nx, nx + 1};
+    MgAgg a;
+    double bs[4] = {0.0, 0.0, 0.0, 0.0};
+    if (on) {
+        const double yc = kMgOver * ld_if(in.c[0], C.y, (t.gj >> 1) * C.nx + (t.gi >> 1), 0.0);
+        a.x[0] = ld_if(in.c[0], L.x, g, 0.0);
+        a.x[3] = ld_if(in.c[3], L.x, g + nx + 1, 0.0);
+        agg_load(L, t.gi, t.gj, in, a);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a.b[c] = ld_if(in.c[c], L.b, g + off[c], 0.0);
+        if (CG1 && bb_src) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) bs[c] = ld_if(t.interior && in.c[c], bb_src, g + off[c], 0.0);
+        }
+        if (in.c[0]) a.x[0] += yc;
+        if (in.c[3]) a.x[3] += yc;
+    }
+    if (done) return;
+    if (on) agg_invert(a);
+    t.border(s);
+    agg_up(a, s, on, CG1);
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if constexpr (CG1) __syncthreads();
+    if (t.interior) {
+        double w[4] = {0.0, 0.0, 0.0, 0.0};
+        if constexpr (CG1) {
+            red_sums(a, s, w[0], w[3]);
+            black_sums(a, s, w[1], w[2]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (!in.c[c]) continue;
+            out[g + off[c]] = a.x[c];
+            if constexpr (CG1) {
+                const double wq = a.d[c] * a.x[c] - w[c];
+                w_out[g + off[c]] = wq;
+                acc[0] += a.b[c] * a.x[c];
+                acc[1] += a.b[c] * a.b[c];
+                acc[2] += wq * a.x[c];
+                acc[3] += bs[c] * bs[c];
+            }
+        }
+    }
+    if constexpr (CG1) block_partials<4, false>(acc, part);
+}
+
+// The V-cycle from level lc down to le and back, in one block: reads b of level lc, writes y of
+// level lc (and on level 0 the CG partial sums).  A thread owns one aggregate of one of the levels
+// lc .. le - 1 (all operators are loaded at once at the start), so a phase is a barrier and at most
+// one aggregate's update; the residual sum of thread t's aggregate is cell t of the array of the
+// coarser levels' right-hand sides.  The exact level is solved with the dense inverse, each of its
+// rows by kMgExactChunks threads.  A chain of ~36 dependent phases of ~100 ns; with the operators in
+// LDS and the levels' cells dealt anew to the threads in every phase it took 26 us (50 x 50 down to
+// 7 x 7).
 __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgState* st, double* part,
                                                           const double* bb_src)
 {
-    if (st && st->done) return;
-    __shared__ double sb[kMgCoarseCells], sx[kMgCoarseCells], sdi[kMgCoarseCells], swe[kMgCoarseCells],
-        swn[kMgCoarseCells];
-    const int lc = mg_coarse_first(h);
-    const int nl = h.le + 1;   // levels lc .. le; le is solved exactly
-    int off[kMgMaxLevels];
+    constexpr int NE = kMgExactCells, NC = kMgExactChunks, PER = NE / NC;
+    // a level of bx x by aggregates takes 4 (bx + 2) (by + 2) slots; a row of n aggregates is the worst
+    __shared__ double sx[12 * kMgThreads + 24 * kMgMaxLevels];
+    __shared__ double sb[kMgThreads], ye[NE], pp[NC][NE];
+    const int done = st ? st->done : 0;
+    const int le = h.le, lc = mg_coarse_first(h);
+    const int tid = threadIdx.x;
+    int lv = -1, base = 0, xo = 0;        // this thread's level, its first thread and first slot
+    int own_b = 0;                        // where this level's right-hand side starts in sb
+    for (int l = lc, b0 = 0, x0 = 0, prev = 0; l < le; ++l) {
+        const int n = h.lv[l + 1].nx * h.lv[l + 1].ny;
+        if (tid >= b0 && tid < b0 + n) {
+            lv = l;
+            base = b0;
+            xo = x0;
+            own_b = prev;
+        }
+        prev = b0;
+        b0 += n;
+        x0 += 4 * (h.lv[l + 1].nx + 2) * (h.lv[l + 1].ny + 2);
+    }
+    const bool has = lv >= 0;
+    const int ll = has ? lv : le;
+    const MgLevel L = h.lv[ll];
+    const int bx = has ? h.lv[ll + 1].nx : 1, by = has ? h.lv[ll + 1].ny : 1;
+    const int J = has ? (tid - base) / bx : 0, I = has ? (tid - base) - J * bx : 0;
+    const MgPlanes s{sx + xo + (J + 1) * (bx + 2) + I + 1, bx + 2, (bx + 2) * (by + 2)};
+    const MgIn in = agg_in(L, 2 * I, 2 * J);
+    const int nx = L.nx, g = 2 * J * nx + 2 * I;
+    const int off[4] = {0, 1, nx, nx + 1};
+    MgAgg a;
+    if (has) {
+        agg_load(L, 2 * I, 2 * J, in, a);
+        if (lv == lc) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) a.b[c] = ld_if(in.c[c], L.b, g + off[c], 0.0);
+        }
+    }
+    const int ne = h.lv[le].nx * h.lv[le].ny;
+    const int er = tid & (NE - 1), ec = tid / NE;   // exact level: row and chunk of this thread
+    double inv[PER];   // the inverse is symmetric: its columns are read for coalesced rows
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        inv[i] = (er < ne && ec * PER + i < ne) ? h.inv[(ec * PER + i) * ne + er] : 0.0;
+    if (lc == le && tid < ne) sb[tid] = L.b[tid];
+    if (done) return;
+    if (has) {
+        agg_invert(a);
+        planes_border(s, I == 0, I == bx - 1, J == 0, J == by - 1);
+    }
+    int eb = 0;   // the exact level's right-hand side in sb
+    for (int l = lc; l < le; ++l) {
+        const bool on = lv == l;
+        if (on && l > lc) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) a.b[c] = in.c[c] ? sb[own_b + g + off[c]] : 0.0;
+        }
+        const double rc = agg_down(a, s, on);
+        if (on) sb[tid] = rc;
+        if (l > lc) eb += h.lv[l].nx * h.lv[l].ny;
+        __syncthreads();
+    }
+    if (lc == le) __syncthreads();
     {
-        int o = 0;
-        for (int l = lc; l < nl; ++l) { off[l] = o; o += h.lv[l].nx * h.lv[l].ny; }
-    }
-    for (int l = lc; l < nl; ++l) {
-        const MgLevel& L = h.lv[l];
-        const int n = L.nx * L.ny;
-        for (int t = threadIdx.x; t < n; t += blockDim.x) {
-            const double d = L.d[t];
-            sdi[off[l] + t] = 1.0 / d;
-            swe[off[l] + t] = L.we[t];
-            swn[off[l] + t] = L.wn[t];
-            sb[off[l] + t] = (l == lc) ? L.b[t] : 0.0;
-            sx[off[l] + t] = 0.0;
-        }
-    }
-    __syncthreads();
-    // A x of cell (i, j) at flat LDS index f of a level nx x ny
-    auto ax = [&](int f, int i, int j, int nx, int ny) -> double {
-        const bool e = i + 1 < nx, w = i > 0, nn = j + 1 < ny, so = j > 0;
-        const int fe = f + (e ? 1 : 0), fw = f - (w ? 1 : 0), fn = f + (nn ? nx : 0), fs = f - (so ? nx : 0);
-        const double ce = e ? swe[f] : 0.0, cw = w ? swe[fw] : 0.0, cn = nn ? swn[f] : 0.0, cs = so ? swn[fs] : 0.0;
-        return sx[f] / sdi[f] - ce * sx[fe] - cw * sx[fw] - cn * sx[fn] - cs * sx[fs];
-    };
-    auto half = [&](int l, int color) {   // cells of the colour only: row j holds i = (color - j) & 1, +2, ...
-        const int nx = h.lv[l].nx, ny = h.lv[l].ny, o = off[l];
-        const int hw = (nx + 1) / 2;
-        for (int u = threadIdx.x; u < ny * hw; u += blockDim.x) {
-            const int j = u / hw;
-            const int i = ((color - j) & 1) + 2 * (u - j * hw);
-            if (i >= nx) continue;
-            const int f = o + j * nx + i;
-            const bool e = i + 1 < nx, w = i > 0, nn = j + 1 < ny, so = j > 0;
-            const int fe = f + (e ? 1 : 0), fw = f - (w ? 1 : 0), fn = f + (nn ? nx : 0), fs = f - (so ? nx : 0);
-            const double ce = e ? swe[f] : 0.0, cw = w ? swe[fw] : 0.0, cn = nn ? swn[f] : 0.0, cs = so ? swn[fs] : 0.0;
-            const double s = sb[f] + ce * sx[fe] + cw * sx[fw] + cn * sx[fn] + cs * sx[fs];
-            sx[f] = s * sdi[f];
-        }
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) v += inv[i] * (ec * PER + i < ne ? sb[eb + ec * PER + i] : 0.0);
+        pp[ec][er] = v;
         __syncthreads();
-    };
-    for (int l = lc; l < nl - 1; ++l) {
-        half(l, 0); half(l, 1); half(l, 0); half(l, 1);
-        const int nx = h.lv[l].nx, ny = h.lv[l].ny, o = off[l];
-        const int cnx = h.lv[l + 1].nx, cny = h.lv[l + 1].ny, co = off[l + 1];
-        for (int t = threadIdx.x; t < cnx * cny; t += blockDim.x) {   // b_coarse = P^T (b - A x)
-            const int J = t / cnx, I = t - J * cnx;
-            double s = 0.0;
-            for (int dj = 0; dj < 2; ++dj)
-                for (int di = 0; di < 2; ++di) {
-                    const int i = 2 * I + di, j = 2 * J + dj;
-                    if (i < nx && j < ny) {
-                        const int f = o + j * nx + i;
-                        s += sb[f] - ax(f, i, j, nx, ny);
-                    }
-                }
-            sb[co + t] = s;
+        if (tid < NE) {
+            double y = 0.0;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) y += pp[c][tid];
+            ye[tid] = y;
         }
         __syncthreads();
     }
-    {
-        const int o = off[nl - 1], n = h.lv[nl - 1].nx * h.lv[nl - 1].ny;   // level le: exact
-        for (int t = threadIdx.x; t < n; t += blockDim.x) {
-            double v = 0.0;
-            for (int j = 0; j < n; ++j) v += h.inv[t * n + j] * sb[o + j];
-            sx[o + t] = v;
+    for (int l = le - 1; l >= lc; --l) {
+        const bool on = lv == l;
+        if (on) {
+            double yc;
+            if (l + 1 == le) {
+                yc = ye[tid - base];
+            } else {   // cell (I, J) of the next level, in that level's planes
+                const int cbx = h.lv[l + 2].nx, cby = h.lv[l + 2].ny;
+                const double* cx = sx + xo + 4 * s.plane;
+                yc = cx[((J & 1) * 2 + (I & 1)) * (cbx + 2) * (cby + 2) + ((J >> 1) + 1) * (cbx + 2) + (I >> 1) + 1];
+            }
+            if (in.c[0]) a.x[0] += kMgOver * yc;
+            if (in.c[3]) a.x[3] += kMgOver * yc;
         }
+        agg_up(a, s, on, true);
         __syncthreads();
     }
-    for (int l = nl - 2; l >= lc; --l) {
-        const int nx = h.lv[l].nx, ny = h.lv[l].ny, o = off[l];
-        const int cnx = h.lv[l + 1].nx, co = off[l + 1];
-        for (int t = threadIdx.x; t < nx * ny; t += blockDim.x) {
-            const int j = t / nx, i = t - j * nx;
-            sx[o + t] += kMgOver * sx[co + (j >> 1) * cnx + (i >> 1)];
-        }
-        __syncthreads();
-        half(l, 1); half(l, 0); half(l, 1); half(l, 0);
-    }
-    const MgLevel& L = h.lv[lc];
-    const int n = L.nx * L.ny, o = off[lc];
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        L.y[t] = sx[o + t];
-        acc[0] += sb[o + t] * sx[o + t];
-        acc[1] += sb[o + t] * sb[o + t];
-        if (bb_src) acc[2] += bb_src[t] * bb_src[t];
+    if (lc == le) {
+        if (tid < ne) {
+            L.y[tid] = ye[tid];
+            acc[0] = sb[tid] * ye[tid];
+            acc[1] = sb[tid] * sb[tid];
+            if (bb_src) acc[2] = bb_src[tid] * bb_src[tid];
+        }
+    } else if (lv == lc) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (!in.c[c]) continue;
+            L.y[g + off[c]] = a.x[c];
+            acc[0] += a.b[c] * a.x[c];
+            acc[1] += a.b[c] * a.b[c];
+            if (bb_src) acc[2] += bb_src[g + off[c]] * bb_src[g + off[c]];
+        }
     }
     acc[3] = acc[1];
     if (part) block_partials<4, false>(acc, part);
@@ -741,38 +906,34 @@ void launch_mg_setup(hipStream_t s, const Geo2& g, const double* ke, const doubl
     hipLaunchKernelGGL(k_mg_inverse, dim3(1), dim3(kMgThreads), 0, s, h);
 }
 
+static void mg_down0(hipStream_t s, const MgHier& h, int l, const PcgState* st)
+{
+    hipLaunchKernelGGL(k_mg_down<false>, dim3(mg_tiles(h.lv[l])), dim3(mg_tile_threads(kMgHalo)), 0, s, h.lv[l],
+                       h.lv[l + 1], st, MgCg1{});
+}
+
+static void mg_up0(hipStream_t s, const MgHier& h, int l, const PcgState* st)
+{
+    hipLaunchKernelGGL(k_mg_up<false>, dim3(mg_tiles(h.lv[l])), dim3(mg_tile_threads(kMgHalo)), 0, s, h.lv[l],
+                       h.lv[l + 1], h.lv[l].y, st, nullptr, nullptr, nullptr);
+}
+
 void launch_mg_vcycle(hipStream_t s, const MgHier& h, const PcgState* st, double* part, const double* bb_src)
 {
     const int lc = mg_coarse_level(h);
-    for (int l = 0; l < lc; ++l)
-        hipLaunchKernelGGL(k_mg_down<0>, dim3(mg_tiles(h.lv[l])), dim3(kMgThreads), 0, s, h, l, st, MgUpd{},
-                           MgCg1{});
+    for (int l = 0; l < lc; ++l) mg_down0(s, h, l, st);
     hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, h, st, lc == 0 ? part : nullptr,
                        lc == 0 ? bb_src : nullptr);
-    for (int l = lc - 1; l >= 0; --l)
-        hipLaunchKernelGGL(k_mg_up<false>, dim3(mg_tiles(h.lv[l])), dim3(kMgThreads), 0, s, h, l, h.lv[l].y, st,
-                           l == 0 ? part : nullptr, l == 0 ? bb_src : nullptr, nullptr);
+    for (int l = lc - 1; l >= 0; --l) mg_up0(s, h, l, st);
 }
 
 void launch_mg_vcycle_upd(hipStream_t s, const MgHier& h, const PcgState* st, double* part, const MgUpd& u)
 {
     MgHier hh = h;
     hh.lv[0].b = u.r_new;   // level 0 of this V-cycle: the updated residual
-    const int lc = mg_coarse_level(hh);
-    if (lc == 0) {   // a surface of <= 32 x 32 cells: the update as its own kernel
-        hipLaunchKernelGGL(k_pcg_update_mg, dim3(grid_for(h.lv[0].nx * h.lv[0].ny)), dim3(kBlock), 0, s,
-                           h.lv[0].nx * h.lv[0].ny, u);
-        launch_mg_vcycle(s, hh, st, part, nullptr);
-        return;
-    }
-    hipLaunchKernelGGL(k_mg_down<1>, dim3(mg_tiles(hh.lv[0])), dim3(kMgThreads), 0, s, hh, 0, st, u, MgCg1{});
-    for (int l = 1; l < lc; ++l)
-        hipLaunchKernelGGL(k_mg_down<0>, dim3(mg_tiles(hh.lv[l])), dim3(kMgThreads), 0, s, hh, l, st, MgUpd{},
-                           MgCg1{});
-    hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, hh, st, nullptr, nullptr);
-    for (int l = lc - 1; l >= 0; --l)
-        hipLaunchKernelGGL(k_mg_up<false>, dim3(mg_tiles(hh.lv[l])), dim3(kMgThreads), 0, s, hh, l, hh.lv[l].y, st,
-                           l == 0 ? part : nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_pcg_update_mg, dim3(grid_for(h.lv[0].nx * h.lv[0].ny)), dim3(kBlock), 0, s,
+                       h.lv[0].nx * h.lv[0].ny, u);
+    launch_mg_vcycle(s, hh, st, part, nullptr);
 }
 
 // The V-cycle below level 0 (down kernels of levels 1 .. lc-1, the single-block kernel, up
@@ -781,21 +942,17 @@ static void mg_vcycle_cg1_rest(hipStream_t s, const MgHier& h, const PcgState* s
                                const double* bb_src, double* w)
 {
     const int lc = mg_coarse_level(h);
-    for (int l = 1; l < lc; ++l)
-        hipLaunchKernelGGL(k_mg_down<0>, dim3(mg_tiles(h.lv[l])), dim3(kMgThreads), 0, s, h, l, st, MgUpd{},
-                           MgCg1{});
+    for (int l = 1; l < lc; ++l) mg_down0(s, h, l, st);
     hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, h, st, nullptr, nullptr);
-    for (int l = lc - 1; l >= 1; --l)
-        hipLaunchKernelGGL(k_mg_up<false>, dim3(mg_tiles(h.lv[l])), dim3(kMgThreads), 0, s, h, l, h.lv[l].y, st,
-                           nullptr, nullptr, nullptr);
-    hipLaunchKernelGGL(k_mg_up<true>, dim3(mg_tiles(h.lv[0])), dim3(kMgThreads), 0, s, h, 0, h.lv[0].y, st, part,
-                       bb_src, w);
+    for (int l = lc - 1; l >= 1; --l) mg_up0(s, h, l, st);
+    hipLaunchKernelGGL(k_mg_up<true>, dim3(mg_tiles(h.lv[0])), dim3(mg_tile_threads(kMgHaloA)), 0, s, h.lv[0], h.lv[1],
+                       h.lv[0].y, st, part, bb_src, w);
 }
 
 void launch_mg_vcycle_cg1_start(hipStream_t s, const MgHier& h, const PcgState* st, double* part,
                                 const double* bb_src, double* w)
 {
-    hipLaunchKernelGGL(k_mg_down<0>, dim3(mg_tiles(h.lv[0])), dim3(kMgThreads), 0, s, h, 0, st, MgUpd{}, MgCg1{});
+    mg_down0(s, h, 0, st);
     mg_vcycle_cg1_rest(s, h, st, part, bb_src, w);
 }
 
@@ -814,7 +971,8 @@ void launch_mg_vcycle_cg1(hipStream_t s, const MgHier& h, const PcgState* st, do
 {
     MgHier hh = h;
     hh.lv[0].b = v.r_new;   // level 0 of this V-cycle: the updated residual
-    hipLaunchKernelGGL(k_mg_down<2>, dim3(mg_tiles(hh.lv[0])), dim3(kMgThreads), 0, s, hh, 0, st, MgUpd{}, v);
+    hipLaunchKernelGGL(k_mg_down<true>, dim3(mg_tiles(hh.lv[0])), dim3(mg_tile_threads(kMgHalo)), 0, s, hh.lv[0],
+                       hh.lv[1], st, v);
     mg_vcycle_cg1_rest(s, hh, st, part, nullptr, v.w);
 }
 
