@@ -89,23 +89,54 @@ __device__ __forceinline__ int lin_tid() { return threadIdx.x + threadIdx.y * bl
 __device__ __forceinline__ int lin_nthreads() { return blockDim.x * blockDim.y; }
 __device__ __forceinline__ int lin_bid() { return blockIdx.x + blockIdx.y * gridDim.x; }
 
+// Lane moves of the wave reductions through the data-parallel primitives (a few cycles each; the
+// LDS-permute butterfly they replace waited ~100 cycles in each of its six steps, which the small
+// launches of a solve paid twice per reduction).  CTRL: the DPP control; lanes without a source,
+// or in a row that ROWS masks out, get `other`.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v, double other)
+{
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(other), __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(other), __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;   // within rows of 16
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;   // last lane of a row / of two rows to the next
+
+// Total over the wave (all 64 lanes take part), in every lane.
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
+    v += dpp_move<kDppShr1, 0xf>(v, 0.0);
+    v += dpp_move<kDppShr2, 0xf>(v, 0.0);
+    v += dpp_move<kDppShr4, 0xf>(v, 0.0);
+    v += dpp_move<kDppShr8, 0xf>(v, 0.0);
+    v += dpp_move<kDppBcast15, 0xa>(v, 0.0);
+    v += dpp_move<kDppBcast31, 0xc>(v, 0.0);
+    return lane_value(v, kWave - 1);
 }
 
 __device__ __forceinline__ double wave_max(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kWave));
-    return v;
+    v = fmax(v, dpp_move<kDppShr1, 0xf>(v, v));
+    v = fmax(v, dpp_move<kDppShr2, 0xf>(v, v));
+    v = fmax(v, dpp_move<kDppShr4, 0xf>(v, v));
+    v = fmax(v, dpp_move<kDppShr8, 0xf>(v, v));
+    v = fmax(v, dpp_move<kDppBcast15, 0xa>(v, v));
+    v = fmax(v, dpp_move<kDppBcast31, 0xc>(v, v));
+    return lane_value(v, kWave - 1);
 }
 
-// Block reduction of NV values; the result is valid in every lane of wave 0.
-// lds must hold NV * 16 doubles.
-template <int NV, bool MAX>
+// Block reduction of NV values, the result in every thread: each wave leaves its totals in LDS and,
+// after one barrier, reduces all of them itself.  lds must hold NV * 16 doubles and not be in use by
+// an earlier reduction whose results some wave may still be reading (FENCE: a barrier first).
+template <int NV, bool MAX, bool FENCE = true>
 __device__ __forceinline__ void block_reduce(double (&v)[NV], double* lds)
 {
     const int tid = lin_tid();
@@ -113,18 +144,17 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV], double* lds)
     const int nw = lin_nthreads() / kWave;
 #pragma unroll
     for (int i = 0; i < NV; ++i) v[i] = MAX ? wave_max(v[i]) : wave_sum(v[i]);
-    __syncthreads();
+    if (FENCE) __syncthreads();
     if (lane == 0) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) lds[i * 16 + wid] = v[i];
     }
     __syncthreads();
-    if (wid == 0) {
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            double t = (lane < nw) ? lds[i * 16 + lane] : (MAX ? -INFINITY : 0.0);
-            v[i] = MAX ? wave_max(t) : wave_sum(t);
-        }
+    for (int i = 0; i < NV; ++i) {
+        // sums start from +0 and maxima from the first wave's value: idle lanes change neither
+        const double t = lds[i * 16 + (lane < nw ? lane : 0)];
+        v[i] = MAX ? wave_max(t) : wave_sum(lane < nw ? t : 0.0);
     }
 }
 
@@ -141,7 +171,7 @@ template <int NV, bool MAX>
 __device__ __forceinline__ void block_partials(double (&v)[NV], double* part, int bid)
 {
     __shared__ double lds[NV * 16];
-    block_reduce<NV, MAX>(v, lds);
+    block_reduce<NV, MAX, false>(v, lds);   // a kernel's last step: its LDS is used once
     if (lin_tid() == 0) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) part[i * kMaxBlocks + bid] = v[i];
@@ -161,7 +191,6 @@ __device__ __forceinline__ void sum_partials(const double* __restrict__ part, in
                                             double (&out)[NV])
 {
     __shared__ double lds[NV * 16];
-    __shared__ double res[NV];
     double acc[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) acc[i] = 0.0;
@@ -170,14 +199,9 @@ __device__ __forceinline__ void sum_partials(const double* __restrict__ part, in
         for (int i = 0; i < NV; ++i)
             if (i < nv) acc[i] += part[i * kMaxBlocks + b];
     }
-    block_reduce<NV, false>(acc, lds);
-    if (lin_tid() == 0) {
+    block_reduce<NV, false, false>(acc, lds);   // a kernel's first step: its LDS is used once
 #pragma unroll
-        for (int i = 0; i < NV; ++i) res[i] = acc[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NV; ++i) out[i] = res[i];
+    for (int i = 0; i < NV; ++i) out[i] = acc[i];
 }
 
 }  // namespace dh

@@ -889,7 +889,6 @@ int overland_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         (any_mg && ((rc = upload_args(e, e->a_omg, e->h_omg)) || (rc = upload_args(e, e->olf_mgm, mgm)))))
         return rc;
     const MapRef r2 = use_map(e, e->cm2);
-    dh::launch_batched(e->s, dh::BK_OLF_H, e->a_olf, r2.map, r2.n, e->active);
     dh::launch_batched(e->s, dh::BK_OLF_FACES, e->a_olf, r2.map, r2.n, e->active);
     dh::launch_batched(e->s, dh::BK_OLF_ASM, e->a_olf, r2.map, r2.n, e->active);
     if (any_mg) dh::launch_batched_olf_mgcg_block(e->s, e->a_omg, M, e->olf_mgm);

@@ -220,18 +220,9 @@ __device__ __forceinline__ double op2_row(const Geo2& g, int c, double Dc, doubl
 }
 
 // Totals of three per-thread values, returned to every thread of the block.
-__device__ __forceinline__ void block_sum3(double (&v)[3], double* lds, double* res)
+__device__ __forceinline__ void block_sum3(double (&v)[3], double* lds)
 {
     block_reduce<3, false>(v, lds);
-    if (lin_tid() == 0) {
-        res[0] = v[0];
-        res[1] = v[1];
-        res[2] = v[2];
-    }
-    __syncthreads();
-    v[0] = res[0];
-    v[1] = res[1];
-    v[2] = res[2];
 }
 
 // The overland Jacobi-PCG of a whole surface in one workgroup (surfaces of at most
@@ -391,7 +382,7 @@ void launch_cast_f32(hipStream_t s, int n, const double* in, float* out);
 void launch_cast_f64(hipStream_t s, int n, const float* in, double* out);
 
 // Overland
-void launch_olf_faces(hipStream_t s, const OlfArgs& a);
+void launch_olf_faces(hipStream_t s, const OlfArgs& a);   // H = h + z and the face conductances
 void launch_olf_assemble(hipStream_t s, const OlfArgs& a);
 // z = NULL: Jacobi (p = r/D + beta p); otherwise p = z + beta p with z the preconditioned residual.
 void launch_pcg2_spmv(hipStream_t s, const Geo2& g, const double* ke, const double* kn,
@@ -448,7 +439,7 @@ void launch_batched_cg1_init(hipStream_t s, bool fp32, const void* args, const B
 void launch_batched_cg1(hipStream_t s, bool fp32, const void* args, const BlkMap* map, int nblocks,
                         const int* active, const int* it_base, int k);
 enum BatchKind { BK_VG = 0, BK_VG_PICARD, BK_SURF_PRE, BK_SURF_POST, BK_ASM_F64, BK_ASM_MIXED,
-                 BK_REFINE_ADD, BK_REFINE_RES, BK_END, BK_OLF_H, BK_OLF_FACES, BK_OLF_ASM, BK_OLF_POST,
+                 BK_REFINE_ADD, BK_REFINE_RES, BK_END, BK_OLF_FACES, BK_OLF_ASM, BK_OLF_POST,
                  BK_PICARD_INC };   // BK_PICARD_INC: VgArgs, the increment of psi (x) over psi_m alone
 // args points to an array of the argument struct of the kind (VgArgs, SurfArgs, AsmArgs,
 // RefineArgs, EndArgs or OlfArgs), one per model.

@@ -1682,46 +1682,38 @@ __device__ __forceinline__ double olf_face_k(double gdir, double gcross, double 
     return K0;
 }
 
-// H = h + z, then the east and north face conductances of every face the eliminated
-// system uses, each evaluated from its non-ring cell (the row that owns the coupling in
-// the reference matrix).
-__device__ __forceinline__ void b_olf_H(OlfArgs a, Blk bk)
-{
-    for (int c = bk.id * blockDim.x + threadIdx.x; c < a.g.n; c += bk.n * blockDim.x)
-        a.H[c] = a.h[c] + a.z[c];
-}
-
-__global__ __launch_bounds__(kBlock) void k_olf_H(OlfArgs a)
-{
-    b_olf_H(a, hw_blk());
-}
-
+// H = h + z (stored; formed again for the neighbours, from the same two values), and the east and
+// north face conductances of every face the eliminated system uses, each evaluated from its
+// non-ring cell (the row that owns the coupling in the reference matrix).
 __device__ __forceinline__ void b_olf_faces(OlfArgs a, Blk bk)
 {
     const Geo2 g = a.g;
     const int nx = g.nx;
-    const double* __restrict__ H = a.H;
     const double* __restrict__ h = a.h;
+    const double* __restrict__ z = a.z;
     const double* __restrict__ m = a.mann;
+    auto H = [&](int c) { return h[c] + z[c]; };
     for (int c = bk.id * blockDim.x + threadIdx.x; c < g.n; c += bk.n * blockDim.x) {
         const int j = c / nx, i = c - j * nx;
+        const double Hc = H(c);
+        a.H[c] = Hc;
         double ke = 0.0, kn = 0.0;
         // east face (i,j)-(i+1,j): used when row j is interior
         if (i < nx - 1 && j > 0 && j < g.ny - 1) {
-            const double gx = (H[c + 1] - H[c]) / g.dx;
-            const double gy = (H[c + nx + 1] + H[c + nx] - H[c - nx + 1] - H[c - nx]) / (4 * g.dy);
+            const double gx = (H(c + 1) - Hc) / g.dx;
+            const double gy = (H(c + nx + 1) + H(c + nx) - H(c - nx + 1) - H(c - nx)) / (4 * g.dy);
             const bool west_owner = !is_ring(g, i, j);
             // owner's view: neighbour upwind if its H is strictly higher
-            const bool up_east = west_owner ? (H[c + 1] > H[c]) : !(H[c] > H[c + 1]);
+            const bool up_east = west_owner ? (H(c + 1) > Hc) : !(Hc > H(c + 1));
             ke = olf_face_k(gx, gy, h[c + 1], h[c], m[c + 1], m[c], up_east, a.hmin, a.delta, a.K0);
             // olf_face_k's "neighbour" is the east cell here
         }
         // north face (i,j)-(i,j+1): used when column i is interior
         if (j < g.ny - 1 && i > 0 && i < nx - 1) {
-            const double gyy = (H[c + nx] - H[c]) / g.dy;
-            const double gxx = (H[c + nx + 1] + H[c + 1] - H[c + nx - 1] - H[c - 1]) / (4 * g.dx);
+            const double gyy = (H(c + nx) - Hc) / g.dy;
+            const double gxx = (H(c + nx + 1) + H(c + 1) - H(c + nx - 1) - H(c - 1)) / (4 * g.dx);
             const bool south_owner = !is_ring(g, i, j);
-            const bool up_north = south_owner ? (H[c + nx] > H[c]) : !(H[c] > H[c + nx]);
+            const bool up_north = south_owner ? (H(c + nx) > Hc) : !(Hc > H(c + nx));
             kn = olf_face_k(gyy, gxx, h[c + nx], h[c], m[c + nx], m[c], up_north, a.hmin, a.delta, a.K0);
         }
         a.ke[c] = ke;
@@ -1833,7 +1825,6 @@ __global__ __launch_bounds__(kBlock) void k_pcg2_spmv(Geo2 g, const double* __re
 __device__ __forceinline__ void b_olf_cg_block(const OlfCgArgs& a)
 {
     __shared__ double lds[3 * 16];
-    __shared__ double res[3];
     const Geo2 g = a.g;
     const int n = g.n, tid = threadIdx.x, nt = blockDim.x;
     const double* __restrict__ D = a.D;
@@ -1850,7 +1841,7 @@ __device__ __forceinline__ void b_olf_cg_block(const OlfCgArgs& a)
         v[1] += rc * rc;
         v[2] += b[c] * b[c];
     }
-    block_sum3(v, lds, res);
+    block_sum3(v, lds);
     double rz = v[0], rr = v[1], beta = 0.0;
     const double bb = v[2], tol2 = a.tol * a.tol * bb;
     int it = 0, conv = 0, nan = !isfinite(bb);
@@ -1868,7 +1859,7 @@ __device__ __forceinline__ void b_olf_cg_block(const OlfCgArgs& a)
             zq[c] = qc;
             w[0] += pc * qc;
         }
-        block_sum3(w, lds, res);
+        block_sum3(w, lds);
         const double alpha = rz / w[0];
         if (!(w[0] != 0.0) || !isfinite(alpha)) {
             nan = 1;
@@ -1884,7 +1875,7 @@ __device__ __forceinline__ void b_olf_cg_block(const OlfCgArgs& a)
             u[0] += rc * zc;
             u[1] += rc * rc;
         }
-        block_sum3(u, lds, res);
+        block_sum3(u, lds);
         ++it;
         beta = u[0] / rz;
         rz = u[0];
@@ -2883,7 +2874,6 @@ void launch_cast_f64(hipStream_t s, int n, const float* in, double* out)
 
 void launch_olf_faces(hipStream_t s, const OlfArgs& a)
 {
-    hipLaunchKernelGGL(k_olf_H, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
     hipLaunchKernelGGL(k_olf_faces, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
 }
 
@@ -2952,8 +2942,6 @@ void launch_batched(hipStream_t s, BatchKind kind, const void* args, const BlkMa
         break;
     case BK_END:
         hipLaunchKernelGGL((kb_args<EndArgs, b_end_step>), gr, bl, 0, s, (const EndArgs*)args, map, active); break;
-    case BK_OLF_H:
-        hipLaunchKernelGGL((kb_args<OlfArgs, b_olf_H>), gr, bl, 0, s, (const OlfArgs*)args, map, active); break;
     case BK_OLF_FACES:
         hipLaunchKernelGGL((kb_args<OlfArgs, b_olf_faces>), gr, bl, 0, s, (const OlfArgs*)args, map, active);
         break;

@@ -59,21 +59,19 @@ __device__ __forceinline__ int mg_coarse_first(const MgHier& h) { return mg_firs
 
 // Level-0 operator: the eliminated overland matrix.  Diagonal = the assembled D (ring rows 1);
 // weights only between two interior cells (couplings to the ring moved to the right-hand side).
+__device__ __forceinline__ void mg_fine_cell(const Geo2& g, const double* ke, const double* kn, double* we, double* wn,
+                                             int i, int j)
+{
+    const int c = j * g.nx + i;
+    const bool in = i > 0 && j > 0 && i < g.nx - 1 && j < g.ny - 1;
+    we[c] = (in && i + 1 < g.nx - 1) ? g.cx * ke[c] : 0.0;
+    wn[c] = (in && j + 1 < g.ny - 1) ? g.cy * kn[c] : 0.0;
+}
+
 __device__ __forceinline__ void mg_fine_cells(const Geo2& g, const double* ke, const double* kn, double* we,
                                               double* wn, int first, int stride)
 {
-    for (int c = first; c < g.n; c += stride) {
-        const int j = c / g.nx, i = c - j * g.nx;
-        const bool in = i > 0 && j > 0 && i < g.nx - 1 && j < g.ny - 1;
-        we[c] = (in && i + 1 < g.nx - 1) ? g.cx * ke[c] : 0.0;
-        wn[c] = (in && j + 1 < g.ny - 1) ? g.cy * kn[c] : 0.0;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_mg_fine(Geo2 g, const double* ke, const double* kn, double* we,
-                                                    double* wn)
-{
-    mg_fine_cells(g, ke, kn, we, wn, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    for (int c = first; c < g.n; c += stride) mg_fine_cell(g, ke, kn, we, wn, c % g.nx, c / g.nx);
 }
 
 // Galerkin coarse operator of 2 x 2 aggregates: d_C = sum d_f - 2 (couplings inside C),
@@ -103,6 +101,19 @@ __device__ __forceinline__ void mg_coarsen_cells(const MgLevel& F, const MgLevel
 __global__ __launch_bounds__(kBlock) void k_mg_coarsen(MgLevel F, MgLevel C)
 {
     mg_coarsen_cells(F, C, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+
+// The level-0 weights and the operator of level 1 (whose cells need only their own children's).
+__global__ __launch_bounds__(kBlock) void k_mg_fine_coarsen(Geo2 g, const double* __restrict__ ke,
+                                                            const double* __restrict__ kn, MgLevel F, MgLevel C)
+{
+    for (int cc = blockIdx.x * blockDim.x + threadIdx.x; cc < C.nx * C.ny; cc += gridDim.x * blockDim.x) {
+        const int J = cc / C.nx, I = cc - J * C.nx;
+        for (int dj = 0; dj < 2; ++dj)
+            for (int di = 0; di < 2; ++di)
+                if (2 * I + di < F.nx && 2 * J + dj < F.ny) mg_fine_cell(g, ke, kn, F.we, F.wn, 2 * I + di, 2 * J + dj);
+        mg_coarsen_cells(F, C, cc, C.nx * C.ny);   // this cell alone
+    }
 }
 
 // A thread's 2 x 2 aggregate of a level: cells 0 (i, j), 1 (i + 1, j), 2 (i, j + 1), 3 (i + 1, j + 1)
@@ -606,19 +617,24 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgSta
     if (part) block_partials<4, false>(acc, part);
 }
 
-// Dense inverse of level le's operator (at most 64 cells) by Gauss-Jordan elimination in LDS;
-// the operator is symmetric positive definite and diagonally dominant, so no pivoting.
-// The dense inverse of level le's operator in M (kMgExactCells^2 doubles, row pitch
-// kMgExactCells), by a block of kMgThreads threads.
-__device__ __forceinline__ void mg_gauss_jordan(const MgHier& h, double* M)
+// Dense inverse of level le's operator (at most 64 cells) by Gauss-Jordan elimination; the operator
+// is symmetric positive definite and diagonally dominant, so no pivoting.  A lane holds column
+// `lane` of the rows w, w + 16, w + 32, w + 48 of its wave w in registers: a row's own pivot-column
+// entry is a lane read, and only the pivot row goes through LDS (two buffers, one barrier a
+// step).  With the matrix in LDS and two barriers a step the 49 steps of a 7 x 7 level took 48 us.
+// The result goes to out, row pitch `pitch` (rows and columns < n).  Every thread of a block of
+// kMgThreads calls it; a barrier must follow before out is read.
+__device__ __forceinline__ void mg_gauss_jordan(const MgLevel& L, double* out, int pitch)
 {
-    constexpr int NE = kMgExactCells, PER = NE * NE / kMgThreads;   // row pitch NE: i = e >> 6, j = e & 63
-    static_assert(NE == 64, "index arithmetic assumes a 64-wide pitch");
-    static_assert(NE * NE % kMgThreads == 0, "whole elements per thread");
-    const MgLevel L = h.lv[h.le];
+    constexpr int NE = kMgExactCells, NW = kMgThreads / kWave, PER = NE / NW;
+    static_assert(NE == kWave && NE % NW == 0, "a lane is a column, a wave whole rows");
+    __shared__ double row[2][NE];
     const int nx = L.nx, n = L.nx * L.ny;
-    for (int e = threadIdx.x; e < NE * NE; e += blockDim.x) {
-        const int i = e >> 6, j = e & 63;
+    const int j = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    double m[PER];
+#pragma unroll
+    for (int c = 0; c < PER; ++c) {
+        const int i = w + c * NW;
         double v = 0.0;
         if (i < n && j < n) {
             if (i == j) v = L.d[i];
@@ -627,35 +643,47 @@ __device__ __forceinline__ void mg_gauss_jordan(const MgHier& h, double* M)
             else if (j == i + nx) v = -L.wn[i];
             else if (i == j + nx) v = -L.wn[j];
         }
-        M[e] = v;
+        m[c] = v;
     }
-    __syncthreads();
-    for (int k = 0; k < n; ++k) {
-        const double ip = 1.0 / M[k * NE + k];
-        double nv[PER];
 #pragma unroll
-        for (int c = 0; c < PER; ++c) {
-            const int e = threadIdx.x + c * kMgThreads, i = e >> 6, j = e & 63;
-            const double rk = (j == k) ? ip : M[k * NE + j] * ip;   // row k, scaled
-            nv[c] = (i == k) ? rk : ((j == k) ? -M[i * NE + k] * ip : M[e] - M[i * NE + k] * rk);
+    for (int ck = 0; ck < PER; ++ck)
+        for (int kk = 0; kk < NW; ++kk) {
+            const int k = ck * NW + kk;
+            if (k >= n) break;
+            if (w == kk) row[k & 1][j] = m[ck];
+            __syncthreads();
+            const double pr = row[k & 1][j];
+            const double ip = 1.0 / lane_value(pr, k);
+            const double rk = (j == k) ? ip : pr * ip;   // row k, scaled
+#pragma unroll
+            for (int c = 0; c < PER; ++c) {
+                const double f = lane_value(m[c], k);
+                const double v = (j == k) ? -f * ip : m[c] - f * rk;
+                m[c] = (c == ck && w == kk) ? rk : v;
+            }
         }
-        __syncthreads();
 #pragma unroll
-        for (int c = 0; c < PER; ++c) M[threadIdx.x + c * kMgThreads] = nv[c];
-        __syncthreads();
+    for (int c = 0; c < PER; ++c) {
+        const int i = w + c * NW;
+        if (i < n && j < n) out[i * pitch + j] = m[c];
     }
 }
 
-__global__ __launch_bounds__(kMgThreads) void k_mg_inverse(MgHier h)
+// The operators of the levels below the first one the single-block kernel handles (and level 0's
+// weights when that is level 0), and the exact level's inverse, by one block: a launch per level
+// took longer than their few cells.
+__global__ __launch_bounds__(kMgThreads) void k_mg_setup_coarse(Geo2 g, const double* ke, const double* kn, MgHier h)
 {
-    constexpr int NE = kMgExactCells;
-    __shared__ double M[NE * NE];
-    mg_gauss_jordan(h, M);
-    const int n = h.lv[h.le].nx * h.lv[h.le].ny;
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-        const int i = e / n, j = e - i * n;
-        h.inv[e] = M[i * NE + j];
+    const int lc = mg_coarse_first(h);
+    if (lc == 0) {
+        mg_fine_cells(g, ke, kn, h.lv[0].we, h.lv[0].wn, threadIdx.x, blockDim.x);
+        __syncthreads();
     }
+    for (int l = lc; l < h.le; ++l) {
+        mg_coarsen_cells(h.lv[l], h.lv[l + 1], threadIdx.x, blockDim.x);
+        __syncthreads();
+    }
+    mg_gauss_jordan(h.lv[h.le], h.inv, h.lv[h.le].nx * h.lv[h.le].ny);
 }
 
 // The update of MgUpd as a kernel of its own (surfaces handled entirely by the coarse kernel).
@@ -765,7 +793,6 @@ __device__ __forceinline__ void b_olf_mgcg_block(const OlfCgArgs& a, const MgHie
 {
     __shared__ double Minv[kMgExactCells * kMgExactCells];
     __shared__ double lds[3 * 16];
-    __shared__ double res[3];
     const Geo2 g = a.g;
     const int n = g.n, tid = threadIdx.x, nt = blockDim.x;
     // the operators of this step's system: level-0 weights, Galerkin coarse levels, exact inverse
@@ -775,7 +802,8 @@ __device__ __forceinline__ void b_olf_mgcg_block(const OlfCgArgs& a, const MgHie
         mg_coarsen_cells(h.lv[l], h.lv[l + 1], tid, nt);
         __syncthreads();
     }
-    mg_gauss_jordan(h, Minv);
+    mg_gauss_jordan(h.lv[h.le], Minv, kMgExactCells);
+    __syncthreads();
     const double* __restrict__ b = a.b;
     double* __restrict__ x = a.x;
     double* __restrict__ r = a.r;
@@ -791,7 +819,7 @@ __device__ __forceinline__ void b_olf_mgcg_block(const OlfCgArgs& a, const MgHie
         v[1] += rc * rc;
         v[2] += b[c] * b[c];
     }
-    block_sum3(v, lds, res);
+    block_sum3(v, lds);
     double rz = v[0], rr = v[1], beta = 0.0;
     const double bb = v[2], tol2 = a.tol * a.tol * bb;
     int it = 0, conv = 0, nan = !isfinite(bb);
@@ -809,7 +837,7 @@ __device__ __forceinline__ void b_olf_mgcg_block(const OlfCgArgs& a, const MgHie
             q[c] = qc;
             w[0] += pc * qc;
         }
-        block_sum3(w, lds, res);
+        block_sum3(w, lds);
         const double alpha = rz / w[0];
         if (!(w[0] != 0.0) || !isfinite(alpha)) {
             nan = 1;
@@ -824,7 +852,7 @@ __device__ __forceinline__ void b_olf_mgcg_block(const OlfCgArgs& a, const MgHie
         }
         mgb_vcycle(h, Minv, r, z);   // its first barrier orders the r writes before its reads
         for (int c = tid; c < n; c += nt) u[0] += r[c] * z[c];
-        block_sum3(u, lds, res);
+        block_sum3(u, lds);
         ++it;
         beta = u[0] / rz;
         rz = u[0];
@@ -898,12 +926,16 @@ int mg_partials(const MgHier& h)
 
 void launch_mg_setup(hipStream_t s, const Geo2& g, const double* ke, const double* kn, const MgHier& h)
 {
-    hipLaunchKernelGGL(k_mg_fine, dim3(grid_for(g.n)), dim3(kBlock), 0, s, g, ke, kn, h.lv[0].we, h.lv[0].wn);
-    for (int l = 0; l < h.le; ++l) {
+    // levels 0 and 1 together, the other levels above the single-block kernel's first one a launch each
+    const int lc = mg_coarse_level(h);
+    if (lc > 0)
+        hipLaunchKernelGGL(k_mg_fine_coarsen, dim3(grid_for(h.lv[1].nx * h.lv[1].ny)), dim3(kBlock), 0, s, g, ke, kn,
+                           h.lv[0], h.lv[1]);
+    for (int l = 1; l < lc; ++l) {
         const int nc = h.lv[l + 1].nx * h.lv[l + 1].ny;
         hipLaunchKernelGGL(k_mg_coarsen, dim3(grid_for(nc)), dim3(kBlock), 0, s, h.lv[l], h.lv[l + 1]);
     }
-    hipLaunchKernelGGL(k_mg_inverse, dim3(1), dim3(kMgThreads), 0, s, h);
+    hipLaunchKernelGGL(k_mg_setup_coarse, dim3(1), dim3(kMgThreads), 0, s, g, ke, kn, h);
 }
 
 static void mg_down0(hipStream_t s, const MgHier& h, int l, const PcgState* st)
