@@ -1098,11 +1098,13 @@ int do_overland_step(dhara_ctx* c, dhara_step_stats* st)
     double* const pp[2] = {c->p2[0], c->p2[1]};
     dh::SolveCtl sc = solve_ctl(c, c->st_olf, c->p.olf_maxiter, dh::grid_for(c->S), false, true);
     sc.lin_tol = c->p.olf_tol;
-    // the *_BLOCK forms on a surface of at most kOlfBlockCells cells: the whole solve in one
-    // workgroup (either preconditioner); multigrid on a surface with tiled levels: the
+    // a multigrid solve that fits one workgroup's registers and LDS (mg_small): the whole solve in one
+    // launch; the *_BLOCK forms on a surface of at most kOlfBlockCells cells: the same with the
+    // surface in memory (either preconditioner); multigrid on a surface with tiled levels: the
     // single-reduction CG, one V-cycle per iteration
-    const bool small = (op == DHARA_OLF_PRECOND_MG_BLOCK || op == DHARA_OLF_PRECOND_JACOBI_BLOCK) &&
-                       c->S <= dh::kOlfBlockCells;
+    const bool chip = mg && dh::mg_small(c->mg);
+    const bool small = chip || ((op == DHARA_OLF_PRECOND_MG_BLOCK || op == DHARA_OLF_PRECOND_JACOBI_BLOCK) &&
+                                c->S <= dh::kOlfBlockCells);
     const bool cg1 = mg && !small && dh::mg_coarse_level(c->mg) > 0;
     if (mg && !small) {
         // z0 = M^-1 r0; its kernel writes the partials the first CG kernel reads
@@ -1114,7 +1116,8 @@ int do_overland_step(dhara_ctx* c, dhara_step_stats* st)
     LAUNCHCHK(c);
     int rc;
     if (small) {   // the whole CG in one workgroup
-        if (mg) dh::launch_olf_mgcg_block(c->s, dh::OlfMgArgs{olf_cg_args(c, c->st_olf), c->mg});
+        if (chip) dh::launch_olf_mgcg_small(c->s, dh::OlfMgArgs{olf_cg_args(c, c->st_olf), c->mg});
+        else if (mg) dh::launch_olf_mgcg_block(c->s, dh::OlfMgArgs{olf_cg_args(c, c->st_olf), c->mg});
         else dh::launch_olf_cg_block(c->s, olf_cg_args(c, c->st_olf));
         LAUNCHCHK(c);
         rc = read_state(c, c->st_olf);

@@ -540,6 +540,12 @@ void launch_olf_mgcg_block(hipStream_t s, const OlfMgArgs& a);
 // One workgroup per model of args[0 .. nmodels-1]; active[m] == 0 skips model m.
 void launch_batched_olf_mgcg_block(hipStream_t s, const OlfMgArgs* args, int nmodels, const int* active);
 
+// The same for surfaces that fit one workgroup's registers and LDS (mg_small: up to 64 x 64 cells and
+// shapes like it), single-reduction form; of h only the levels' sizes are used.
+bool mg_small(const MgHier& h);
+void launch_olf_mgcg_small(hipStream_t s, const OlfMgArgs& a);
+void launch_batched_olf_mgcg_small(hipStream_t s, const OlfMgArgs* args, int nmodels, const int* active);
+
 // z_0 = V-cycle(r_0), w_0 = A z_0, partials of the above (bb_src: the right-hand side).
 void launch_mg_vcycle_cg1_start(hipStream_t s, const MgHier& h, const PcgState* st, double* part,
                                 const double* bb_src, double* w);

@@ -29,6 +29,8 @@
 //     level's aggregates on threads of their own.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace dh {
@@ -38,7 +40,6 @@ constexpr int kMgT = 32;          // tile edge of the large-level kernels (even)
 constexpr int kMgHalo = 2;        // halo in aggregates: the three half-sweeps after the first and the residual
 constexpr int kMgHaloA = 3;       // the four half-sweeps after the prolongation, and A z
 constexpr int kMgThreads = 1024;   // threads of the single-block kernels
-constexpr int kMgExactChunks = kMgThreads / kMgExactCells;   // threads per row of the exact solve
 
 // The first level handled by the single-block kernel: the finest whose aggregates and those of
 // every coarser level (an aggregate of a level is a cell of the next) fit its threads (50 x 50 ...
@@ -490,21 +491,112 @@ __global__ __launch_bounds__(mg_tile_threads(CG1 ? kMgHaloA : kMgHalo)) void k_m
     if constexpr (CG1) block_partials<4, false>(acc, part);
 }
 
+// Dense inverse of level le's operator (at most 64 cells) by Gauss-Jordan elimination; the operator
+// is symmetric positive definite and diagonally dominant, so no pivoting.  A lane holds column
+// `lane` of the rows w, w + 16, w + 32, w + 48 of its wave w in registers: a row's own pivot-column
+// entry is a lane read, and only the pivot row goes through LDS (two buffers, one barrier a
+// step).  With the matrix in LDS and two barriers a step the 49 steps of a 7 x 7 level took 48 us.
+// m[c] receives the inverse's entry (w + 16 c, lane); every thread of a block of kMgThreads calls it.
+constexpr int kMgInvRows = kMgExactCells / (kMgThreads / kWave);   // rows of the inverse per wave
+__device__ __forceinline__ void mg_gauss_jordan(const MgLevel& L, double (&m)[kMgInvRows])
+{
+    constexpr int NE = kMgExactCells, NW = kMgThreads / kWave, PER = kMgInvRows;
+    static_assert(NE == kWave && NE % NW == 0, "a lane is a column, a wave whole rows");
+    __shared__ double row[2][NE];
+    const int nx = L.nx, n = L.nx * L.ny;
+    const int j = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+#pragma unroll
+    for (int c = 0; c < PER; ++c) {
+        const int i = w + c * NW;
+        double v = 0.0;
+        if (i < n && j < n) {
+            if (i == j) v = L.d[i];
+            else if (j == i + 1 && i % nx != nx - 1) v = -L.we[i];
+            else if (i == j + 1 && j % nx != nx - 1) v = -L.we[j];
+            else if (j == i + nx) v = -L.wn[i];
+            else if (i == j + nx) v = -L.wn[j];
+        }
+        m[c] = v;
+    }
+#pragma unroll
+    for (int ck = 0; ck < PER; ++ck)
+        for (int kk = 0; kk < NW; ++kk) {
+            const int k = ck * NW + kk;
+            if (k >= n) break;
+            if (w == kk) row[k & 1][j] = m[ck];
+            __syncthreads();
+            const double pr = row[k & 1][j];
+            const double ip = 1.0 / lane_value(pr, k);
+            const double rk = (j == k ? 1.0 : pr) * ip;   // row k, scaled (its own column holds the inverse)
+#pragma unroll
+            for (int c = 0; c < PER; ++c) {
+                const double f = lane_value(m[c], k);
+                const double v = fma(-f, rk, j == k ? 0.0 : m[c]);
+                m[c] = (c == ck && w == kk) ? rk : v;
+            }
+        }
+}
+
+// Entries (w + 16 c, lane) of an n x n matrix, from or to memory (row pitch n; zeros outside).
+__device__ __forceinline__ void mg_store_inverse(const double (&m)[kMgInvRows], double* out, int n, int pitch)
+{
+    const int j = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+#pragma unroll
+    for (int c = 0; c < kMgInvRows; ++c) {
+        const int i = w + c * (kMgThreads / kWave);
+        if (i < n && j < n) out[i * pitch + j] = m[c];
+    }
+}
+__device__ __forceinline__ void mg_load_inverse(double (&m)[kMgInvRows], const double* inv, int n)
+{
+    const int j = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+#pragma unroll
+    for (int c = 0; c < kMgInvRows; ++c) {
+        const int i = w + c * (kMgThreads / kWave);
+        m[c] = (i < n && j < n) ? inv[i * n + j] : 0.0;
+    }
+}
+
+// ye = inverse * rhs (n entries in LDS), the inverse symmetric and held as above: each wave sums
+// its rows' share of every entry, then one wave the shares.  A barrier before and inside; one must
+// follow before ye is read.
+struct MgExactLds {
+    double pp[kMgThreads / kWave][kMgExactCells], ye[kMgExactCells];
+};
+__device__ __forceinline__ void mg_exact_solve(const double (&m)[kMgInvRows], const double* rhs, int n, MgExactLds& e)
+{
+    const int j = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    constexpr int NW = kMgThreads / kWave;
+    double v = 0.0;
+#pragma unroll
+    for (int c = 0; c < kMgInvRows; ++c) {
+        const int i = w + c * NW;
+        v += m[c] * (i < n ? rhs[i] : 0.0);
+    }
+    e.pp[w][j] = v;
+    __syncthreads();
+    if (w == 0) {
+        double y = 0.0;
+#pragma unroll
+        for (int c = 0; c < NW; ++c) y += e.pp[c][j];
+        e.ye[j] = y;
+    }
+}
+
 // The V-cycle from level lc down to le and back, in one block: reads b of level lc, writes y of
 // level lc (and on level 0 the CG partial sums).  A thread owns one aggregate of one of the levels
 // lc .. le - 1 (all operators are loaded at once at the start), so a phase is a barrier and at most
 // one aggregate's update; the residual sum of thread t's aggregate is cell t of the array of the
-// coarser levels' right-hand sides.  The exact level is solved with the dense inverse, each of its
-// rows by kMgExactChunks threads.  A chain of ~36 dependent phases of ~100 ns; with the operators in
+// coarser levels' right-hand sides.  A chain of ~36 dependent phases of ~100 ns; with the operators in
 // LDS and the levels' cells dealt anew to the threads in every phase it took 26 us (50 x 50 down to
 // 7 x 7).
 __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgState* st, double* part,
                                                           const double* bb_src)
 {
-    constexpr int NE = kMgExactCells, NC = kMgExactChunks, PER = NE / NC;
     // a level of bx x by aggregates takes 4 (bx + 2) (by + 2) slots; a row of n aggregates is the worst
     __shared__ double sx[12 * kMgThreads + 24 * kMgMaxLevels];
-    __shared__ double sb[kMgThreads], ye[NE], pp[NC][NE];
+    __shared__ double sb[kMgThreads];
+    __shared__ MgExactLds ex;
     const int done = st ? st->done : 0;
     const int le = h.le, lc = mg_coarse_first(h);
     const int tid = threadIdx.x;
@@ -540,11 +632,8 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgSta
         }
     }
     const int ne = h.lv[le].nx * h.lv[le].ny;
-    const int er = tid & (NE - 1), ec = tid / NE;   // exact level: row and chunk of this thread
-    double inv[PER];   // the inverse is symmetric: its columns are read for coalesced rows
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-        inv[i] = (er < ne && ec * PER + i < ne) ? h.inv[(ec * PER + i) * ne + er] : 0.0;
+    double inv[kMgInvRows];
+    mg_load_inverse(inv, h.inv, ne);
     if (lc == le && tid < ne) sb[tid] = L.b[tid];
     if (done) return;
     if (has) {
@@ -564,26 +653,14 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgSta
         __syncthreads();
     }
     if (lc == le) __syncthreads();
-    {
-        double v = 0.0;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) v += inv[i] * (ec * PER + i < ne ? sb[eb + ec * PER + i] : 0.0);
-        pp[ec][er] = v;
-        __syncthreads();
-        if (tid < NE) {
-            double y = 0.0;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) y += pp[c][tid];
-            ye[tid] = y;
-        }
-        __syncthreads();
-    }
+    mg_exact_solve(inv, sb + eb, ne, ex);
+    __syncthreads();
     for (int l = le - 1; l >= lc; --l) {
         const bool on = lv == l;
         if (on) {
             double yc;
             if (l + 1 == le) {
-                yc = ye[tid - base];
+                yc = ex.ye[tid - base];
             } else {   // cell (I, J) of the next level, in that level's planes
                 const int cbx = h.lv[l + 2].nx, cby = h.lv[l + 2].ny;
                 const double* cx = sx + xo + 4 * s.plane;
@@ -598,8 +675,8 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgSta
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     if (lc == le) {
         if (tid < ne) {
-            L.y[tid] = ye[tid];
-            acc[0] = sb[tid] * ye[tid];
+            L.y[tid] = ex.ye[tid];
+            acc[0] = sb[tid] * ex.ye[tid];
             acc[1] = sb[tid] * sb[tid];
             if (bb_src) acc[2] = bb_src[tid] * bb_src[tid];
         }
@@ -617,58 +694,6 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgSta
     if (part) block_partials<4, false>(acc, part);
 }
 
-// Dense inverse of level le's operator (at most 64 cells) by Gauss-Jordan elimination; the operator
-// is symmetric positive definite and diagonally dominant, so no pivoting.  A lane holds column
-// `lane` of the rows w, w + 16, w + 32, w + 48 of its wave w in registers: a row's own pivot-column
-// entry is a lane read, and only the pivot row goes through LDS (two buffers, one barrier a
-// step).  With the matrix in LDS and two barriers a step the 49 steps of a 7 x 7 level took 48 us.
-// The result goes to out, row pitch `pitch` (rows and columns < n).  Every thread of a block of
-// kMgThreads calls it; a barrier must follow before out is read.
-__device__ __forceinline__ void mg_gauss_jordan(const MgLevel& L, double* out, int pitch)
-{
-    constexpr int NE = kMgExactCells, NW = kMgThreads / kWave, PER = NE / NW;
-    static_assert(NE == kWave && NE % NW == 0, "a lane is a column, a wave whole rows");
-    __shared__ double row[2][NE];
-    const int nx = L.nx, n = L.nx * L.ny;
-    const int j = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    double m[PER];
-#pragma unroll
-    for (int c = 0; c < PER; ++c) {
-        const int i = w + c * NW;
-        double v = 0.0;
-        if (i < n && j < n) {
-            if (i == j) v = L.d[i];
-            else if (j == i + 1 && i % nx != nx - 1) v = -L.we[i];
-            else if (i == j + 1 && j % nx != nx - 1) v = -L.we[j];
-            else if (j == i + nx) v = -L.wn[i];
-            else if (i == j + nx) v = -L.wn[j];
-        }
-        m[c] = v;
-    }
-#pragma unroll
-    for (int ck = 0; ck < PER; ++ck)
-        for (int kk = 0; kk < NW; ++kk) {
-            const int k = ck * NW + kk;
-            if (k >= n) break;
-            if (w == kk) row[k & 1][j] = m[ck];
-            __syncthreads();
-            const double pr = row[k & 1][j];
-            const double ip = 1.0 / lane_value(pr, k);
-            const double rk = (j == k) ? ip : pr * ip;   // row k, scaled
-#pragma unroll
-            for (int c = 0; c < PER; ++c) {
-                const double f = lane_value(m[c], k);
-                const double v = (j == k) ? -f * ip : m[c] - f * rk;
-                m[c] = (c == ck && w == kk) ? rk : v;
-            }
-        }
-#pragma unroll
-    for (int c = 0; c < PER; ++c) {
-        const int i = w + c * NW;
-        if (i < n && j < n) out[i * pitch + j] = m[c];
-    }
-}
-
 // The operators of the levels below the first one the single-block kernel handles (and level 0's
 // weights when that is level 0), and the exact level's inverse, by one block: a launch per level
 // took longer than their few cells.
@@ -683,7 +708,10 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_setup_coarse(Geo2 g, const do
         mg_coarsen_cells(h.lv[l], h.lv[l + 1], threadIdx.x, blockDim.x);
         __syncthreads();
     }
-    mg_gauss_jordan(h.lv[h.le], h.inv, h.lv[h.le].nx * h.lv[h.le].ny);
+    const int n = h.lv[h.le].nx * h.lv[h.le].ny;
+    double m[kMgInvRows];
+    mg_gauss_jordan(h.lv[h.le], m);
+    mg_store_inverse(m, h.inv, n, n);
 }
 
 // The update of MgUpd as a kernel of its own (surfaces handled entirely by the coarse kernel).
@@ -695,6 +723,365 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_mg(int n, MgUpd u)
         u.x[c] = u.x[c] + alpha * u.p[c];
         u.r_new[c] = u.r_old[c] - alpha * u.q[c];
     }
+}
+
+// ---- the whole multigrid-preconditioned CG of a small surface in one workgroup, on chip ------
+// Surfaces whose level 0 has at most one aggregate per thread (64 x 64 cells).  A thread keeps its
+// level-0 aggregate -- operator, residual, search direction, solution -- in registers for the whole
+// solve; the coarser levels' operators and right-hand sides and every level's planes are in LDS, so
+// after the first loads an iteration moves nothing but register spills.  The iteration is the
+// single-reduction form of the grid-wide solve: one V-cycle, A z and one block reduction, a chain of
+// ~40 barriers bound by LDS latency: 14 us on 64 x 48, where the grid-wide kernels took three
+// launches (26 us) and the set-up three more.
+constexpr int kMgDeepAggs = 384;       // aggregates of levels 1 .. le - 1 together
+constexpr int kMgSmallPlanes = 7168;   // plane slots of all levels together
+constexpr int kMgOps = 16;             // operator values of a coarser aggregate
+struct MgSmallLevel {
+    int bx, by, x, op, b;   // aggregates; first plane slot, operator column, right-hand side entry
+};
+
+__device__ __forceinline__ double olf_we(const Geo2& g, const double* __restrict__ ke, int i, int j)
+{
+    return (i > 0 && j > 0 && i < g.nx - 2 && j < g.ny - 1) ? g.cx * ke[j * g.nx + i] : 0.0;
+}
+__device__ __forceinline__ double olf_wn(const Geo2& g, const double* __restrict__ kn, int i, int j)
+{
+    return (i > 0 && j > 0 && i < g.nx - 1 && j < g.ny - 2) ? g.cy * kn[j * g.nx + i] : 0.0;
+}
+
+__device__ __forceinline__ void b_olf_mgcg_small(const OlfCgArgs& a, const MgHier& h)
+{
+    __shared__ double sx[kMgSmallPlanes], sop[kMgOps * kMgDeepAggs], sb[kMgThreads + kMgDeepAggs];
+    __shared__ MgExactLds ex;
+    __shared__ MgSmallLevel lev[kMgMaxLevels];
+    __shared__ double red[4 * 16];
+    const Geo2 g2 = a.g;
+    const int le = h.le, tid = threadIdx.x;
+    if (tid == 0) {
+        int x = 0, op = 0, b = 0;
+        for (int l = 0; l <= le; ++l) {
+            const int bx = (h.lv[l].nx + 1) / 2, by = (h.lv[l].ny + 1) / 2;
+            lev[l] = MgSmallLevel{bx, by, x, op, b};
+            x += 4 * (bx + 2) * (by + 2);
+            if (l > 0) op += bx * by;
+            if (l > 0) b += h.lv[l].nx * h.lv[l].ny;
+        }
+    }
+    // level 0: the aggregate of this thread
+    const int nx = g2.nx, ny = g2.ny, bx0 = (nx + 1) / 2, by0 = (ny + 1) / 2;
+    const bool on0 = tid < bx0 * by0;
+    const int J0 = on0 ? tid / bx0 : 0, I0 = on0 ? tid - J0 * bx0 : 0;
+    const int gi = 2 * I0, gj = 2 * J0, g = gj * nx + gi;
+    const int off[4] = {0, 1, nx, nx + 1};
+    const MgLevel dims{nx, ny, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    MgIn in = agg_in(dims, gi, gj);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) in.c[c] = in.c[c] && on0;
+    const MgPlanes s0{sx + (J0 + 1) * (bx0 + 2) + I0 + 1, bx0 + 2, (bx0 + 2) * (by0 + 2)};
+    MgAgg A;
+    double p[4] = {}, s[4] = {}, x[4], bb = 0.0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        A.d[c] = ld_if(in.c[c], a.D, g + off[c], 1.0);
+        A.b[c] = ld_if(in.c[c], a.r, g + off[c], 0.0);
+        A.x[c] = 0.0;
+        x[c] = ld_if(in.c[c], a.x, g + off[c], 0.0);
+        const double bc = ld_if(in.c[c], a.b, g + off[c], 0.0);
+        bb += bc * bc;
+    }
+    A.h0 = olf_we(g2, a.ke, gi, gj);
+    A.h1 = olf_we(g2, a.ke, gi, gj + 1);
+    A.w0 = olf_we(g2, a.ke, gi - 1, gj);
+    A.w2 = olf_we(g2, a.ke, gi - 1, gj + 1);
+    A.e1 = olf_we(g2, a.ke, gi + 1, gj);
+    A.e3 = olf_we(g2, a.ke, gi + 1, gj + 1);
+    A.v0 = olf_wn(g2, a.kn, gi, gj);
+    A.v1 = olf_wn(g2, a.kn, gi + 1, gj);
+    A.s0 = olf_wn(g2, a.kn, gi, gj - 1);
+    A.s1 = olf_wn(g2, a.kn, gi + 1, gj - 1);
+    A.n2 = olf_wn(g2, a.kn, gi, gj + 1);
+    A.n3 = olf_wn(g2, a.kn, gi + 1, gj + 1);
+    agg_invert(A);
+    // the coarser operators: each aggregate's cell of the next level (d, east, north couplings)
+    // goes to LDS, the next level's aggregates collect theirs from there
+    double inv[kMgInvRows];
+    {
+        constexpr int CS = kMgThreads;
+        double *cd = sx, *ce = sx + CS, *cn = sx + 2 * CS;   // the planes are not in use yet
+        if (le == 0) {
+            if (on0) {
+                const double we[4] = {A.h0, A.e1, A.h1, A.e3}, wn[4] = {A.v0, A.v1, A.n2, A.n3};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (in.c[c]) {
+                        cd[g + off[c]] = A.d[c];
+                        ce[g + off[c]] = we[c];
+                        cn[g + off[c]] = wn[c];
+                    }
+            }
+        } else if (on0) {
+            cd[tid] = (in.c[0] ? A.d[0] : 0.0) + (in.c[1] ? A.d[1] : 0.0) + (in.c[2] ? A.d[2] : 0.0) +
+                      (in.c[3] ? A.d[3] : 0.0) - 2.0 * (A.h0 + A.h1 + A.v0 + A.v1);
+            ce[tid] = A.e1 + A.e3;
+            cn[tid] = A.n2 + A.n3;
+        }
+        __syncthreads();
+        for (int l = 1; l < le; ++l) {
+            const MgSmallLevel v = lev[l];
+            const MgLevel C{h.lv[l].nx, h.lv[l].ny, cd, ce, cn, nullptr, nullptr, nullptr};
+            double cdn = 0.0, cen = 0.0, cnn = 0.0;
+            const bool on = tid < v.bx * v.by;
+            if (on) {
+                MgAgg t;
+                const int J = tid / v.bx, I = tid - J * v.bx;
+                const MgIn ti = agg_in(C, 2 * I, 2 * J);
+                agg_load(C, 2 * I, 2 * J, ti, t);
+                agg_invert(t);
+                const double o[kMgOps] = {t.di[0], t.di[1], t.di[2], t.di[3], t.h0, t.h1, t.v0, t.v1,
+                                          t.w0, t.w2, t.e1, t.e3, t.s0, t.s1, t.n2, t.n3};
+#pragma unroll
+                for (int q = 0; q < kMgOps; ++q) sop[q * kMgDeepAggs + v.op + tid] = o[q];
+                cdn = (ti.c[0] ? t.d[0] : 0.0) + (ti.c[1] ? t.d[1] : 0.0) + (ti.c[2] ? t.d[2] : 0.0) +
+                      (ti.c[3] ? t.d[3] : 0.0) - 2.0 * (t.h0 + t.h1 + t.v0 + t.v1);
+                cen = t.e1 + t.e3;
+                cnn = t.n2 + t.n3;
+            }
+            __syncthreads();
+            if (on) {
+                cd[tid] = cdn;
+                ce[tid] = cen;
+                cn[tid] = cnn;
+            }
+            __syncthreads();
+        }
+        const MgLevel E{h.lv[le].nx, h.lv[le].ny, cd, ce, cn, nullptr, nullptr, nullptr};
+        mg_gauss_jordan(E, inv);
+        __syncthreads();   // the planes are used from here on
+    }
+    const int ne = h.lv[le].nx * h.lv[le].ny;
+    if (on0) planes_border(s0, I0 == 0, I0 == bx0 - 1, J0 == 0, J0 == by0 - 1);
+    for (int l = 1; l < le; ++l) {
+        const MgSmallLevel v = lev[l];
+        if (tid < v.bx * v.by) {
+            const int J = tid / v.bx, I = tid - J * v.bx;
+            planes_border(MgPlanes{sx + v.x + (J + 1) * (v.bx + 2) + I + 1, v.bx + 2, (v.bx + 2) * (v.by + 2)}, I == 0,
+                          I == v.bx - 1, J == 0, J == v.by - 1);
+        }
+    }
+    // a coarser level's aggregate of this thread, from LDS (only what the caller uses is read)
+    struct Deep {
+        bool on;
+        int I, J;
+        MgIn in;
+        MgPlanes s;
+        const double *o, *b;
+        int nx;
+        __device__ __forceinline__ MgAgg get() const
+        {
+            MgAgg t;
+            auto q = [&](int i) { return o[i * kMgDeepAggs]; };
+            t.di[0] = q(0); t.di[1] = q(1); t.di[2] = q(2); t.di[3] = q(3);
+            t.h0 = q(4); t.h1 = q(5); t.v0 = q(6); t.v1 = q(7);
+            t.w0 = q(8); t.w2 = q(9); t.e1 = q(10); t.e3 = q(11);
+            t.s0 = q(12); t.s1 = q(13); t.n2 = q(14); t.n3 = q(15);
+            t.b[0] = in.c[0] ? b[0] : 0.0;
+            t.b[1] = in.c[1] ? b[1] : 0.0;
+            t.b[2] = in.c[2] ? b[nx] : 0.0;
+            t.b[3] = in.c[3] ? b[nx + 1] : 0.0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) t.x[c] = s.at(c, 0);
+            return t;
+        }
+    };
+    auto deep = [&](int l) {
+        const MgSmallLevel v = lev[l];
+        Deep t;
+        t.on = tid < v.bx * v.by;
+        t.J = t.on ? tid / v.bx : 0;
+        t.I = t.on ? tid - t.J * v.bx : 0;
+        const MgLevel d{h.lv[l].nx, h.lv[l].ny, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+        t.in = agg_in(d, 2 * t.I, 2 * t.J);
+        t.s = MgPlanes{sx + v.x + (t.J + 1) * (v.bx + 2) + t.I + 1, v.bx + 2, (v.bx + 2) * (v.by + 2)};
+        t.o = sop + v.op + (t.on ? tid : 0);
+        t.nx = d.nx;
+        t.b = sb + v.b + 2 * t.J * d.nx + 2 * t.I;
+        return t;
+    };
+    auto sweep = [&](const Deep& t, bool red_cells) {   // one half-sweep and its barrier
+        if (t.on) {
+            MgAgg v = t.get();
+            if (red_cells) red_sweep(v, t.s);
+            else black_sweep(v, t.s);
+        }
+        __syncthreads();
+    };
+    auto vcycle = [&]() {   // A.x = V-cycle(A.b)
+        if (le == 0) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (in.c[c]) sb[g + off[c]] = A.b[c];
+            __syncthreads();
+            mg_exact_solve(inv, sb, ne, ex);
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < 4; ++c) A.x[c] = in.c[c] ? ex.ye[g + off[c]] : 0.0;
+            if (on0) {
+                put_red(A, s0);
+                s0.put(1, A.x[1]);
+                s0.put(2, A.x[2]);
+            }
+            return;
+        }
+        {
+            const double rc = agg_down(A, s0, on0);
+            if (on0) sb[tid] = rc;
+            __syncthreads();
+        }
+        for (int l = 1; l < le; ++l) {
+            const Deep t = deep(l);
+            if (t.on) {
+                MgAgg v = t.get();
+                v.x[0] = v.b[0] * v.di[0];
+                v.x[3] = v.b[3] * v.di[3];
+                put_red(v, t.s);
+            }
+            __syncthreads();
+            sweep(t, false);
+            double u0 = 0.0, u3 = 0.0;
+            if (t.on) {
+                MgAgg v = t.get();
+                red_sums(v, t.s, u0, u3);
+                v.x[0] = (v.b[0] + u0) * v.di[0];
+                v.x[3] = (v.b[3] + u3) * v.di[3];
+                put_red(v, t.s);
+            }
+            __syncthreads();
+            sweep(t, false);
+            if (t.on) {
+                MgAgg v = t.get();
+                double t0, t3;
+                red_sums(v, t.s, t0, t3);
+                sb[lev[l + 1].b + tid] = (t0 - u0) + (t3 - u3);
+            }
+            __syncthreads();
+        }
+        mg_exact_solve(inv, sb + lev[le].b, ne, ex);
+        __syncthreads();
+        // the correction of aggregate (I, J) of level l: that cell of level l + 1
+        auto correction = [&](int l, int I, int J, int t) {
+            if (l + 1 == le) return ex.ye[t];
+            const MgSmallLevel v = lev[l + 1];
+            return sx[v.x + ((J & 1) * 2 + (I & 1)) * (v.bx + 2) * (v.by + 2) + ((J >> 1) + 1) * (v.bx + 2) + (I >> 1) + 1];
+        };
+        for (int l = le - 1; l >= 1; --l) {
+            const Deep t = deep(l);
+            if (t.on) {
+                const double yc = kMgOver * correction(l, t.I, t.J, tid);
+                if (t.in.c[0]) t.s.put(0, t.s.at(0, 0) + yc);
+                if (t.in.c[3]) t.s.put(3, t.s.at(3, 0) + yc);
+            }
+            __syncthreads();
+            sweep(t, false);
+            sweep(t, true);
+            sweep(t, false);
+            sweep(t, true);
+        }
+        if (on0) {
+            const double yc = kMgOver * correction(0, I0, J0, tid);
+            if (in.c[0]) A.x[0] += yc;
+            if (in.c[3]) A.x[3] += yc;
+        }
+        agg_up(A, s0, on0, true);
+    };
+    double w[4] = {};
+    double sums[4];
+    auto cycle = [&]() {   // z = A.x = V-cycle(r), w = A z and the sums (r, z), (r, r), (w, z)
+        vcycle();
+        __syncthreads();
+        double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
+        if (on0) {
+            red_sums(A, s0, t0, t3);
+            black_sums(A, s0, t1, t2);
+        }
+        const double t[4] = {t0, t1, t2, t3};
+        sums[0] = sums[1] = sums[2] = 0.0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            w[c] = in.c[c] ? A.d[c] * A.x[c] - t[c] : 0.0;
+            if (!in.c[c]) continue;
+            sums[0] += A.b[c] * A.x[c];
+            sums[1] += A.b[c] * A.b[c];
+            sums[2] += w[c] * A.x[c];
+        }
+    };
+    cycle();
+    sums[3] = bb;
+    block_reduce<4, false>(sums, red);
+    bb = sums[3];
+    const double tol2 = a.tol * a.tol * bb;
+    double gam_old = 0.0, pi_old = 0.0;
+    int it = 0, conv = 0, nan = !isfinite(bb);
+    for (;;) {
+        const double gam = sums[0], rr = sums[1], del = sums[2];
+        nan |= !isfinite(rr);
+        conv = (rr <= tol2) ? 1 : 0;
+        if (conv || nan || it >= a.maxit) break;
+        const double beta = it == 0 ? 0.0 : gam / gam_old;
+        const double pi = it == 0 ? del : del - beta * beta * pi_old;
+        const double alpha = gam / pi;
+        if (!(pi > 0.0) || !isfinite(alpha) || !isfinite(beta)) {
+            nan = 1;
+            conv = 0;
+            break;
+        }
+        gam_old = gam;
+        pi_old = pi;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            s[c] = w[c] + beta * s[c];
+            A.b[c] -= alpha * s[c];
+            p[c] = A.x[c] + beta * p[c];
+            x[c] += alpha * p[c];
+        }
+        ++it;
+        cycle();
+        sums[3] = 0.0;
+        block_reduce<4, false>(sums, red);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (in.c[c]) a.x[g + off[c]] = x[c];
+    if (tid == 0) {
+        PcgState* st = a.st;
+        st->bb = bb;
+        st->tol2 = tol2;
+        st->iter = it;
+        st->conv = conv && !nan;
+        st->rr = sums[1];
+        st->nan = nan;
+        st->outer_conv = conv && !nan;
+        st->done = 1;
+    }
+}
+
+__global__ __launch_bounds__(kMgThreads) void k_olf_mgcg_small(OlfMgArgs a)
+{
+    b_olf_mgcg_small(a.cg, a.h);
+}
+
+// One workgroup per model; models whose flag is off return.
+__global__ __launch_bounds__(kMgThreads) void kb_olf_mgcg_small(const OlfMgArgs* __restrict__ args,
+                                                               const int* __restrict__ active)
+{
+    if (active && !active[blockIdx.x]) return;
+    __shared__ MgHier hs;
+    __shared__ OlfCgArgs cs;
+    if (threadIdx.x == 0) {
+        hs = args[blockIdx.x].h;
+        cs = args[blockIdx.x].cg;
+    }
+    __syncthreads();
+    b_olf_mgcg_small(cs, hs);
 }
 
 // ---- the multigrid-preconditioned CG of a small surface in one workgroup -----------------
@@ -802,7 +1189,11 @@ __device__ __forceinline__ void b_olf_mgcg_block(const OlfCgArgs& a, const MgHie
         mg_coarsen_cells(h.lv[l], h.lv[l + 1], tid, nt);
         __syncthreads();
     }
-    mg_gauss_jordan(h.lv[h.le], Minv, kMgExactCells);
+    {
+        double m[kMgInvRows];
+        mg_gauss_jordan(h.lv[h.le], m);
+        mg_store_inverse(m, Minv, h.lv[h.le].nx * h.lv[h.le].ny, kMgExactCells);
+    }
     __syncthreads();
     const double* __restrict__ b = a.b;
     double* __restrict__ x = a.x;
@@ -986,6 +1377,29 @@ void launch_mg_vcycle_cg1_start(hipStream_t s, const MgHier& h, const PcgState* 
 {
     mg_down0(s, h, 0, st);
     mg_vcycle_cg1_rest(s, h, st, part, bb_src, w);
+}
+
+bool mg_small(const MgHier& h)
+{
+    int deep = 0, planes = 0;
+    for (int l = 0; l < std::max(h.le, 1); ++l) {
+        const int bx = (h.lv[l].nx + 1) / 2, by = (h.lv[l].ny + 1) / 2;
+        if (l == 0 && bx * by > kMgThreads) return false;
+        if (l > 0) deep += bx * by;
+        planes += 4 * (bx + 2) * (by + 2);
+    }
+    return deep <= kMgDeepAggs && planes <= kMgSmallPlanes;
+}
+
+void launch_olf_mgcg_small(hipStream_t s, const OlfMgArgs& a)
+{
+    hipLaunchKernelGGL(k_olf_mgcg_small, dim3(1), dim3(kMgThreads), 0, s, a);
+}
+
+void launch_batched_olf_mgcg_small(hipStream_t s, const OlfMgArgs* args, int nmodels, const int* active)
+{
+    if (nmodels > 0)
+        hipLaunchKernelGGL(kb_olf_mgcg_small, dim3(nmodels), dim3(kMgThreads), 0, s, args, active);
 }
 
 void launch_olf_mgcg_block(hipStream_t s, const OlfMgArgs& a)
