@@ -217,17 +217,14 @@ def calibrate_copy():
 
 
 def aa_pass_bytes(npass, depth, mixed):
-    """Algorithmic bytes per cell of the Anderson passes of one step (k_aa_column after every
-    Picard iteration but the last).  Pass j holds min(j, depth) ring columns; its first sweep
-    reads x, psi_m (+ f, y of the previous pass and the ring's older columns) and writes f, y
-    (+ the new ring column of dF and dY), its second reads y, the ring's dY and Ks and writes
-    psi_m, theta, K, C (+ K32)."""
+    """Algorithmic bytes per cell of the Anderson passes of one step (k_picard_next after every
+    Picard iteration but the last).  Pass j combines min(j, depth) earlier passes; its first sweep
+    reads x, psi_m and the ring's f and writes f, y, its second reads the ring's y and Ks and
+    writes psi_m, theta, K, C (+ K32)."""
     total = 0
     for j in range(npass):
-        have = 1 if j > 0 else 0
         nc = min(j, depth)
-        total += 8 * (2 + 2 * have + max(nc - 1, 0)) + 8 * (2 + 2 * have)
-        total += 8 * (2 + nc) + 8 * 4 + (4 if mixed else 0)
+        total += 8 * (2 + nc + 2) + 8 * (nc + 1) + 8 * 4 + (4 if mixed else 0)
     return total
 
 

@@ -120,32 +120,16 @@ static_assert(dh::kAaMaxDepth == DHARA_PICARD_ACCEL_MAX, "Anderson ring size");
 int alloc_aa(dhara_ctx* c)
 {
     int rc;
-    if (!c->aa_f && ((rc = dalloc(c, &c->aa_f, (size_t)c->N)) || (rc = dalloc(c, &c->aa_y, (size_t)c->N))))
-        return rc;
-    for (int i = 0; i < c->p.picard_accel; ++i) {
-        if (!c->aa_df[i] && ((rc = dalloc(c, &c->aa_df[i], (size_t)c->N)) || (rc = dalloc(c, &c->aa_dy[i], (size_t)c->N))))
-            return rc;
+    for (int i = 0; i <= c->p.picard_accel; ++i) {
+        if (!c->aa_f[i] && (rc = dalloc(c, &c->aa_f[i], (size_t)c->N))) return rc;
+        if (!c->aa_y[i] && (rc = dalloc(c, &c->aa_y[i], (size_t)c->N))) return rc;
     }
     return DHARA_OK;
 }
 
-dh::AaArgs aa_args(dhara_ctx* c, const dh::PcgState* st)
+dh::AaArgs aa_args(dhara_ctx* c)
 {
-    const int depth = c->p.picard_accel;
-    int nc = c->aa_ncols;
-    int order[dh::kAaMaxDepth];
-    for (int i = 0; i < nc; ++i) order[i] = c->aa_order[i];
-    if (c->aa_have) {   // the new difference: a free slot, or the oldest column's once full
-        int slot = nc;
-        if (nc == depth) {
-            slot = order[0];
-            for (int i = 1; i < nc; ++i) order[i - 1] = order[i];
-            --nc;
-        }
-        order[nc++] = slot;
-    }
-    c->aa_pend_ncols = nc;
-    for (int i = 0; i < nc; ++i) c->aa_pend_order[i] = order[i];
+    const int depth = c->p.picard_accel, slots = depth + 1;
     dh::AaArgs a{};
     a.g = c->g;
     a.soil = soil_of(c);
@@ -155,19 +139,13 @@ dh::AaArgs aa_args(dhara_ctx* c, const dh::PcgState* st)
     a.K = c->K;
     a.C = c->C;
     a.K32 = c->K32;
-    a.f_prev = c->aa_f;
-    a.y_prev = c->aa_y;
-    for (int t = 0; t < nc; ++t) {   // newest first
-        a.df[t] = c->aa_df[order[nc - 1 - t]];
-        a.dy[t] = c->aa_dy[order[nc - 1 - t]];
+    a.ncols = std::min(c->aa_count, depth);
+    for (int i = 0; i <= a.ncols; ++i) {   // newest first
+        a.f[i] = c->aa_f[(c->aa_count - i) % slots];
+        a.y[i] = c->aa_y[(c->aa_count - i) % slots];
     }
-    a.ncols = nc;
-    a.have = c->aa_have;
     a.beta = 1.0 - c->p.am;
     a.active = c->aa_active;
-    a.red = c->dred;
-    a.tol = c->p.picard_tol;
-    a.st = st;
     return a;
 }
 
@@ -184,31 +162,31 @@ void queue_picard_pass(dhara_ctx* c, const dh::PcgState* gate)
     if (inc_only) dh::launch_picard_inc(c->s, va, gate);
     else if (gate) dh::launch_vg_picard_gated(c->s, va, gate);
     else dh::launch_vg_picard(c->s, va);
-    dh::launch_max_rows2(c->s, c->part[0], dh::grid_for(c->N), c->dred);
-    if (aa) {
-        const dh::LaunchEv ev{c->prof ? c->aa_ev[0] : nullptr, c->prof ? c->aa_ev[1] : nullptr};
-        dh::launch_aa_column(c->s, aa_args(c, gate), c->p.picard_accel, &ev);
+    if (!aa) {
+        dh::launch_max_rows2(c->s, c->part[0], dh::grid_for(c->N), c->dred);
+        return;
     }
-    if (inc_only) dh::launch_vg_final(c->s, va, c->dred, c->p.picard_tol, c->aa_active, gate);
+    const dh::LaunchEv ev{c->prof ? c->aa_ev[0] : nullptr, c->prof ? c->aa_ev[1] : nullptr};
+    dh::NextArgs na{};
+    na.aa = aa_args(c);
+    na.vg = va;
+    na.part = c->part[0];
+    na.nparts = dh::grid_for(c->N);
+    na.fin = inc_only ? 1 : 0;
+    na.tol = c->p.picard_tol;
+    na.red = c->dred;
+    na.st = gate;
+    dh::launch_picard_next(c->s, na, c->p.picard_accel, &ev);
 }
 
-// Algorithmic HBM bytes of the Anderson pass about to be adopted (ring of aa_pend_ncols columns,
-// a previous pass of this step or not): sweep 1 reads x, psi_m (+ f, y, the older columns) and
-// writes f, y (+ the new column of dF and dY); sweep 2 reads y, the ring's dY, Ks (+ alpha, n)
-// and writes psi_m, theta, K, C (+ K32).
+// Algorithmic HBM bytes of the Anderson pass about to be counted: sweep 1 reads x, psi_m and the
+// ring's f and writes f, y; sweep 2 reads the ring's y, Ks (+ alpha, n) and writes psi_m, theta, K,
+// C (+ K32).
 double aa_pass_bytes(const dhara_ctx* c)
 {
-    const int h = c->aa_have ? 1 : 0, nc = c->aa_pend_ncols;
-    const double arrays = (2 + 2 * h + std::max(nc - 1, 0)) + (2 + 2 * h) + (2 + nc + (c->has_alpha ? 1 : 0) +
-                          (c->has_n ? 1 : 0)) + 4;
+    const int nc = std::min(c->aa_count, c->p.picard_accel);
+    const double arrays = (2 + nc) + 2 + (nc + 1 + (c->has_alpha ? 1 : 0) + (c->has_n ? 1 : 0)) + 4;
     return (double)c->N * (8.0 * arrays + (c->K32 ? 4.0 : 0.0));
-}
-
-void aa_commit(dhara_ctx* c)
-{
-    c->aa_have = 1;
-    c->aa_ncols = c->aa_pend_ncols;
-    for (int i = 0; i < c->aa_ncols; ++i) c->aa_order[i] = c->aa_pend_order[i];
 }
 
 int validate_params(dhara_ctx* c, const dhara_params* p)
@@ -912,8 +890,7 @@ int do_subsurface_step(dhara_ctx* c, dhara_step_stats* st)
     if (aa) {
         int rc = alloc_aa(c);
         if (rc) return rc;
-        c->aa_have = 0;
-        c->aa_ncols = 0;
+        c->aa_count = 0;
     }
     if (c->p.am != 0.0 || aa)
         HIPCHK(c, hipMemcpyAsync(c->psi_m, c->psi_n, (size_t)c->N * 8, hipMemcpyDeviceToDevice, c->s));
@@ -972,7 +949,7 @@ int do_subsurface_step(dhara_ctx* c, dhara_step_stats* st)
                     c->prof_acc.aa_launches += 1;
                     c->prof_acc.aa_bytes += aa_pass_bytes(c);
                 }
-                aa_commit(c);   // the pass has run: psi^m, theta^m, K, C of the next iterate
+                ++c->aa_count;   // the pass has run: psi^m, theta^m, K, C of the next iterate
             } else if (c->p.am == 0.0) {
                 std::swap(c->theta_m, c->theta_new);
             } else {
@@ -1099,10 +1076,10 @@ int do_overland_step(dhara_ctx* c, dhara_step_stats* st)
     dh::SolveCtl sc = solve_ctl(c, c->st_olf, c->p.olf_maxiter, dh::grid_for(c->S), false, true);
     sc.lin_tol = c->p.olf_tol;
     // a multigrid solve that fits one workgroup's registers and LDS (mg_small): the whole solve in one
-    // launch; the *_BLOCK forms on a surface of at most kOlfBlockCells cells: the same with the
-    // surface in memory (either preconditioner); multigrid on a surface with tiled levels: the
+    // launch; the *_BLOCK forms on a surface of at most kOlfBlockCells cells: the ensemble's
+    // one-workgroup solve with the surface in memory (either preconditioner); multigrid on a surface with tiled levels: the
     // single-reduction CG, one V-cycle per iteration
-    const bool chip = mg && dh::mg_small(c->mg);
+    const bool chip = op == DHARA_OLF_PRECOND_MG && dh::mg_small(c->mg);
     const bool small = chip || ((op == DHARA_OLF_PRECOND_MG_BLOCK || op == DHARA_OLF_PRECOND_JACOBI_BLOCK) &&
                                 c->S <= dh::kOlfBlockCells);
     const bool cg1 = mg && !small && dh::mg_coarse_level(c->mg) > 0;

@@ -60,14 +60,12 @@ struct dhara_ctx {
     double* h_red = nullptr;  // pinned: the Picard increment and NaN flag of a k_vg_picard queued
                               // by the linear solve (vg_ready)
     bool vg_ready = false;    // the solve ended with k_vg_picard already run, h_red its maxima
-    // Anderson-accelerated Picard update (picard_accel > 0; allocated on first use): f and y of
-    // the last pass and the ring of their differences.  aa_order lists the ring's slots oldest
-    // first; aa_pend_* is the ring after the pass queued last, adopted once it has run.
-    double *aa_f = nullptr, *aa_y = nullptr;
-    double* aa_df[dh::kAaMaxDepth] = {};
-    double* aa_dy[dh::kAaMaxDepth] = {};
-    int aa_have = 0, aa_ncols = 0, aa_pend_ncols = 0;
-    int aa_order[dh::kAaMaxDepth] = {}, aa_pend_order[dh::kAaMaxDepth] = {};
+    // Anderson-accelerated Picard update (picard_accel > 0; allocated on first use): the ring of f
+    // and y of the last picard_accel + 1 passes, pass p of a step in slot p mod (picard_accel + 1);
+    // aa_count: passes of this step that have run.
+    double* aa_f[dh::kAaMaxDepth + 1] = {};
+    double* aa_y[dh::kAaMaxDepth + 1] = {};
+    int aa_count = 0;
     int aa_active = 0;        // the Picard pass after the current solve may update (not the last)
     hipEvent_t aa_ev[2] = {nullptr, nullptr};   // kernel timestamps of the last queued pass (profiling)
     dh::PcgState* st_sub = nullptr;
@@ -140,11 +138,9 @@ dh::SurfArgs surf_args(dhara_ctx* c);
 dh::AsmArgs asm_args(dhara_ctx* c, bool dir);
 int alloc_mixed(dhara_ctx* c);
 int alloc_line(dhara_ctx* c, bool mixed);
-// Anderson pass after the current solve: its arguments (the ring as it will be once the pass has
-// run, gated on st->gate == 2 when st is set) and the adoption of that ring
+// Anderson pass after the current solve
 int alloc_aa(dhara_ctx* c);
-dh::AaArgs aa_args(dhara_ctx* c, const dh::PcgState* st);
-void aa_commit(dhara_ctx* c);
+dh::AaArgs aa_args(dhara_ctx* c);
 void queue_picard_pass(dhara_ctx* c, const dh::PcgState* gate);
 dh::SolveCtl solve_ctl(dhara_ctx* c, dh::PcgState* st, int maxit, int nparts, bool mixed_inner,
                        bool first_sweep);

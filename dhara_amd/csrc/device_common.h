@@ -89,48 +89,52 @@ __device__ __forceinline__ int lin_tid() { return threadIdx.x + threadIdx.y * bl
 __device__ __forceinline__ int lin_nthreads() { return blockDim.x * blockDim.y; }
 __device__ __forceinline__ int lin_bid() { return blockIdx.x + blockIdx.y * gridDim.x; }
 
-// Lane moves of the wave reductions through the data-parallel primitives (a few cycles each; the
-// LDS-permute butterfly they replace waited ~100 cycles in each of its six steps, which the small
-// launches of a solve paid twice per reduction).  CTRL: the DPP control; lanes without a source,
-// or in a row that ROWS masks out, get `other`.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_move(double v, double other)
+// Reduction over the wave (all 64 lanes take part), the result in every lane: a butterfly from
+// distance 32 down.  The half waves and the rows of 16 lanes are exchanged by the lane swaps, the
+// rest by moves within a row, a few cycles each; LDS permutes waited ~100 cycles in each of the
+// six steps, which the small launches of a solve paid twice per reduction.  (Within a row, rotating
+// by 8 is lane ^ 8; after that step lanes 8 apart agree, so rotating by 4 gives lane ^ 4.)
+template <int CTRL>
+__device__ __forceinline__ double row_move(double v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(other), __double2loint(v), CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(other), __double2hiint(v), CTRL, ROWS, 0xf, false);
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
     return __hiloint2double(hi, lo);
+}
+
+template <class Op>
+__device__ __forceinline__ double wave_reduce(double v, Op op)
+{
+    {   // element 0 holds the lower half's (even rows') values on both sides, element 1 the others'
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = op(__hiloint2double(hi[0], lo[0]), __hiloint2double(hi[1], lo[1]));
+    }
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = op(__hiloint2double(hi[0], lo[0]), __hiloint2double(hi[1], lo[1]));
+    }
+    v = op(v, row_move<0x128>(v));   // rotate by 8
+    v = op(v, row_move<0x124>(v));   // rotate by 4
+    v = op(v, row_move<0x4e>(v));    // quad [2, 3, 0, 1]
+    return op(v, row_move<0xb1>(v));   // quad [1, 0, 3, 2]
+}
+
+__device__ __forceinline__ double wave_sum(double v)
+{
+    return wave_reduce(v, [](double a, double b) { return a + b; });
+}
+
+__device__ __forceinline__ double wave_max(double v)
+{
+    return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
 }
 
 __device__ __forceinline__ double lane_value(double v, int lane)
 {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                             __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-
-constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;   // within rows of 16
-constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;   // last lane of a row / of two rows to the next
-
-// Total over the wave (all 64 lanes take part), in every lane.
-__device__ __forceinline__ double wave_sum(double v)
-{
-    v += dpp_move<kDppShr1, 0xf>(v, 0.0);
-    v += dpp_move<kDppShr2, 0xf>(v, 0.0);
-    v += dpp_move<kDppShr4, 0xf>(v, 0.0);
-    v += dpp_move<kDppShr8, 0xf>(v, 0.0);
-    v += dpp_move<kDppBcast15, 0xa>(v, 0.0);
-    v += dpp_move<kDppBcast31, 0xc>(v, 0.0);
-    return lane_value(v, kWave - 1);
-}
-
-__device__ __forceinline__ double wave_max(double v)
-{
-    v = fmax(v, dpp_move<kDppShr1, 0xf>(v, v));
-    v = fmax(v, dpp_move<kDppShr2, 0xf>(v, v));
-    v = fmax(v, dpp_move<kDppShr4, 0xf>(v, v));
-    v = fmax(v, dpp_move<kDppShr8, 0xf>(v, v));
-    v = fmax(v, dpp_move<kDppBcast15, 0xa>(v, v));
-    v = fmax(v, dpp_move<kDppBcast31, 0xc>(v, v));
-    return lane_value(v, kWave - 1);
 }
 
 // Block reduction of NV values, the result in every thread: each wave leaves its totals in LDS and,

@@ -64,7 +64,7 @@ struct dhara_ensemble {
     dh::OlfArgs* a_olf = nullptr;
     dh::OlfCgArgs* a_ocg = nullptr;   // one-workgroup overland solves (olf_kind 1, 2)
     dh::OlfMgArgs* a_omg = nullptr;
-    int *olf_jac = nullptr, *olf_mgm = nullptr, *olf_mgs = nullptr;   // per-member masks of those launches
+    int *olf_jac = nullptr, *olf_mgm = nullptr;   // per-member masks of those launches
     void* a_k3 = nullptr;
     dh::KrylovArgs<double>* a_k2 = nullptr;
     std::vector<dh::VgArgs> h_vg;
@@ -76,7 +76,7 @@ struct dhara_ensemble {
     std::vector<dh::OlfCgArgs> h_ocg;
     std::vector<dh::OlfMgArgs> h_omg;
     // each member's overland form: a surface of at most kOlfBlockCells cells the one-workgroup
-    // solve (1: Jacobi, 2: multigrid, 3: multigrid on chip, mg_small), one launch for all such members, each workgroup to its
+    // solve (1: Jacobi, 2: multigrid), one launch for all such members, each workgroup to its
     // own member's stopping point; a larger one (0) the batched lockstep Jacobi-PCG
     std::vector<int> olf_kind;
     std::vector<dh::KrylovArgs<double>> h_k3d, h_k2;
@@ -105,7 +105,6 @@ struct dhara_ensemble {
     // batched pass over aa_blocks(g) blocks per member
     int aa_depth = 0;
     dh::BlkMap* map_aa = nullptr;
-    int nb_aa = 0;
     dh::AaArgs* a_aa = nullptr;
     std::vector<dh::AaArgs> h_aa;
     // Block maps restricted to the active members: a batched launch over the full map spends a
@@ -628,8 +627,7 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         dhara_ctx* c = e->mem[m];
         if (c->p.am != 0.0 || e->aa_depth)
             EHIP(e, hipMemcpyAsync(c->psi_m, c->psi_n, (size_t)c->N * 8, hipMemcpyDeviceToDevice, e->s));
-        c->aa_have = 0;
-        c->aa_ncols = 0;
+        c->aa_count = 0;
         e->h_surf[m] = surf_args(c);
     }
     std::vector<int> all(M, 1), surf(M, 0);
@@ -771,9 +769,8 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
                 if (!accel[m]) continue;
                 dhara_ctx* c = e->mem[m];
                 c->aa_active = 1;
-                e->h_aa[m] = aa_args(c, nullptr);
-                e->h_aa[m].red = nullptr;   // decided here
-                aa_commit(c);
+                e->h_aa[m] = aa_args(c);
+                ++c->aa_count;
             }
             if ((rc = upload_args(e, e->a_aa, e->h_aa)) || (rc = set_active(e, accel))) return rc;
             const MapRef r = use_map(e, e->cmaa);
@@ -858,7 +855,6 @@ int overland_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         const bool mg = op == DHARA_OLF_PRECOND_MG || op == DHARA_OLF_PRECOND_MG_BLOCK;
         e->olf_kind[m] = c->S > dh::kOlfBlockCells ? 0 : mg ? 2 : 1;
         if (e->olf_kind[m] == 2 && (rc = ensure_mg(c))) return eset(e, rc, c->err);
-        if (e->olf_kind[m] == 2 && dh::mg_small(c->mg)) e->olf_kind[m] = 3;
     }
     for (int m = 0; m < M; ++m) {
         dhara_ctx* c = e->mem[m];
@@ -874,29 +870,25 @@ int overland_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         k.spmv = ctl(c, &e->st[M + m], c->p.olf_maxiter, c->p.olf_tol, false, true, c->part[0], np, c->part[1]);
         k.upd = ctl(c, &e->st[M + m], c->p.olf_maxiter, c->p.olf_tol, false, true, c->part[1], np, c->part[0]);
         e->h_ocg[m] = olf_cg_args(c, &e->st[M + m]);
-        if (e->olf_kind[m] >= 2) e->h_omg[m] = dh::OlfMgArgs{e->h_ocg[m], c->mg};
+        if (e->olf_kind[m] == 2) e->h_omg[m] = dh::OlfMgArgs{e->h_ocg[m], c->mg};
     }
-    std::vector<int> jac(M, 0), mgm(M, 0), mgs(M, 0), lock(M, 0);
+    std::vector<int> jac(M, 0), mgm(M, 0), lock(M, 0);
     for (int m = 0; m < M; ++m) {
         jac[m] = on[m] && e->olf_kind[m] == 1;
         mgm[m] = on[m] && e->olf_kind[m] == 2;
-        mgs[m] = on[m] && e->olf_kind[m] == 3;
         lock[m] = on[m] && e->olf_kind[m] == 0;
     }
     const bool any_jac = std::count(jac.begin(), jac.end(), 1) > 0, any_mg = std::count(mgm.begin(), mgm.end(), 1) > 0;
-    const bool any_small = std::count(mgs.begin(), mgs.end(), 1) > 0;
     const bool any_lock = std::count(lock.begin(), lock.end(), 1) > 0;
     if ((rc = upload_args(e, e->a_olf, e->h_olf)) || (rc = upload_args(e, e->a_k2, e->h_k2)) || (rc = set_active(e, on)))
         return rc;
     if ((any_jac && ((rc = upload_args(e, e->a_ocg, e->h_ocg)) || (rc = upload_args(e, e->olf_jac, jac)))) ||
-        ((any_mg || any_small) && (rc = upload_args(e, e->a_omg, e->h_omg))) ||
-        (any_mg && (rc = upload_args(e, e->olf_mgm, mgm))) || (any_small && (rc = upload_args(e, e->olf_mgs, mgs))))
+        (any_mg && ((rc = upload_args(e, e->a_omg, e->h_omg)) || (rc = upload_args(e, e->olf_mgm, mgm)))))
         return rc;
     const MapRef r2 = use_map(e, e->cm2);
     dh::launch_batched(e->s, dh::BK_OLF_FACES, e->a_olf, r2.map, r2.n, e->active);
     dh::launch_batched(e->s, dh::BK_OLF_ASM, e->a_olf, r2.map, r2.n, e->active);
     if (any_mg) dh::launch_batched_olf_mgcg_block(e->s, e->a_omg, M, e->olf_mgm);
-    if (any_small) dh::launch_batched_olf_mgcg_small(e->s, e->a_omg, M, e->olf_mgs);
     if (any_jac) dh::launch_batched_olf_cg_block(e->s, e->a_ocg, M, e->olf_jac);
     EHIP(e, hipGetLastError());
     // the lockstep solve reads every member's state after its batches; without it, read them here
@@ -1010,7 +1002,7 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
         (rc = ealloc(e, &e->a_surf, n)) || (rc = ealloc(e, &e->a_asm, n)) || (rc = ealloc(e, &e->a_ref, n)) ||
         (rc = ealloc(e, &e->a_end, n)) || (rc = ealloc(e, &e->a_olf, n)) || (rc = ealloc(e, &e->a_k2, n)) ||
         (rc = ealloc(e, &e->a_ocg, n)) || (rc = ealloc(e, &e->a_omg, n)) || (rc = ealloc(e, &e->olf_jac, n)) ||
-        (rc = ealloc(e, &e->olf_mgm, n)) || (rc = ealloc(e, &e->olf_mgs, n))) {
+        (rc = ealloc(e, &e->olf_mgm, n))) {
         dhara_ensemble_destroy(e);
         return rc;
     }
@@ -1027,14 +1019,13 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
         if (e->nb_l[b] && !(rc = ealloc(e, &e->map_l[b], ml[b].size()))) rc = upload(e, e->map_l[b], ml[b]);
     }
     e->aa_depth = e->mem[0]->p.picard_accel;
+    std::vector<dh::BlkMap> ma;
     if (!rc && e->aa_depth > 0) {
-        std::vector<dh::BlkMap> ma;
         for (int m = 0; m < n && !rc; ++m) {
             const int nb = dh::aa_blocks(e->mem[m]->g);
             for (int b = 0; b < nb; ++b) ma.push_back(dh::BlkMap{m, b, nb});
             rc = alloc_aa(e->mem[m]);
         }
-        e->nb_aa = (int)ma.size();
         if (!rc) rc = ealloc(e, &e->map_aa, ma.size());
         if (!rc) rc = upload(e, e->map_aa, ma);
         if (!rc) rc = ealloc(e, &e->a_aa, n);
@@ -1059,14 +1050,7 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
         dhara_ensemble_destroy(e);
         return rc;
     }
-    if (e->aa_depth > 0) {
-        std::vector<dh::BlkMap> ma;
-        for (int m = 0; m < n; ++m) {
-            const int nb = dh::aa_blocks(e->mem[m]->g);
-            for (int b = 0; b < nb; ++b) ma.push_back(dh::BlkMap{m, b, nb});
-        }
-        if ((rc = init_cmap(e, e->cmaa, e->map_aa, ma))) { dhara_ensemble_destroy(e); return rc; }
-    }
+    if ((rc = init_cmap(e, e->cmaa, e->map_aa, ma))) { dhara_ensemble_destroy(e); return rc; }
     std::vector<dh::PcgState> zero(2 * n);
     if ((rc = upload(e, e->st, zero))) { dhara_ensemble_destroy(e); return rc; }
     e->h_vg.resize(n); e->h_surf.resize(n); e->h_asm.resize(n); e->h_ref.resize(n); e->h_end.resize(n);

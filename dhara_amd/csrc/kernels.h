@@ -96,10 +96,10 @@ struct VgArgs {
     double* part_out;        // Picard pass: [max increment, NaN flag] per block (host-reduced)
 };
 
-// Anderson-accelerated Picard update, one thread per column of cells (k_aa_column).  The
-// increment f = x - psi^m and relaxed update y = psi^m + beta f of this pass, their differences
-// with those of the previous pass (one new column of the ring) and, per column of cells, the
-// least-squares coefficients over the ring; then psi^m <- y - dY gamma and theta, K, C at it.
+// Anderson-accelerated Picard update (k_picard_next).  The increment f = x - psi^m and relaxed
+// update y = psi^m + beta f of this pass and of the last ncols passes, whose differences are the
+// columns of dF and dY; per column of cells, the least-squares coefficients over them; then
+// psi^m <- y - dY gamma and theta, K, C at it.
 constexpr int kAaMaxDepth = 5;  // = DHARA_PICARD_ACCEL_MAX
 constexpr double kAaDrop = 1e-3;   // a ring column is left out when its part orthogonal to the
                                    // newer ones is below this fraction of its norm
@@ -112,19 +112,25 @@ struct AaArgs {
     double* K;
     double* C;
     float* K32;
-    double* f_prev;          // in: f, y of the previous pass (when have), out: of this pass
-    double* y_prev;
-    double* df[kAaMaxDepth]; // ring columns, NEWEST first; df[0] / dy[0] are written (when have)
-    double* dy[kAaMaxDepth];
-    int ncols;               // columns after this pass (0 when !have)
-    int have;                // f_prev, y_prev hold a previous pass of this step
+    double* f[kAaMaxDepth + 1];   // f of this pass (written) and of the previous ncols passes, newest first
+    double* y[kAaMaxDepth + 1];   // y likewise
+    int ncols;               // previous passes of this step in the ring, at most the depth
     double beta;             // 1 - am
-    // gates: the pass runs only when active, red[1] (NaN flag) == 0, red[0] (the Picard
-    // increment) >= tol and, with st set, st->gate == 2 (queued behind a mixed solve); with red
-    // null the host has decided and only `active` counts
-    int active;
-    const double* red;
+    int active;              // the pass may update (not the one at the iteration limit)
+};
+
+// What follows a Picard increment (k_picard_next): the maxima of the increment's block partials
+// [increment, NaN flag] to red; then, unless a NaN was seen, the Anderson update when the increment
+// is not below tol (and aa.active), else theta, K, C of the converged x (fin set).  With st the
+// pass was queued behind a solve: nothing runs unless st->gate == 2.
+struct NextArgs {
+    AaArgs aa;
+    VgArgs vg;
+    const double* part;
+    int nparts;
+    int fin;
     double tol;
+    double* red;
     const PcgState* st;
 };
 
@@ -262,14 +268,11 @@ void launch_max_rows2(hipStream_t s, const double* part, int nparts, double* out
 // in st->rr_update), and k_vg_picard run only in that case
 void launch_refine_conv(hipStream_t s, const double* part, int nparts, double lin_tol, PcgState* st);
 void launch_vg_picard_gated(hipStream_t s, const VgArgs& a, const PcgState* st);
-// Anderson pass over the ring of depth `depth` (1..kAaMaxDepth), gated as AaArgs says
-void launch_aa_column(hipStream_t s, const AaArgs& a, int depth, const LaunchEv* ev = nullptr);
-// The Anderson path's Picard pass (rules ABS_PSI / REL_PSI): the increment of a.psi against
-// a.psi_m into a.part_out, and theta, K, C of a.psi after the last pass (red: the increment and
-// NaN flag from launch_max_rows2; active: not the pass at the iteration limit); with st, both
-// run only when st->gate == 2 (queued behind a mixed solve)
+// The Picard pass's second kernel with the Anderson update of depth `depth` (1..kAaMaxDepth)
+void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const LaunchEv* ev = nullptr);
+// Its first kernel for the rules on psi (ABS_PSI / REL_PSI): the increment of a.psi against a.psi_m
+// into a.part_out; with st it runs only when st->gate == 2 (queued behind a mixed solve)
 void launch_picard_inc(hipStream_t s, const VgArgs& a, const PcgState* st);
-void launch_vg_final(hipStream_t s, const VgArgs& a, const double* red, double tol, int active, const PcgState* st);
 void launch_vg_inverse(hipStream_t s, const Geo& g, const Soil& soil, const double* theta,
                        double* psi);
 void launch_row_flags(hipStream_t s, const Geo& g, const int* const bctype[6], uint8_t* flags);
@@ -450,8 +453,8 @@ void launch_batched(hipStream_t s, BatchKind kind, const void* args, const BlkMa
 // the start-up z = T^-1 r of a fresh residual).
 void launch_batched_spmv_z(hipStream_t s, bool fp32, const void* kargs, const BlkMap* map, int nblocks,
                            const int* active, const int* it_base, int k);
-// Anderson pass of the active members (their AaArgs with red = null: the host has decided), over a
-// map of aa_blocks(g) blocks per member; every member has the same depth.
+// Anderson pass of the active members (the host has decided), over a map of aa_blocks(g) blocks
+// per member; every member has the same depth.
 void launch_batched_aa(hipStream_t s, int depth, const AaArgs* args, const BlkMap* map, int nblocks,
                        const int* active);
 int aa_blocks(const Geo& g);
@@ -544,7 +547,6 @@ void launch_batched_olf_mgcg_block(hipStream_t s, const OlfMgArgs* args, int nmo
 // shapes like it), single-reduction form; of h only the levels' sizes are used.
 bool mg_small(const MgHier& h);
 void launch_olf_mgcg_small(hipStream_t s, const OlfMgArgs& a);
-void launch_batched_olf_mgcg_small(hipStream_t s, const OlfMgArgs* args, int nmodels, const int* active);
 
 // z_0 = V-cycle(r_0), w_0 = A z_0, partials of the above (bb_src: the right-hand side).
 void launch_mg_vcycle_cg1_start(hipStream_t s, const MgHier& h, const PcgState* st, double* part,

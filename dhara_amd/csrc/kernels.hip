@@ -131,25 +131,31 @@ __global__ __launch_bounds__(kBlock) void k_vg_picard_gated(VgArgs a, const PcgS
 // out a column whose pivot is below kAaDrop^2 of its diagonal (the pivot is the squared norm of
 // the column's part orthogonal to the newer ones); then psi^m <- y - dY gamma, and theta, K, C
 // at the new iterate (what the next assembly reads).
-// A block owns kAaCols columns of cells; each column is split into kAaChunks runs of planes, one
-// per wave (the 64 lanes of a wave: 64 neighbouring columns, so every plane access is one
-// coalesced row).  Pass 1 streams a thread's planes once (new ring column, f and y kept for the
-// next pass, its share of G and dF^T f), the shares of a column are summed through LDS in chunk
-// order (every thread of the column gets the same sums and the same gamma), pass 2 streams the
-// planes once more (the update and vG).
+// A block owns kAaCols columns of cells; each column is split into kAaChunks runs of planes, one per wave
+// (the 64 lanes of a wave: 64 neighbouring columns, so every plane access is one coalesced
+// row).  Pass 1 streams a thread's planes once (f and y kept for the next passes, the differences of
+// the ring's f formed as they are read, its share of G and dF^T f), the shares of a column are
+// summed through LDS in chunk order (every thread of the column gets the same sums and the same
+// gamma), pass 2 streams the planes once more (the update and vG); this pass's y waits in LDS.
+// The ring holds f and y themselves and not their differences: with a full ring of 3 a pass moves
+// 5 + 2 + 4 + 4 arrays (124 B per cell with K32) instead of 160 B, with the same differences.
+// Bytes bound it: 118 us a launch at 400 x 400 x 30 (672 MB / 130 us with the differences stored),
+// 750 us at 1024 x 1024 x 30 (909 us).  Sixteen chunks instead of four on small surfaces changed nothing.
 constexpr int kAaCols = 64, kAaChunks = kBlock / kAaCols;
+constexpr int kAaLds = 32;   // planes whose y is kept in LDS
 
 // Block `bid` (kAaCols columns of cells) of the pass; every thread of the block calls it.
 template <int M>
 __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
 {
-    constexpr int NV = M * (M + 1) / 2 + M;   // lower triangle of G, then dF^T f
-    __shared__ double share[kAaChunks][NV][kAaCols];
+    constexpr int CH = kAaChunks, NV = M * (M + 1) / 2 + M;   // lower triangle of G, then dF^T f
+    __shared__ double share[CH][NV][kAaCols];
+    __shared__ double ysh[kAaLds][kAaCols];
     const Geo g = a.g;
     const int lane = threadIdx.x % kAaCols, chunk = threadIdx.x / kAaCols;
     const int col = bid * kAaCols + lane;
-    const bool in = col < g.nxy;
-    const int per = (g.nz + kAaChunks - 1) / kAaChunks;
+    const bool in = col < g.nxy, ylds = g.nz <= kAaLds;
+    const int per = (g.nz + CH - 1) / CH;
     const int k0 = min(g.nz, chunk * per), k1 = min(g.nz, k0 + per);
     const int nc = a.ncols;
     double G[M][M], rhs[M];
@@ -164,41 +170,28 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
     // for the previous plane's arithmetic (in pass 2 the van Genuchten evaluation).
     if (in && k0 < k1) {
         int c = k0 * g.nxy + col;
-        double pm = a.psi_m[c], xv = a.x[c], fp = 0.0, yp = 0.0, old[M];
-        if (a.have) {
-            fp = a.f_prev[c];
-            yp = a.y_prev[c];
-        }
+        double pm = a.psi_m[c], xv = a.x[c], fo[M];
 #pragma unroll
-        for (int i = 1; i < M; ++i) old[i] = (i < nc) ? a.df[i][c] : 0.0;
+        for (int i = 0; i < M; ++i) fo[i] = (i < nc) ? a.f[i + 1][c] : 0.0;
         for (int k = k0; k < k1; ++k) {
             const int cn = c + g.nxy;
-            double pm1 = 0.0, x1 = 0.0, fp1 = 0.0, yp1 = 0.0, old1[M];
+            double pm1 = 0.0, x1 = 0.0, fo1[M];
 #pragma unroll
-            for (int i = 1; i < M; ++i) old1[i] = 0.0;
+            for (int i = 0; i < M; ++i) fo1[i] = 0.0;
             if (k + 1 < k1) {
                 pm1 = a.psi_m[cn];
                 x1 = a.x[cn];
-                if (a.have) {
-                    fp1 = a.f_prev[cn];
-                    yp1 = a.y_prev[cn];
-                }
 #pragma unroll
-                for (int i = 1; i < M; ++i) old1[i] = (i < nc) ? a.df[i][cn] : 0.0;
+                for (int i = 0; i < M; ++i) fo1[i] = (i < nc) ? a.f[i + 1][cn] : 0.0;
             }
             const double f = xv - pm;
             const double y = pm + a.beta * f;
+            a.f[0][c] = f;
+            a.y[0][c] = y;
+            if (ylds) ysh[k][lane] = y;
             double v[M];
-            v[0] = 0.0;
-            if (a.have) {
-                v[0] = f - fp;
-                a.df[0][c] = v[0];
-                a.dy[0][c] = y - yp;
-            }
-            a.f_prev[c] = f;
-            a.y_prev[c] = y;
 #pragma unroll
-            for (int i = 1; i < M; ++i) v[i] = old[i];
+            for (int i = 0; i < M; ++i) v[i] = (i == 0 ? f : fo[i - 1]) - fo[i];
 #pragma unroll
             for (int i = 0; i < M; ++i) {
                 if (i < nc) {
@@ -209,10 +202,8 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
             }
             pm = pm1;
             xv = x1;
-            fp = fp1;
-            yp = yp1;
 #pragma unroll
-            for (int i = 1; i < M; ++i) old[i] = old1[i];
+            for (int i = 0; i < M; ++i) fo[i] = fo1[i];
             c = cn;
         }
     }
@@ -234,7 +225,7 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
             for (int j = 0; j <= i; ++j) {
                 double v = 0.0;
 #pragma unroll
-                for (int h = 0; h < kAaChunks; ++h) v += share[h][q][lane];
+                for (int h = 0; h < CH; ++h) v += share[h][q][lane];
                 G[i][j] = v;
                 ++q;
             }
@@ -242,7 +233,7 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
         for (int i = 0; i < M; ++i) {
             double v = 0.0;
 #pragma unroll
-            for (int h = 0; h < kAaChunks; ++h) v += share[h][q][lane];
+            for (int h = 0; h < CH; ++h) v += share[h][q][lane];
             rhs[i] = v;
             ++q;
         }
@@ -299,26 +290,26 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
     const Soil& sl = a.soil;
     if (k0 >= k1) return;
     int c = k0 * g.nxy + col;
-    double yv = a.y_prev[c], ks = sl.Ks[c], al = cell_alpha(sl, c), nv = cell_n(sl, c), dyv[M];
+    double yv = ylds ? ysh[k0][lane] : a.y[0][c], ks = sl.Ks[c], al = cell_alpha(sl, c), nv = cell_n(sl, c), yo[M];
 #pragma unroll
-    for (int t = 0; t < M; ++t) dyv[t] = (t < nc) ? a.dy[t][c] : 0.0;
+    for (int t = 0; t < M; ++t) yo[t] = (t < nc) ? a.y[t + 1][c] : 0.0;
     for (int k = k0; k < k1; ++k) {
         const int cn = c + g.nxy;
-        double y1 = 0.0, ks1 = 0.0, al1 = 0.0, nv1 = 0.0, dy1[M];
+        double y1 = 0.0, ks1 = 0.0, al1 = 0.0, nv1 = 0.0, yo1[M];
 #pragma unroll
-        for (int t = 0; t < M; ++t) dy1[t] = 0.0;
+        for (int t = 0; t < M; ++t) yo1[t] = 0.0;
         if (k + 1 < k1) {
-            y1 = a.y_prev[cn];
+            y1 = ylds ? ysh[k + 1][lane] : a.y[0][cn];
             ks1 = sl.Ks[cn];
             al1 = cell_alpha(sl, cn);
             nv1 = cell_n(sl, cn);
 #pragma unroll
-            for (int t = 0; t < M; ++t) dy1[t] = (t < nc) ? a.dy[t][cn] : 0.0;
+            for (int t = 0; t < M; ++t) yo1[t] = (t < nc) ? a.y[t + 1][cn] : 0.0;
         }
         double v = yv;
 #pragma unroll
         for (int t = 0; t < M; ++t)
-            if (t < nc) v -= gam[t] * dyv[t];
+            if (t < nc) v -= gam[t] * ((t == 0 ? yv : yo[t - 1]) - yo[t]);
         a.psi_m[c] = v;
         double th, K, C;
         vg_eval(v, ks, al, nv, sl.ts, sl.tr, th, K, C);
@@ -331,22 +322,14 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
         al = al1;
         nv = nv1;
 #pragma unroll
-        for (int t = 0; t < M; ++t) dyv[t] = dy1[t];
+        for (int t = 0; t < M; ++t) yo[t] = yo1[t];
         c = cn;
     }
 }
 
-template <int M>
-__global__ __launch_bounds__(kBlock) void k_aa_column(AaArgs a)
-{
-    if (a.st && a.st->gate != 2) return;
-    if (!a.active || (a.red && (a.red[1] > 0.0 || !(a.red[0] >= a.tol)))) return;
-    b_aa_column<M>(a, blockIdx.x);
-}
-
 // The Picard increment of the Anderson path (rules DHARA_PICARD_ABS_PSI / _REL_PSI): the block
 // maxima of |x - psi^m| and the NaN flag only.  theta, K, C of x are needed only after the last
-// pass (k_vg_final); the other passes evaluate them at the next iterate in k_aa_column.
+// pass; the other passes evaluate them at the next iterate (both in k_picard_next).
 __device__ __forceinline__ void b_picard_inc(const double* __restrict__ x, const double* __restrict__ pm, int n,
                                              int rule, double* part_out, Blk bk)
 {
@@ -367,14 +350,28 @@ __global__ __launch_bounds__(kBlock) void k_picard_inc(const double* x, const do
     b_picard_inc(x, pm, n, rule, part_out, hw_blk());
 }
 
-// theta, K, C of x after the last Picard pass of a step (converged, or the pass at the iteration
-// limit), gated as k_aa_column is but the other way round.
-__global__ __launch_bounds__(kBlock) void k_vg_final(VgArgs a, const double* red, double tol, int active,
-                                                       const PcgState* st)
+// After the increment: every block takes its maxima from the block partials (a maximum does not
+// depend on the order), and the launch is the Anderson update or theta, K, C of the converged x, or
+// (a NaN, or rule on theta and converged) neither.  One launch where the maxima, the update and the
+// final evaluation each took one of 2 to 4 us, two of them idle.
+template <int M>
+__global__ __launch_bounds__(kBlock) void k_picard_next(NextArgs a)
 {
-    if (st && st->gate != 2) return;
-    if (red[1] > 0.0 || (active && red[0] >= tol)) return;
-    b_vg(a, hw_blk());
+    if (a.st && a.st->gate != 2) return;
+    __shared__ double lds[2 * 16];
+    double mx[2] = {-INFINITY, -INFINITY};
+    for (int b = threadIdx.x; b < a.nparts; b += blockDim.x) {
+        mx[0] = fmax(mx[0], a.part[b]);
+        mx[1] = fmax(mx[1], a.part[kMaxBlocks + b]);
+    }
+    block_reduce<2, true, false>(mx, lds);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.red[0] = mx[0];
+        a.red[1] = mx[1];
+    }
+    if (mx[1] > 0.0) return;
+    if (a.aa.active && mx[0] >= a.tol) b_aa_column<M>(a.aa, blockIdx.x);
+    else if (a.fin) b_vg(a.vg, hw_blk());
 }
 
 // Maxima of rows 0 and 1 of a partial buffer (nparts blocks each) into out[0], out[1], in one
@@ -2488,6 +2485,14 @@ __global__ __launch_bounds__(kBlock) void kb_cg1(const Cg1Args<T>* __restrict__ 
 // =========================================================================================
 // Launchers
 // =========================================================================================
+// Krylov launches: through hipExtLaunchKernelGGL so that profiling events, when given, carry
+// the kernel's own begin/end timestamps.
+template <typename F, typename... Args>
+static void launch_ev(F kernel, dim3 gr, dim3 bl, hipStream_t s, const LaunchEv& ev, Args... args)
+{
+    hipExtLaunchKernelGGL(kernel, gr, bl, 0, s, ev.start, ev.stop, 0, args...);
+}
+
 void launch_vg(hipStream_t s, const VgArgs& a)
 {
     hipLaunchKernelGGL(k_vg, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
@@ -2503,19 +2508,16 @@ void launch_vg_picard_gated(hipStream_t s, const VgArgs& a, const PcgState* st)
     hipLaunchKernelGGL(k_vg_picard_gated, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a, st);
 }
 
-void launch_aa_column(hipStream_t s, const AaArgs& a, int depth, const LaunchEv* ev)
+void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const LaunchEv* ev)
 {
-    const dim3 grid((a.g.nxy + kAaCols - 1) / kAaCols), block(kBlock);
-    auto go = [&](auto kern) {
-        if (ev && ev->start) hipExtLaunchKernelGGL(kern, grid, block, 0, s, ev->start, ev->stop, 0, a);
-        else hipLaunchKernelGGL(kern, grid, block, 0, s, a);
-    };
+    const dim3 grid(aa_blocks(a.aa.g)), block(kBlock);
+    const LaunchEv e = ev ? *ev : LaunchEv{};
     switch (depth) {
-    case 1: go(k_aa_column<1>); break;
-    case 2: go(k_aa_column<2>); break;
-    case 3: go(k_aa_column<3>); break;
-    case 4: go(k_aa_column<4>); break;
-    default: go(k_aa_column<kAaMaxDepth>); break;
+    case 1: launch_ev(k_picard_next<1>, grid, block, s, e, a); break;
+    case 2: launch_ev(k_picard_next<2>, grid, block, s, e, a); break;
+    case 3: launch_ev(k_picard_next<3>, grid, block, s, e, a); break;
+    case 4: launch_ev(k_picard_next<4>, grid, block, s, e, a); break;
+    default: launch_ev(k_picard_next<kAaMaxDepth>, grid, block, s, e, a); break;
     }
 }
 
@@ -2523,11 +2525,6 @@ void launch_picard_inc(hipStream_t s, const VgArgs& a, const PcgState* st)
 {
     hipLaunchKernelGGL(k_picard_inc, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a.psi, a.psi_m, a.g.n, a.rule,
                        a.part_out, st);
-}
-
-void launch_vg_final(hipStream_t s, const VgArgs& a, const double* red, double tol, int active, const PcgState* st)
-{
-    hipLaunchKernelGGL(k_vg_final, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a, red, tol, active, st);
 }
 
 void launch_refine_conv(hipStream_t s, const double* part, int nparts, double lin_tol, PcgState* st)
@@ -2672,14 +2669,6 @@ int launch_refine_tiled(hipStream_t s, const RefineArgs& a, const TileCfg& t)
 void launch_end_step(hipStream_t s, const EndArgs& a)
 {
     hipLaunchKernelGGL(k_end_step, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
-}
-
-// Krylov launches: through hipExtLaunchKernelGGL so that profiling events, when given, carry
-// the kernel's own begin/end timestamps.
-template <typename F, typename... Args>
-static void launch_ev(F kernel, dim3 gr, dim3 bl, hipStream_t s, const LaunchEv& ev, Args... args)
-{
-    hipExtLaunchKernelGGL(kernel, gr, bl, 0, s, ev.start, ev.stop, 0, args...);
 }
 
 template <typename T>

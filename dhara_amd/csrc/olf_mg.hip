@@ -1069,21 +1069,6 @@ __global__ __launch_bounds__(kMgThreads) void k_olf_mgcg_small(OlfMgArgs a)
     b_olf_mgcg_small(a.cg, a.h);
 }
 
-// One workgroup per model; models whose flag is off return.
-__global__ __launch_bounds__(kMgThreads) void kb_olf_mgcg_small(const OlfMgArgs* __restrict__ args,
-                                                               const int* __restrict__ active)
-{
-    if (active && !active[blockIdx.x]) return;
-    __shared__ MgHier hs;
-    __shared__ OlfCgArgs cs;
-    if (threadIdx.x == 0) {
-        hs = args[blockIdx.x].h;
-        cs = args[blockIdx.x].cg;
-    }
-    __syncthreads();
-    b_olf_mgcg_small(cs, hs);
-}
-
 // ---- the multigrid-preconditioned CG of a small surface in one workgroup -----------------
 // The V-cycle of the grid kernels (same smoother, restriction, coarse correction and exact
 // level), each phase a pass of the block over a level held in global memory, a barrier between
@@ -1394,12 +1379,6 @@ bool mg_small(const MgHier& h)
 void launch_olf_mgcg_small(hipStream_t s, const OlfMgArgs& a)
 {
     hipLaunchKernelGGL(k_olf_mgcg_small, dim3(1), dim3(kMgThreads), 0, s, a);
-}
-
-void launch_batched_olf_mgcg_small(hipStream_t s, const OlfMgArgs* args, int nmodels, const int* active)
-{
-    if (nmodels > 0)
-        hipLaunchKernelGGL(kb_olf_mgcg_small, dim3(nmodels), dim3(kMgThreads), 0, s, args, active);
 }
 
 void launch_olf_mgcg_block(hipStream_t s, const OlfMgArgs& a)

@@ -12,7 +12,7 @@ TOL = 1e-8   # m: ponding and heads of every coupled parity case
 
 
 @pytest.mark.parametrize("nx,ny", [(8, 8), (9, 8), (16, 17), (33, 31), (47, 86), (64, 64), (65, 64), (3, 200)])
-@pytest.mark.parametrize("form", [_abi.OLF_PRECOND_MG, _abi.OLF_PRECOND_MG_BLOCK])
+@pytest.mark.parametrize("form", [_abi.OLF_PRECOND_MG])
 def test_small_surfaces_match_oracle(hip, orc, nx, ny, form):
     w = inputs.c2_coupled(nx=nx, ny=ny, nz=3, rain_mm_h=150.0)
     p = _abi.Params.from_buffer_copy(w.params)
