@@ -842,7 +842,7 @@ int colstore(dhara_ctx* c, const double* wt, double ww, double* W, double* rw, d
 {
     dh::launch_adj_colstore(c->s, c->g, c->theta_n, wt, ww, W, rw, c->part[0]);
     LAUNCHCHK(c);
-    return host_reduce(c, dh::grid_for(c->S), 1, false, sum);
+    return host_reduce(c, dh::grid_for(c->S), 1, sum);
 }
 
 dh::LinArgs lin_args(dhara_ctx* c, const double* psi1, const double* psin)
@@ -890,7 +890,7 @@ int solve_jt(dhara_ctx* c, const double* psi1, const double* b, double* x, doubl
     dh::launch_bi_init(c->s, n, b, a.br, a.brh, a.bp, a.bv, x, c->part[0]);
     LAUNCHCHK(c);
     double bb;
-    int rc = host_reduce(c, np, 1, false, &bb);
+    int rc = host_reduce(c, np, 1, &bb);
     if (rc) return rc;
     *conv = true;
     if (bb == 0.0) return DHARA_OK;
@@ -906,13 +906,13 @@ int solve_jt(dhara_ctx* c, const double* psi1, const double* b, double* x, doubl
         dh::launch_adj_jac(c->s, c->g, true, psi1, a.K1, a.dK1, a.Ld, a.by, a.bv, a.brh, c->part[0]);
         LAUNCHCHK(c);
         double d2[2];
-        if ((rc = host_reduce(c, np, 2, false, d2))) return rc;
+        if ((rc = host_reduce(c, np, 2, d2))) return rc;
         alpha = rho / d2[0];
         if (!std::isfinite(alpha)) break;
         dh::launch_bi_s(c->s, n, a.br, a.bv, a.Jd, alpha, a.bs, a.bz, c->part[0]);
         LAUNCHCHK(c);
         double ss;
-        if ((rc = host_reduce(c, np, 1, false, &ss))) return rc;
+        if ((rc = host_reduce(c, np, 1, &ss))) return rc;
         ++it;
         if (std::sqrt(ss) <= tol * bn) {
             dh::launch_bi_x(c->s, n, x, a.by, a.bz, a.bs, a.bt, a.brh, alpha, 0.0, a.br, c->part[0]);
@@ -922,11 +922,11 @@ int solve_jt(dhara_ctx* c, const double* psi1, const double* b, double* x, doubl
         }
         dh::launch_adj_jac(c->s, c->g, true, psi1, a.K1, a.dK1, a.Ld, a.bz, a.bt, a.bs, c->part[0]);
         LAUNCHCHK(c);
-        if ((rc = host_reduce(c, np, 2, false, d2))) return rc;
+        if ((rc = host_reduce(c, np, 2, d2))) return rc;
         omega = d2[1] > 0.0 ? d2[0] / d2[1] : 0.0;
         dh::launch_bi_x(c->s, n, x, a.by, a.bz, a.bs, a.bt, a.brh, alpha, omega, a.br, c->part[0]);
         LAUNCHCHK(c);
-        if ((rc = host_reduce(c, np, 2, false, d2))) return rc;
+        if ((rc = host_reduce(c, np, 2, d2))) return rc;
         rho1 = d2[0];
         if (std::sqrt(d2[1]) <= tol * bn) { *conv = true; break; }
         if (omega == 0.0) break;

@@ -2,11 +2,11 @@
 //
 // One context = one HIP stream + every device buffer of one model.  The time loop of the
 // reference (src/device.cu:374-475 -> src/subsurface.cu:686-847 -> src/overland.cu:387-419)
-// is driven from here; all arithmetic runs in kernels.hip.  The host synchronises once per
-// Krylov batch, once per Picard iteration and once at the end of a step (the reference
-// synchronised on every dot product, Picard max and mass-balance reduction).  Reductions the
-// host consumes (Picard increment, mass balance, discharge) are summed on the host from the
-// per-block partials in block order.
+// is driven from here; all arithmetic runs in kernels.hip.  The host waits once per Krylov batch
+// -- the Picard pass is queued behind it -- and once at the end of a step (the reference
+// synchronised on every dot product, Picard max and mass-balance reduction).  What the host
+// reads (solver state, Picard increment, mass balance, discharge) the last kernel of a queue
+// leaves in pinned memory (HostReport).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -151,19 +151,18 @@ dh::AaArgs aa_args(dhara_ctx* c)
 
 // The Picard pass after a linear solve: theta, K, C of x with the increment (k_vg_picard), or on
 // the Anderson path with a rule on psi the increment alone, then the Anderson update or, after
-// the last pass, theta, K, C of x; the increment's maxima go to c->dred.  With gate, every kernel
-// that depends on the solve runs only once the device's outer test has passed (queued behind a
-// mixed solve).
-void queue_picard_pass(dhara_ctx* c, const dh::PcgState* gate)
+// the last pass, theta, K, C of x; the increment's maxima and the solver state go to c->rep.  With a
+// gate the pass is queued behind the solve's launches and runs only if the solve ended as it says.
+void queue_picard_pass(dhara_ctx* c, dh::GateKind kind)
 {
     const bool aa = c->p.picard_accel > 0;
     const bool inc_only = aa && c->p.picard_rule != DHARA_PICARD_REL_THETA;
     const dh::VgArgs va = vg_args(c, c->x, c->theta_new);
+    const dh::Gate gate{c->st_sub, kind};
     if (inc_only) dh::launch_picard_inc(c->s, va, gate);
-    else if (gate) dh::launch_vg_picard_gated(c->s, va, gate);
-    else dh::launch_vg_picard(c->s, va);
+    else dh::launch_vg_picard(c->s, va, gate);
     if (!aa) {
-        dh::launch_max_rows2(c->s, c->part[0], dh::grid_for(c->N), c->dred);
+        dh::launch_picard_report(c->s, c->part[0], dh::grid_for(c->N), gate, c->rep);
         return;
     }
     const dh::LaunchEv ev{c->prof ? c->aa_ev[0] : nullptr, c->prof ? c->aa_ev[1] : nullptr};
@@ -174,8 +173,8 @@ void queue_picard_pass(dhara_ctx* c, const dh::PcgState* gate)
     na.nparts = dh::grid_for(c->N);
     na.fin = inc_only ? 1 : 0;
     na.tol = c->p.picard_tol;
-    na.red = c->dred;
-    na.st = gate;
+    na.gate = gate;
+    na.rep = c->rep;
     dh::launch_picard_next(c->s, na, c->p.picard_accel, &ev);
 }
 
@@ -223,29 +222,31 @@ dh::Soil soil_of(const dhara_ctx* c)
     return s;
 }
 
-// Sum (or max) the first nv partial rows of the last host-reduced kernel, in block order.
-int host_reduce(dhara_ctx* c, int nparts, int nv, bool take_max, double* out)
+int sync_stream(dhara_ctx* c)
 {
-    const size_t span = (size_t)(nv - 1) * dh::kMaxBlocks + nparts;
-    HIPCHK(c, hipMemcpyAsync(c->h_part, c->part[0], span * sizeof(double), hipMemcpyDeviceToHost, c->s));
     HIPCHK(c, hipStreamSynchronize(c->s));
-    for (int v = 0; v < nv; ++v) {
-        double acc = take_max ? -INFINITY : 0.0;
-        const double* row = c->h_part + (size_t)v * dh::kMaxBlocks;
-        for (int b = 0; b < nparts; ++b) acc = take_max ? std::max(acc, row[b]) : acc + row[b];
-        out[v] = acc;
-    }
     return DHARA_OK;
 }
 
-// Sum of n per-block partials at dev (a row of a partial buffer), in block order.
+// Sums of the first nv partial rows of part[0] (nparts partials each).
+int host_reduce(dhara_ctx* c, int nparts, int nv, double* out)
+{
+    dh::launch_report_sums(c->s, c->part[0], nparts, nv, c->rep);
+    LAUNCHCHK(c);
+    int rc = sync_stream(c);
+    if (rc) return rc;
+    std::copy(c->rep->sums, c->rep->sums + nv, out);
+    return DHARA_OK;
+}
+
+// Sum of n per-block partials at dev (a row of a partial buffer).
 int host_sum(dhara_ctx* c, const double* dev, int n, double* out)
 {
-    HIPCHK(c, hipMemcpyAsync(c->h_part, dev, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->s));
-    HIPCHK(c, hipStreamSynchronize(c->s));
-    double acc = 0.0;
-    for (int b = 0; b < n; ++b) acc += c->h_part[b];
-    *out = acc;
+    dh::launch_report_sums(c->s, dev, n, 1, c->rep);
+    LAUNCHCHK(c);
+    int rc = sync_stream(c);
+    if (rc) return rc;
+    *out = c->rep->sums[0];
     return DHARA_OK;
 }
 
@@ -260,9 +261,9 @@ bool has_dirichlet(const dhara_ctx* c)
 
 int read_state(dhara_ctx* c, dh::PcgState* dev)
 {
-    HIPCHK(c, hipMemcpyAsync(c->h_st, dev, sizeof(dh::PcgState), hipMemcpyDeviceToHost, c->s));
-    HIPCHK(c, hipStreamSynchronize(c->s));
-    return DHARA_OK;
+    dh::launch_report(c->s, dev, c->rep);
+    LAUNCHCHK(c);
+    return sync_stream(c);
 }
 
 dh::VgArgs vg_args(dhara_ctx* c, const double* psi, double* theta)
@@ -380,6 +381,25 @@ dh::SolveCtl solve_ctl(dhara_ctx* c, dh::PcgState* st, int maxit, int nparts, bo
     return sc;
 }
 
+// The Picard pass behind a batch of an FP64 solve, which runs if the batch ended the solve: the host
+// then waits once per Picard iteration instead of twice (the batch is sized from the solve of the
+// same Picard iteration one step before).
+bool queue_after_solve(dhara_ctx* c)
+{
+    queue_picard_pass(c, dh::GATE_SOLVED);
+    return true;
+}
+
+// The end of an FP64 solve whose batches queued the Picard pass.
+int end_solve(dhara_ctx* c, dhara_step_stats* st)
+{
+    st->lin_iters += c->h_st->iter;
+    st->lin_converged &= c->h_st->conv;
+    if (c->h_st->nan) st->nan_seen = 1;
+    c->vg_ready = !c->h_st->nan;
+    return DHARA_OK;
+}
+
 int solve_fp64(dhara_ctx* c, dhara_step_stats* st)
 {
     const bool dir = has_dirichlet(c);
@@ -390,8 +410,8 @@ int solve_fp64(dhara_ctx* c, dhara_step_stats* st)
     dh::SolveCtl sc = solve_ctl(c, c->st_sub, c->p.lin_maxiter, dh::grid_for(c->N), false, true);
     const dh::TileCfg tc = c->tile[0];
     const int spmv_parts = tc.tx ? dh::tile_blocks(c->g, tc) : dh::grid_for(c->N);
-    int rc = run_krylov(
-        c, c->st_sub, c->p.lin_maxiter, c->pcg_hint, c->prof, 8.0,
+    int rc = run_krylov_then(
+        c, c->st_sub, c->p.lin_maxiter, c->pcg_hint(), c->prof, 8.0,
         [&](int it, const dh::LaunchEv& ev) {
             dh::SolveCtl k = sc;
             k.it = it;
@@ -405,12 +425,10 @@ int solve_fp64(dhara_ctx* c, dhara_step_stats* st)
             k.nparts = spmv_parts;
             k.part_out = c->part[0];
             dh::launch_pcg_update_f64(c->s, c->N, c->x, c->r, c->D, pp[(it + 1) & 1], c->q, k, ev);
-        });
+        },
+        [&] { return queue_after_solve(c); }, 0, 0);
     if (rc) return rc;
-    st->lin_iters += c->h_st->iter;
-    st->lin_converged &= c->h_st->conv;
-    if (c->h_st->nan) st->nan_seen = 1;
-    return DHARA_OK;
+    return end_solve(c, st);
 }
 
 // Mixed precision: FP32 Jacobi-PCG with FP64 reliable updates.  The FP64 assembly gives
@@ -447,7 +465,7 @@ int solve_mixed(dhara_ctx* c, dhara_step_stats* st)
     bool outer_conv = false;
     for (;;) {
         int rc = run_krylov(
-            c, c->st_sub, maxit, c->pcg_hint, c->prof, 4.0,
+            c, c->st_sub, maxit, updates ? c->seg_hint : c->pcg_hint(), c->prof, 4.0,
             [&](int k_it, const dh::LaunchEv& ev) {
                 dh::SolveCtl k = sc;
                 k.it = k_it;
@@ -516,7 +534,7 @@ int solve_fp64_cg1(dhara_ctx* c, dhara_step_stats* st)
         dh::launch_cg1_init_f64(c->s, c->g, c->tile[0], c->K, c->D, rb[0], pb[1], k);
     }
     const int init_parts = dh::cg1_init_blocks(c->g, c->tile[0]);
-    int rc = run_krylov1(c, c->st_sub, c->p.lin_maxiter, c->pcg_hint, c->prof, 8.0,
+    int rc = run_krylov1(c, c->st_sub, c->p.lin_maxiter, c->pcg_hint(), c->prof, 8.0,
                          [&](int it, const dh::LaunchEv& ev) {
                              dh::SolveCtl k = sc;
                              k.it = it;
@@ -526,12 +544,10 @@ int solve_fp64_cg1(dhara_ctx* c, dhara_step_stats* st)
                              k.part_out = c->part[it & 1];
                              dh::launch_cg1_f64(c->s, c->g, tc, c->K, c->D, rb[it & 1], rb[(it + 1) & 1],
                                                 pb[(it + 1) & 1], pb[it & 1], c->x, k, ev);
-                         });
+                         },
+                         [&] { return queue_after_solve(c); });
     if (rc) return rc;
-    st->lin_iters += c->h_st->iter;
-    st->lin_converged &= c->h_st->conv;
-    if (c->h_st->nan) st->nan_seen = 1;
-    return DHARA_OK;
+    return end_solve(c, st);
 }
 
 // Column-preconditioned PCG (no Dirichlet rows): the Hestenes-Stiefel iteration of solve_fp64
@@ -555,8 +571,8 @@ int solve_fp64_line(dhara_ctx* c, dhara_step_stats* st)
         k.part_out = c->part_line;
         dh::launch_line_init_f64(c->s, c->g, c->K, c->D, c->r, c->zl, k);
     }
-    rc = run_krylov(
-        c, c->st_sub, c->p.lin_maxiter, c->pcg_hint, c->prof, 8.0,
+    rc = run_krylov_then(
+        c, c->st_sub, c->p.lin_maxiter, c->pcg_hint(), c->prof, 8.0,
         [&](int it, const dh::LaunchEv& ev) {
             dh::SolveCtl k = sc;
             k.it = it;
@@ -571,13 +587,11 @@ int solve_fp64_line(dhara_ctx* c, dhara_step_stats* st)
             k.nparts = spmv_parts;
             k.part_out = c->part[0];
             dh::launch_line_update_f64(c->s, c->g, c->K, c->D, c->x, c->r, pp[(it + 1) & 1], c->q, c->zl, k, ev);
-        });
+        },
+        [&] { return queue_after_solve(c); }, 0, 0);
     if (rc) return rc;
     c->prof_acc.update_bytes = 9.0 * 8.0 * c->N;   // x, p, q, r, K, D read; x, r, z written
-    st->lin_iters += c->h_st->iter;
-    st->lin_converged &= c->h_st->conv;
-    if (c->h_st->nan) st->nan_seen = 1;
-    return DHARA_OK;
+    return end_solve(c, st);
 }
 
 // Mixed precision with the column preconditioner: the reliable-update scheme of solve_mixed,
@@ -609,7 +623,6 @@ int next_segment_batch(const dhara_ctx* c, int n)
 int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
 {
     int rc;
-    c->vg_ready = false;
     if ((rc = alloc_line(c, true))) return rc;
     const int aparts = dh::launch_assemble_tiled(c->s, asm_args(c, false), true, c->tile[0]);
     LAUNCHCHK(c);
@@ -649,7 +662,6 @@ int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
     const double target = c->p.lin_tol * c->p.lin_tol;   // outer target of ||r||^2 / ||b||^2
     bool spec = false, line_update = true;   // line_update: k_refine_line fits the surface
     int spec_parts = 0;
-    hipError_t spec_err = hipSuccess;
     auto expect_floor = [&](double rr0) {   // the next segment's stopping test is its floor
         return line_update && c->p.inner_tol * c->p.inner_tol * rr0 <= 0.5 * 0.25 * target * c->h_st->bb;
     };
@@ -660,15 +672,13 @@ int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
         const int n = dh::launch_refine_line(c->s, ra, c->zl32, dh::kRefineCheck);
         if (!n) return 0;
         dh::launch_refine_conv(c->s, c->part_line, n, c->p.lin_tol, c->st_sub);
-        queue_picard_pass(c, c->st_sub);
-        if (spec_err == hipSuccess)
-            spec_err = hipMemcpyAsync(c->h_red, c->dred, 2 * sizeof(double), hipMemcpyDeviceToHost, c->s);
+        queue_picard_pass(c, dh::GATE_UPDATE);
         return n;
     };
     for (;;) {
         const int seg = it;
         rc = run_krylov_then(
-            c, c->st_sub, maxit, c->pcg_hint, c->prof, 4.0,
+            c, c->st_sub, maxit, c->pcg_hint(), c->prof, 4.0,
             [&](int j, const dh::LaunchEv& ev) {
                 dh::SolveCtl k = sc;
                 k.it = j;
@@ -687,11 +697,11 @@ int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
                                            c->zl32, k, ev);
             },
             [&] {
-                if (spec) spec_parts = queue_update();
+                spec_parts = spec ? queue_update() : 0;
+                return spec_parts != 0;   // the Picard pass left the state in the report
             },
             it, first_batch);
         if (rc) return rc;
-        if (spec_err != hipSuccess) return set_err(c, DHARA_E_DEVICE, hipGetErrorString(spec_err));
         c->prof_acc.update_bytes = 9.0 * 4.0 * c->N;
         if (c->h_st->nan) { st->nan_seen = 1; break; }
         if (c->h_st->outer_conv) { outer_conv = true; break; }   // d == 0 here
@@ -726,8 +736,7 @@ int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
             // unconverged), with one synchronisation for the update, its test and the Picard pass
             if (queue_update()) {
                 LAUNCHCHK(c);
-                if ((rc = read_state(c, c->st_sub))) return rc;
-                if (spec_err != hipSuccess) return set_err(c, DHARA_E_DEVICE, hipGetErrorString(spec_err));
+                if ((rc = sync_stream(c))) return rc;
                 if (c->h_st->gate == 2) {
                     outer_conv = true;
                     c->vg_ready = true;
@@ -824,6 +833,7 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
     int it = 0, updates = 0, refine_parts = aparts;
     bool outer_conv = false;
     for (;;) {
+        int one_launch = 1;
         {
             dh::SolveCtl k = sc;   // fresh residual partials in part[0]
             k.it = it;
@@ -833,7 +843,10 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
             dh::launch_cg1_init_f32(c->s, c->g, c->tile[1], c->K32, c->D32, rb[it & 1], pb[(it + 1) & 1], k);
         }
         const int seg = it;
-        int rc = run_krylov1(c, c->st_sub, maxit, c->pcg_hint, c->prof, 4.0,
+        // after as many updates as the last solve took, this segment's start-up is likely to pass the
+        // outer test: the Picard pass then goes behind its batches
+        const bool last = updates > 0 && updates >= c->upd_hint;
+        int rc = run_krylov1(c, c->st_sub, maxit, last ? one_launch : updates ? c->seg_hint : c->pcg_hint(), c->prof, 4.0,
                              [&](int j, const dh::LaunchEv& ev) {
                                  dh::SolveCtl k = sc;
                                  k.it = j;
@@ -844,10 +857,18 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
                                  dh::launch_cg1_f32(c->s, c->g, tc, c->K32, c->D32, rb[j & 1], rb[(j + 1) & 1],
                                                     pb[(j + 1) & 1], pb[j & 1], c->d32, k, ev);
                              },
+                             [&] {
+                                 if (last) queue_picard_pass(c, dh::GATE_OUTER);
+                                 return last;
+                             },
                              it);
         if (rc) return rc;
         if (c->h_st->nan) { st->nan_seen = 1; break; }
-        if (c->h_st->outer_conv) { outer_conv = true; break; }   // d == 0 here
+        if (c->h_st->outer_conv) {   // d == 0 here
+            outer_conv = true;
+            c->vg_ready = last;
+            break;
+        }
         const int it_end = c->h_st->iter;
         ra.r32 = rb[it_end & 1];
         refine_parts = dh::launch_refine_tiled(c->s, ra, c->tile[0]);
@@ -872,6 +893,7 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
         it = it_end;
         sc.first_sweep = 0;
     }
+    c->upd_hint = updates;
     st->lin_iters += c->h_st->iter;
     st->refine_sweeps += updates;
     st->lin_converged &= outer_conv ? 1 : 0;
@@ -916,24 +938,21 @@ int do_subsurface_step(dhara_ctx* c, dhara_step_stats* st)
         const bool line = c->p.precond == DHARA_PRECOND_COLUMN && !dir && dh::line_supported(c->g);
         // the Anderson pass queued with this iteration's Picard pass updates unless it is the last
         c->aa_active = aa && niter + 1 < c->p.picard_maxiter;
+        c->picard_it = niter;
+        c->vg_ready = false;
         int rc = line ? (mixed ? solve_mixed_line(c, st) : solve_fp64_line(c, st))
                       : mixed ? (one ? solve_mixed_cg1(c, st) : solve_mixed(c, st))
                               : (one ? solve_fp64_cg1(c, st) : solve_fp64(c, st));
         if (rc) return rc;
         if (st->nan_seen) { c->theta_m_current = false; break; }
-        // Picard increment and NaN flag: maxima over the blocks, taken on the device (by the
-        // solve itself when it queued the Picard pass behind its last batch)
-        double pic[2];
-        if (c->vg_ready) {
-            c->vg_ready = false;
-        } else {
-            queue_picard_pass(c, nullptr);
+        // Picard increment and NaN flag: maxima over the blocks, taken on the device (in a pass that
+        // the solve itself queued behind its last batch, or queued here)
+        if (!c->vg_ready) {
+            queue_picard_pass(c, dh::GATE_OPEN);
             LAUNCHCHK(c);
-            HIPCHK(c, hipMemcpyAsync(c->h_red, c->dred, 2 * sizeof(double), hipMemcpyDeviceToHost, c->s));
-            HIPCHK(c, hipStreamSynchronize(c->s));
+            if ((rc = sync_stream(c))) return rc;
         }
-        pic[0] = c->h_red[0];
-        pic[1] = c->h_red[1];
+        const double pic[2] = {c->rep->red[0], c->rep->red[1]};
         ++niter;
         delta = pic[0];
         if (pic[1] > 0.0) { st->nan_seen = 1; c->theta_m_current = false; break; }
@@ -988,7 +1007,7 @@ int do_subsurface_step(dhara_ctx* c, dhara_step_stats* st)
     dh::launch_end_step(c->s, ea);
     LAUNCHCHK(c);
     double sums[9];
-    int rce = host_reduce(c, dh::grid_for(c->N), 9, false, sums);
+    int rce = host_reduce(c, dh::grid_for(c->N), 9, sums);
     if (rce) return rce;
     // theta carry consumed theta_m; the last vG result (theta_new) is theta(psi^n)
     c->theta_m_current = false;
@@ -1108,7 +1127,8 @@ int do_overland_step(dhara_ctx* c, dhara_step_stats* st)
                                        const dh::MgCg1 v{k, c->H, c->p2[0], c->z2, c->w2, sb[it & 1], sb[(it + 1) & 1],
                                                          rb[it & 1], rb[(it + 1) & 1]};
                                        dh::launch_mg_vcycle_cg1(c->s, c->mg, c->st_olf, c->part[0], v);
-                                   })
+                                   },
+                                   [] { return false; })
                      : run_krylov(
             c, c->st_olf, c->p.olf_maxiter, c->olf_hint, false, 8.0,
             [&](int it, const dh::LaunchEv& ev) {
@@ -1138,7 +1158,7 @@ int do_overland_step(dhara_ctx* c, dhara_step_stats* st)
     dh::launch_olf_post(c->s, a);
     LAUNCHCHK(c);
     double q[2];
-    if ((rc = host_reduce(c, dh::grid_for(c->S), 2, false, q))) return rc;
+    if ((rc = host_reduce(c, dh::grid_for(c->S), 2, q))) return rc;
     st->outlet_discharge = q[0];
     st->ring_outflow = q[1];
     return st->nan_seen ? set_err(c, DHARA_E_NUMERIC, "NaN/Inf in the overland state") : DHARA_OK;
@@ -1296,7 +1316,7 @@ int dhara_create(const dhara_grid* grid, const dhara_params* params, dhara_ctx**
     if (grid->nroot_groups > dh::kMaxSums * dh::kMaxBlocks) { dhara_destroy(c); return DHARA_E_ARG; }
     if ((rc = dalloc(c, &c->procmap, S)) || (rc = dalloc(c, &c->root, (size_t)grid->nroot_groups * grid->nz)) ||
         (rc = dalloc(c, &c->flags, N)) || (rc = dalloc(c, &c->part[0], (size_t)dh::kMaxSums * dh::kMaxBlocks)) ||
-        (rc = dalloc(c, &c->part[1], (size_t)dh::kMaxSums * dh::kMaxBlocks)) || (rc = dalloc(c, &c->dred, 16)) ||
+        (rc = dalloc(c, &c->part[1], (size_t)dh::kMaxSums * dh::kMaxBlocks)) ||
         (rc = dalloc(c, &c->st_sub, 1)) || (rc = dalloc(c, &c->st_olf, 1))) {
         dhara_destroy(c);
         return rc;
@@ -1308,12 +1328,12 @@ int dhara_create(const dhara_grid* grid, const dhara_params* params, dhara_ctx**
             return DHARA_E_DEVICE;
         }
     }
-    if (hipHostMalloc((void**)&c->h_st, sizeof(dh::PcgState)) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_red, 16 * sizeof(double)) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_part, (size_t)dh::kMaxSums * dh::kMaxBlocks * sizeof(double)) != hipSuccess) {
+    if (hipHostMalloc((void**)&c->rep, sizeof(dh::HostReport)) != hipSuccess) {
         dhara_destroy(c);
         return DHARA_E_ALLOC;
     }
+    std::memset((void*)c->rep, 0, sizeof(dh::HostReport));
+    c->h_st = &c->rep->st;
     if (c->p.precision == DHARA_MIXED && (rc = alloc_mixed(c))) { dhara_destroy(c); return rc; }
     if (hipStreamSynchronize(c->s) != hipSuccess) { dhara_destroy(c); return DHARA_E_DEVICE; }
     *out = c;
@@ -1329,9 +1349,7 @@ int dhara_destroy(dhara_ctx* c)
     for (hipEvent_t e : c->aa_ev)
         if (e) (void)hipEventDestroy(e);
     for (void* v : c->allocs) (void)hipFree(v);
-    if (c->h_st) (void)hipHostFree(c->h_st);
-    if (c->h_part) (void)hipHostFree(c->h_part);
-    if (c->h_red) (void)hipHostFree(c->h_red);
+    if (c->rep) (void)hipHostFree(c->rep);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
     return DHARA_OK;

@@ -56,10 +56,7 @@ struct dhara_ctx {
     double* zl = nullptr;
     float* zl32 = nullptr;
     double* part_line = nullptr;
-    double* dred = nullptr;   // a few device-reduced values for the host (launch_max_rows2)
-    double* h_red = nullptr;  // pinned: the Picard increment and NaN flag of a k_vg_picard queued
-                              // by the linear solve (vg_ready)
-    bool vg_ready = false;    // the solve ended with k_vg_picard already run, h_red its maxima
+    bool vg_ready = false;    // the solve ended with the Picard pass already run (its maxima in rep)
     // Anderson-accelerated Picard update (picard_accel > 0; allocated on first use): the ring of f
     // and y of the last picard_accel + 1 passes, pass p of a step in slot p mod (picard_accel + 1);
     // aa_count: passes of this step that have run.
@@ -70,15 +67,23 @@ struct dhara_ctx {
     hipEvent_t aa_ev[2] = {nullptr, nullptr};   // kernel timestamps of the last queued pass (profiling)
     dh::PcgState* st_sub = nullptr;
     dh::PcgState* st_olf = nullptr;
-    // pinned host mirrors
+    // pinned host memory that kernels write (HostReport), and the state in it
+    dh::HostReport* rep = nullptr;
     dh::PcgState* h_st = nullptr;
-    double* h_part = nullptr;
 
     bool face_dirichlet[6] = {false, false, false, false, false, false};
     bool has_alpha = false, has_n = false, has_transp = false;
     bool initialized = false;
     bool theta_m_current = true;
-    int pcg_hint = 8, olf_hint = 8;
+    // iterations of the last solve of each kind: of the subsurface solves one per Picard iteration of
+    // a step (a step's solves get shorter as it converges, and the next step's follow them), in
+    // mixed precision for the solve's first segment and, seg_hint, the segments after it
+    static constexpr int kHints = 16;
+    int pcg_hints[kHints], seg_hint = 8, olf_hint = 8, adj_hint = 8;
+    int upd_hint = 1;         // reliable updates of the last mixed solve
+    int picard_it = 0;        // Picard iteration of the step being solved
+    dhara_ctx() { std::fill(pcg_hints, pcg_hints + kHints, 8); }
+    int& pcg_hint() { return pcg_hints[std::min(picard_it, kHints - 1)]; }
     std::vector<void*> allocs;
     // SpMV tile shapes: [0] FP64 solves, [1] FP32 inner solves (tx = 0: untiled kernel)
     dh::TileCfg tile[2] = {{32, 8, 0}, {32, 8, 0}};
@@ -127,8 +132,9 @@ int dalloc(dhara_ctx* c, T** ptr, size_t count)
     return DHARA_OK;
 }
 
-int host_reduce(dhara_ctx* c, int nparts, int nv, bool take_max, double* out);
+int host_reduce(dhara_ctx* c, int nparts, int nv, double* out);   // sums of the first nv rows of part[0]
 int read_state(dhara_ctx* c, dh::PcgState* dev);
+int sync_stream(dhara_ctx* c);
 bool has_dirichlet(const dhara_ctx* c);
 dh::Soil soil_of(const dhara_ctx* c);
 dh::VgArgs vg_args(dhara_ctx* c, const double* psi, double* theta);
@@ -141,7 +147,7 @@ int alloc_line(dhara_ctx* c, bool mixed);
 // Anderson pass after the current solve
 int alloc_aa(dhara_ctx* c);
 dh::AaArgs aa_args(dhara_ctx* c);
-void queue_picard_pass(dhara_ctx* c, const dh::PcgState* gate);
+void queue_picard_pass(dhara_ctx* c, dh::GateKind gate);
 dh::SolveCtl solve_ctl(dhara_ctx* c, dh::PcgState* st, int maxit, int nparts, bool mixed_inner,
                        bool first_sweep);
 int do_subsurface_step(dhara_ctx* c, dhara_step_stats* st);
@@ -157,7 +163,8 @@ int noalloc_setup(dhara_ctx* c);
 // kernel of iteration `it` reads partials A and writes B, the update kernel reads B and
 // writes A.  With profiling on, events bracket each SpMV and update launch of the batch and
 // only the launches that did work (the first ones of the batch) are accumulated.
-// after() queues further work behind every batch, before the state is read back.
+// after() queues further work behind every batch; it returns true if that work leaves the state in
+// the host's report, so that a synchronisation is enough to read it.
 template <class SpmvFn, class UpdFn, class AfterFn>
 int run_krylov_then(dhara_ctx* c, dh::PcgState* st, int maxit, int& hint, bool prof, double elem,
                     SpmvFn spmv, UpdFn upd, AfterFn after, int it_start, int first_batch)
@@ -179,9 +186,9 @@ int run_krylov_then(dhara_ctx* c, dh::PcgState* st, int maxit, int& hint, bool p
             spmv(it, e_spmv);
             upd(it, e_upd);
         }
-        after();
+        const bool reported = after();
         LAUNCHCHK(c);
-        int rc = read_state(c, st);
+        int rc = reported ? sync_stream(c) : read_state(c, st);
         if (rc) return rc;
         const int done_iters = c->h_st->done ? c->h_st->iter : it;
         if (prof) {
@@ -211,14 +218,14 @@ template <class SpmvFn, class UpdFn>
 int run_krylov(dhara_ctx* c, dh::PcgState* st, int maxit, int& hint, bool prof, double elem,
                SpmvFn spmv, UpdFn upd, int it_start = 0, int first_batch = 0)
 {
-    return run_krylov_then(c, st, maxit, hint, prof, elem, spmv, upd, [] {}, it_start, first_batch);
+    return run_krylov_then(c, st, maxit, hint, prof, elem, spmv, upd, [] { return false; }, it_start, first_batch);
 }
 
 // One launch per iteration (one-kernel PCG): the same batching as run_krylov; iteration `it`
 // of the batch is queued by kern(it, events).  Profiling counts every launch that did work
 // as an "spmv" launch of 8 algorithmic arrays.
-template <class KernFn>
-int run_krylov1(dhara_ctx* c, dh::PcgState* st, int maxit, int& hint, bool prof, double elem, KernFn kern,
+template <class KernFn, class AfterFn>
+int run_krylov1(dhara_ctx* c, dh::PcgState* st, int maxit, int& hint, bool prof, double elem, KernFn kern, AfterFn after,
                 int it_start = 0)
 {
     int it = it_start;
@@ -230,8 +237,9 @@ int run_krylov1(dhara_ctx* c, dh::PcgState* st, int maxit, int& hint, bool prof,
             if (prof) e = dh::LaunchEv{c->ev[2 * b], c->ev[2 * b + 1]};
             kern(it, e);
         }
+        const bool reported = after();
         LAUNCHCHK(c);
-        int rc = read_state(c, st);
+        int rc = reported ? sync_stream(c) : read_state(c, st);
         if (rc) return rc;
         const int done_iters = c->h_st->done ? c->h_st->iter : it;
         if (prof) {

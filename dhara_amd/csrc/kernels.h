@@ -119,10 +119,37 @@ struct AaArgs {
     int active;              // the pass may update (not the one at the iteration limit)
 };
 
+// Whether work queued behind a solve's launches, before the host has seen how the solve ended, may run.
+enum GateKind {
+    GATE_OPEN,       // the host has decided
+    GATE_UPDATE,     // gate == 2: the reliable update's outer test has passed (k_refine_conv)
+    GATE_SOLVED,     // the solve ended, converged or at its limit, without NaN
+    GATE_OUTER,      // mixed precision: the solve ended with its FP64 residual passing the outer test
+};
+struct Gate {
+    const PcgState* st;
+    int kind;
+    __device__ __forceinline__ bool open() const
+    {
+        if (kind == GATE_OPEN) return true;
+        if (kind == GATE_UPDATE) return st->gate == 2;
+        return st->done && !st->nan && (kind == GATE_SOLVED || st->outer_conv);
+    }
+};
+
+// What the last kernel of a queue leaves for the host, in pinned host memory (read after a stream
+// synchronisation): the solver state and, if the Picard pass ran, its [increment, NaN flag].  Written
+// by the kernel itself, which a copy queued behind it would make the host wait a launch longer for.
+struct HostReport {
+    PcgState st;
+    double red[2];
+    double sums[kMaxSums];   // launch_report_sums
+};
+
 // What follows a Picard increment (k_picard_next): the maxima of the increment's block partials
-// [increment, NaN flag] to red; then, unless a NaN was seen, the Anderson update when the increment
-// is not below tol (and aa.active), else theta, K, C of the converged x (fin set).  With st the
-// pass was queued behind a solve: nothing runs unless st->gate == 2.
+// [increment, NaN flag]; then, unless a NaN was seen, the Anderson update when the increment is
+// not below tol (and aa.active), else theta, K, C of the converged x (fin set).  The state and the
+// maxima go to rep.
 struct NextArgs {
     AaArgs aa;
     VgArgs vg;
@@ -130,8 +157,8 @@ struct NextArgs {
     int nparts;
     int fin;
     double tol;
-    double* red;
-    const PcgState* st;
+    Gate gate;
+    HostReport* rep;
 };
 
 struct AsmArgs {
@@ -260,19 +287,22 @@ struct LaunchEv {
 };
 
 void launch_vg(hipStream_t s, const VgArgs& a);                 // theta, K, C of psi
-void launch_vg_picard(hipStream_t s, const VgArgs& a);          // + increment + relax
-// out[0], out[1] = maxima of rows 0 and 1 of part (nparts partials each); one block
-void launch_max_rows2(hipStream_t s, const double* part, int nparts, double* out);
+void launch_vg_picard(hipStream_t s, const VgArgs& a, const Gate& gate);   // + increment + relax
+// the Picard pass's second kernel without the Anderson update: the maxima of rows 0 and 1 of part
+// and the state to rep
+void launch_picard_report(hipStream_t s, const double* part, int nparts, const Gate& gate, HostReport* rep);
+// the state alone; the sums of the first nv rows of part (nparts partials each)
+void launch_report(hipStream_t s, const PcgState* st, HostReport* rep);
+void launch_report_sums(hipStream_t s, const double* part, int nparts, int nv, HostReport* rep);
 // after a gated check-only update (launch_refine_line, kRefineCheck): the outer test on the
 // device (st->gate = 2 when the sum of part's slot-3 partials passes lin_tol^2 ||b||^2, the sum
-// in st->rr_update), and k_vg_picard run only in that case
+// in st->rr_update)
 void launch_refine_conv(hipStream_t s, const double* part, int nparts, double lin_tol, PcgState* st);
-void launch_vg_picard_gated(hipStream_t s, const VgArgs& a, const PcgState* st);
 // The Picard pass's second kernel with the Anderson update of depth `depth` (1..kAaMaxDepth)
 void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const LaunchEv* ev = nullptr);
 // Its first kernel for the rules on psi (ABS_PSI / REL_PSI): the increment of a.psi against a.psi_m
-// into a.part_out; with st it runs only when st->gate == 2 (queued behind a mixed solve)
-void launch_picard_inc(hipStream_t s, const VgArgs& a, const PcgState* st);
+// into a.part_out
+void launch_picard_inc(hipStream_t s, const VgArgs& a, const Gate& gate);
 void launch_vg_inverse(hipStream_t s, const Geo& g, const Soil& soil, const double* theta,
                        double* psi);
 void launch_row_flags(hipStream_t s, const Geo& g, const int* const bctype[6], uint8_t* flags);

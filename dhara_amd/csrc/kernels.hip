@@ -108,16 +108,9 @@ __device__ __forceinline__ void b_vg_picard(VgArgs a, Blk bk)
     block_partials<2, true>(mx, a.part_out, bk.id);
 }
 
-__global__ __launch_bounds__(kBlock) void k_vg_picard(VgArgs a)
+__global__ __launch_bounds__(kBlock) void k_vg_picard(VgArgs a, Gate gate)
 {
-    b_vg_picard(a, hw_blk());
-}
-
-// k_vg_picard queued before the host knows that the linear solve has converged: runs only when
-// the device-side outer test has passed (gate 2, k_refine_conv).
-__global__ __launch_bounds__(kBlock) void k_vg_picard_gated(VgArgs a, const PcgState* st)
-{
-    if (st->gate != 2) return;
+    if (!gate.open()) return;
     b_vg_picard(a, hw_blk());
 }
 
@@ -344,10 +337,52 @@ __device__ __forceinline__ void b_picard_inc(const double* __restrict__ x, const
 }
 
 __global__ __launch_bounds__(kBlock) void k_picard_inc(const double* x, const double* pm, int n, int rule,
-                                                         double* part_out, const PcgState* st)
+                                                         double* part_out, Gate gate)
 {
-    if (st && st->gate != 2) return;
+    if (!gate.open()) return;
     b_picard_inc(x, pm, n, rule, part_out, hw_blk());
+}
+
+// The solver state to the host's report, by the first threads of a block (one word each).
+__device__ __forceinline__ void report_state(const PcgState* st, HostReport* rep)
+{
+    constexpr int NW = sizeof(PcgState) / sizeof(int);
+    static_assert(NW <= kWave && sizeof(PcgState) % sizeof(int) == 0, "one word per lane of a wave");
+    if (threadIdx.x < NW) reinterpret_cast<int*>(&rep->st)[threadIdx.x] = reinterpret_cast<const int*>(st)[threadIdx.x];
+}
+
+__global__ void k_report(const PcgState* st, HostReport* rep) { report_state(st, rep); }
+
+// One wave per row.
+__global__ __launch_bounds__(1024) void k_report_sums(const double* __restrict__ part, int nparts, int nv,
+                                                      HostReport* rep)
+{
+    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    if (w >= nv) return;
+    double v = 0.0;
+    for (int b = lane; b < nparts; b += kWave) v += part[w * kMaxBlocks + b];
+    v = wave_sum(v);
+    if (lane == 0) rep->sums[w] = v;
+}
+
+__device__ __forceinline__ void picard_maxima(const double* __restrict__ part, int nparts, double (&mx)[2])
+{
+    __shared__ double lds[2 * 16];
+    mx[0] = mx[1] = -INFINITY;
+    for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
+        mx[0] = fmax(mx[0], part[b]);
+        mx[1] = fmax(mx[1], part[kMaxBlocks + b]);
+    }
+    block_reduce<2, true, false>(mx, lds);
+}
+
+__global__ __launch_bounds__(kBlock) void k_picard_report(const double* part, int nparts, Gate gate, HostReport* rep)
+{
+    report_state(gate.st, rep);
+    if (!gate.open()) return;
+    double mx[2];
+    picard_maxima(part, nparts, mx);
+    if (threadIdx.x < 2) rep->red[threadIdx.x] = mx[threadIdx.x ? 1 : 0];
 }
 
 // After the increment: every block takes its maxima from the block partials (a maximum does not
@@ -357,40 +392,14 @@ __global__ __launch_bounds__(kBlock) void k_picard_inc(const double* x, const do
 template <int M>
 __global__ __launch_bounds__(kBlock) void k_picard_next(NextArgs a)
 {
-    if (a.st && a.st->gate != 2) return;
-    __shared__ double lds[2 * 16];
-    double mx[2] = {-INFINITY, -INFINITY};
-    for (int b = threadIdx.x; b < a.nparts; b += blockDim.x) {
-        mx[0] = fmax(mx[0], a.part[b]);
-        mx[1] = fmax(mx[1], a.part[kMaxBlocks + b]);
-    }
-    block_reduce<2, true, false>(mx, lds);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        a.red[0] = mx[0];
-        a.red[1] = mx[1];
-    }
+    if (blockIdx.x == 0) report_state(a.gate.st, a.rep);
+    if (!a.gate.open()) return;
+    double mx[2];
+    picard_maxima(a.part, a.nparts, mx);
+    if (blockIdx.x == 0 && threadIdx.x < 2) a.rep->red[threadIdx.x] = mx[threadIdx.x ? 1 : 0];
     if (mx[1] > 0.0) return;
     if (a.aa.active && mx[0] >= a.tol) b_aa_column<M>(a.aa, blockIdx.x);
     else if (a.fin) b_vg(a.vg, hw_blk());
-}
-
-// Maxima of rows 0 and 1 of a partial buffer (nparts blocks each) into out[0], out[1], in one
-// block: the host then reads two values instead of the rows (Picard increment and NaN flag;
-// a maximum does not depend on the order it is taken in).
-__global__ __launch_bounds__(kBlock) void k_max_rows2(const double* __restrict__ part, int nparts,
-                                                      double* __restrict__ out)
-{
-    __shared__ double lds[2 * 16];
-    double v[2] = {-INFINITY, -INFINITY};
-    for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
-        v[0] = fmax(v[0], part[b]);
-        v[1] = fmax(v[1], part[kMaxBlocks + b]);
-    }
-    block_reduce<2, true>(v, lds);
-    if (threadIdx.x == 0) {
-        out[0] = v[0];
-        out[1] = v[1];
-    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_vg_inverse(Geo g, Soil s, const double* theta, double* psi)
@@ -2498,14 +2507,9 @@ void launch_vg(hipStream_t s, const VgArgs& a)
     hipLaunchKernelGGL(k_vg, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
 }
 
-void launch_vg_picard(hipStream_t s, const VgArgs& a)
+void launch_vg_picard(hipStream_t s, const VgArgs& a, const Gate& gate)
 {
-    hipLaunchKernelGGL(k_vg_picard, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
-}
-
-void launch_vg_picard_gated(hipStream_t s, const VgArgs& a, const PcgState* st)
-{
-    hipLaunchKernelGGL(k_vg_picard_gated, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a, st);
+    hipLaunchKernelGGL(k_vg_picard, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a, gate);
 }
 
 void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const LaunchEv* ev)
@@ -2521,10 +2525,10 @@ void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const Launc
     }
 }
 
-void launch_picard_inc(hipStream_t s, const VgArgs& a, const PcgState* st)
+void launch_picard_inc(hipStream_t s, const VgArgs& a, const Gate& gate)
 {
-    hipLaunchKernelGGL(k_picard_inc, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a.psi, a.psi_m, a.g.n, a.rule,
-                       a.part_out, st);
+    hipLaunchKernelGGL(k_picard_inc, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a.psi, a.psi_m, a.g.n, a.rule, a.part_out,
+                       gate);
 }
 
 void launch_refine_conv(hipStream_t s, const double* part, int nparts, double lin_tol, PcgState* st)
@@ -2532,9 +2536,19 @@ void launch_refine_conv(hipStream_t s, const double* part, int nparts, double li
     hipLaunchKernelGGL(k_refine_conv, dim3(1), dim3(kBlock), 0, s, part, nparts, lin_tol, st);
 }
 
-void launch_max_rows2(hipStream_t s, const double* part, int nparts, double* out)
+void launch_picard_report(hipStream_t s, const double* part, int nparts, const Gate& gate, HostReport* rep)
 {
-    hipLaunchKernelGGL(k_max_rows2, dim3(1), dim3(kBlock), 0, s, part, nparts, out);
+    hipLaunchKernelGGL(k_picard_report, dim3(1), dim3(kBlock), 0, s, part, nparts, gate, rep);
+}
+
+void launch_report(hipStream_t s, const PcgState* st, HostReport* rep)
+{
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(kWave), 0, s, st, rep);
+}
+
+void launch_report_sums(hipStream_t s, const double* part, int nparts, int nv, HostReport* rep)
+{
+    hipLaunchKernelGGL(k_report_sums, dim3(1), dim3(nv * kWave), 0, s, part, nparts, nv, rep);
 }
 
 void launch_vg_inverse(hipStream_t s, const Geo& g, const Soil& soil, const double* theta, double* psi)
