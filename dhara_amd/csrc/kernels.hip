@@ -132,24 +132,30 @@ __global__ __launch_bounds__(kBlock) void k_vg_picard(VgArgs a, Gate gate)
 // gamma), pass 2 streams the planes once more (the update and vG); this pass's y waits in LDS.
 // The ring holds f and y themselves and not their differences: with a full ring of 3 a pass moves
 // 5 + 2 + 4 + 4 arrays (124 B per cell with K32) instead of 160 B, with the same differences.
-// Bytes bound it: 118 us a launch at 400 x 400 x 30 (672 MB / 130 us with the differences stored),
-// 750 us at 1024 x 1024 x 30 (909 us).  Sixteen chunks instead of four on small surfaces changed nothing.
+// Bytes bound it on large surfaces: 118 us a launch at 400 x 400 x 30 (672 MB / 130 us with the
+// differences stored), 750 us at 1024 x 1024 x 30 (909 us).  A surface of few columns is bound by the
+// chain of van Genuchten evaluations of a thread (about 1.7 us each, 515 dependent FP64 operations)
+// on the few CUs that its blocks reach: COLS = 16 columns per block spread it over four times the CUs
+// and four times the threads in pass 2; pass 1 keeps the four chunks, so the sums are the same
+// (32 x 32 x 20: 12.7 -> 8.8 us a launch).
 constexpr int kAaCols = 64, kAaChunks = kBlock / kAaCols;
+constexpr int kAaColsSmall = 16;
 constexpr int kAaLds = 32;   // planes whose y is kept in LDS
 
 // Block `bid` (kAaCols columns of cells) of the pass; every thread of the block calls it.
-template <int M>
+template <int M, int COLS>
 __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
 {
     constexpr int CH = kAaChunks, NV = M * (M + 1) / 2 + M;   // lower triangle of G, then dF^T f
-    __shared__ double share[CH][NV][kAaCols];
-    __shared__ double ysh[kAaLds][kAaCols];
+    constexpr int CH2 = kBlock / COLS;                        // chunks of pass 2
+    __shared__ double share[CH][NV][COLS];
+    __shared__ double ysh[kAaLds][COLS];
     const Geo g = a.g;
-    const int lane = threadIdx.x % kAaCols, chunk = threadIdx.x / kAaCols;
-    const int col = bid * kAaCols + lane;
+    const int lane = threadIdx.x % COLS, chunk = threadIdx.x / COLS;
+    const int col = bid * COLS + lane;
     const bool in = col < g.nxy, ylds = g.nz <= kAaLds;
     const int per = (g.nz + CH - 1) / CH;
-    const int k0 = min(g.nz, chunk * per), k1 = min(g.nz, k0 + per);
+    const int k0 = min(g.nz, chunk * per), k1 = min(g.nz, k0 + per);   // (chunk >= CH: none)
     const int nc = a.ncols;
     double G[M][M], rhs[M];
 #pragma unroll
@@ -200,7 +206,7 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
             c = cn;
         }
     }
-    {
+    if (chunk < CH) {
         int q = 0;
 #pragma unroll
         for (int i = 0; i < M; ++i)
@@ -281,17 +287,19 @@ __device__ __forceinline__ void b_aa_column(const AaArgs& a, int bid)
         gam[t] = keep[t] ? v / L[t][t] : 0.0;
     }
     const Soil& sl = a.soil;
-    if (k0 >= k1) return;
-    int c = k0 * g.nxy + col;
-    double yv = ylds ? ysh[k0][lane] : a.y[0][c], ks = sl.Ks[c], al = cell_alpha(sl, c), nv = cell_n(sl, c), yo[M];
+    const int per2 = (g.nz + CH2 - 1) / CH2;
+    const int m0 = min(g.nz, chunk * per2), m1 = min(g.nz, m0 + per2);
+    if (m0 >= m1) return;
+    int c = m0 * g.nxy + col;
+    double yv = ylds ? ysh[m0][lane] : a.y[0][c], ks = sl.Ks[c], al = cell_alpha(sl, c), nv = cell_n(sl, c), yo[M];
 #pragma unroll
     for (int t = 0; t < M; ++t) yo[t] = (t < nc) ? a.y[t + 1][c] : 0.0;
-    for (int k = k0; k < k1; ++k) {
+    for (int k = m0; k < m1; ++k) {
         const int cn = c + g.nxy;
         double y1 = 0.0, ks1 = 0.0, al1 = 0.0, nv1 = 0.0, yo1[M];
 #pragma unroll
         for (int t = 0; t < M; ++t) yo1[t] = 0.0;
-        if (k + 1 < k1) {
+        if (k + 1 < m1) {
             y1 = ylds ? ysh[k + 1][lane] : a.y[0][cn];
             ks1 = sl.Ks[cn];
             al1 = cell_alpha(sl, cn);
@@ -389,7 +397,7 @@ __global__ __launch_bounds__(kBlock) void k_picard_report(const double* part, in
 // depend on the order), and the launch is the Anderson update or theta, K, C of the converged x, or
 // (a NaN, or rule on theta and converged) neither.  One launch where the maxima, the update and the
 // final evaluation each took one of 2 to 4 us, two of them idle.
-template <int M>
+template <int M, int COLS>
 __global__ __launch_bounds__(kBlock) void k_picard_next(NextArgs a)
 {
     if (blockIdx.x == 0) report_state(a.gate.st, a.rep);
@@ -398,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void k_picard_next(NextArgs a)
     picard_maxima(a.part, a.nparts, mx);
     if (blockIdx.x == 0 && threadIdx.x < 2) a.rep->red[threadIdx.x] = mx[threadIdx.x ? 1 : 0];
     if (mx[1] > 0.0) return;
-    if (a.aa.active && mx[0] >= a.tol) b_aa_column<M>(a.aa, blockIdx.x);
+    if (a.aa.active && mx[0] >= a.tol) b_aa_column<M, COLS>(a.aa, blockIdx.x);
     else if (a.fin) b_vg(a.vg, hw_blk());
 }
 
@@ -1963,7 +1971,7 @@ __global__ __launch_bounds__(kBlock) void kb_aa_column(const AaArgs* __restrict_
 {
     const BlkMap e = map[blockIdx.x];
     if (active && !active[e.m]) return;
-    b_aa_column<M>(args[e.m], e.id);
+    b_aa_column<M, kAaCols>(args[e.m], e.id);
 }
 
 template <bool MIXED>
@@ -2512,16 +2520,27 @@ void launch_vg_picard(hipStream_t s, const VgArgs& a, const Gate& gate)
     hipLaunchKernelGGL(k_vg_picard, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a, gate);
 }
 
+// Fewer columns than one block of 64 per CU leave CUs idle: blocks of 16 there.  Where the blocks of 64
+// fill the chip, bytes bound the pass and 16 columns would only shorten the rows of a load to 128 B.
+template <int M>
+static void picard_next(hipStream_t s, const NextArgs& a, const LaunchEv* ev)
+{
+    const LaunchEv e = ev ? *ev : LaunchEv{};
+    const int n = a.aa.g.nxy;
+    if (n < 256 * kAaCols)
+        launch_ev(k_picard_next<M, kAaColsSmall>, dim3((n + kAaColsSmall - 1) / kAaColsSmall), dim3(kBlock), s, e, a);
+    else
+        launch_ev(k_picard_next<M, kAaCols>, dim3(aa_blocks(a.aa.g)), dim3(kBlock), s, e, a);
+}
+
 void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const LaunchEv* ev)
 {
-    const dim3 grid(aa_blocks(a.aa.g)), block(kBlock);
-    const LaunchEv e = ev ? *ev : LaunchEv{};
     switch (depth) {
-    case 1: launch_ev(k_picard_next<1>, grid, block, s, e, a); break;
-    case 2: launch_ev(k_picard_next<2>, grid, block, s, e, a); break;
-    case 3: launch_ev(k_picard_next<3>, grid, block, s, e, a); break;
-    case 4: launch_ev(k_picard_next<4>, grid, block, s, e, a); break;
-    default: launch_ev(k_picard_next<kAaMaxDepth>, grid, block, s, e, a); break;
+    case 1: picard_next<1>(s, a, ev); break;
+    case 2: picard_next<2>(s, a, ev); break;
+    case 3: picard_next<3>(s, a, ev); break;
+    case 4: picard_next<4>(s, a, ev); break;
+    default: picard_next<kAaMaxDepth>(s, a, ev); break;
     }
 }
 
