@@ -97,10 +97,10 @@ struct dhara_ensemble {
     bool c1_full = false;           // the members' whole-column tiles fill the chip together
     int kc_div = 0;                 // dhara_ensemble_autotune: planes per tile = ceil(nz / kc_div); 0: member's tile
     // column-preconditioned PCG (every member with DHARA_PRECOND_COLUMN): the column kernel's
-    // block maps, one per register-array size (nz <= 16, 32, 64)
+    // block map and the planes of the tallest member
     bool line = false;
-    dh::BlkMap* map_l[3] = {nullptr, nullptr, nullptr};
-    int nb_l[3] = {0, 0, 0};
+    dh::BlkMap* map_l = nullptr;
+    int line_nz = 0;
     // Anderson-accelerated Picard update (every member with the same picard_accel > 0): the
     // batched pass over aa_blocks(g) blocks per member
     int aa_depth = 0;
@@ -121,7 +121,7 @@ struct dhara_ensemble {
         std::vector<int> start, count;      // host: member m's blocks are full[start[m] ..)
         unsigned version = 0;               // active set the compaction was made for (0: none)
     };
-    CMap cm3, cm2, cml[3], cmaa;
+    CMap cm3, cm2, cml, cmaa;
     std::vector<int> act;                   // host copy of the active flags
     unsigned act_version = 1;
     std::vector<int*> pinned;
@@ -273,12 +273,8 @@ void krylov_batch(dhara_ensemble* e, bool two_d, int lg)
         } else if (e->line) {
             const MapRef r = use_map(e, e->cm3);
             dh::launch_batched_spmv_z(e->s, e->mixed, e->a_k3, r.map, r.n, e->active, e->it_base, k);
-            for (int b = 0; b < 3; ++b) {
-                const MapRef l = use_map(e, e->cml[b]);
-                if (l.n)
-                    dh::launch_batched_line(e->s, e->mixed, false, 16 << b, e->a_k3, l.map, l.n, e->active,
-                                            e->it_base, k);
-            }
+            const MapRef l = use_map(e, e->cml);
+            dh::launch_batched_line(e->s, e->mixed, false, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, k);
         } else if (e->one) {
             dh::launch_batched_cg1(e->s, e->mixed, e->a_c1, e->map_c1, e->nb_c1, e->active, e->it_base, k);
         } else {
@@ -326,11 +322,8 @@ int krylov_solve(dhara_ensemble* e, bool two_d, const std::vector<int>& on, int 
         EHIP(e, hipGetLastError());
     }
     if (!two_d && e->line) {   // z = T^-1 r of the fresh residual
-        for (int b = 0; b < 3; ++b) {
-            const MapRef l = use_map(e, e->cml[b]);
-            if (l.n)
-                dh::launch_batched_line(e->s, e->mixed, true, 16 << b, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
-        }
+        const MapRef l = use_map(e, e->cml);
+        dh::launch_batched_line(e->s, e->mixed, true, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
         EHIP(e, hipGetLastError());
     }
     const int off = two_d ? e->M : 0;
@@ -528,9 +521,9 @@ int mixed_line_solve(dhara_ensemble* e, const std::vector<int>& on, std::vector<
     for (int m = 0; m < M; ++m) e->h_k3f[m].seg0 = 0;
     if ((rc = upload_k3(e)) || (rc = set_active(e, solving))) return rc;
     EHIP(e, hipMemsetAsync(e->it_base, 0, sizeof(int), e->s));   // outside any captured graph
-    for (int b = 0; b < 3; ++b) {   // z = T^-1 r of the assembly's residual
-        const MapRef l = use_map(e, e->cml[b]);
-        if (l.n) dh::launch_batched_line(e->s, true, true, 16 << b, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
+    {   // z = T^-1 r of the assembly's residual
+        const MapRef l = use_map(e, e->cml);
+        dh::launch_batched_line(e->s, true, true, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
     }
     EHIP(e, hipGetLastError());
     const int maxit = e->mem[0]->p.inner_maxiter, maxr = e->mem[0]->p.refine_maxiter;
@@ -598,11 +591,8 @@ int mixed_line_solve(dhara_ensemble* e, const std::vector<int>& on, std::vector<
             const MapRef r = use_map(e, e->cm3);
             dh::launch_batched(e->s, dh::BK_REFINE_ADD, e->a_ref, r.map, r.n, e->active);
             dh::launch_batched(e->s, dh::BK_REFINE_RES, e->a_ref, r.map, r.n, e->active);
-            for (int b = 0; b < 3; ++b) {
-                const MapRef l = use_map(e, e->cml[b]);
-                if (l.n)
-                    dh::launch_batched_line(e->s, true, true, 16 << b, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
-            }
+            const MapRef l = use_map(e, e->cml);
+            dh::launch_batched_line(e->s, true, true, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
             EHIP(e, hipGetLastError());
             // a restarted segment is as long as the refinement segments before it
             lg = 0;
@@ -959,7 +949,7 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
     e->line = true;
     for (dhara_ctx* c : e->mem)
         if (c->p.precond != DHARA_PRECOND_COLUMN || !dh::line_supported(c->g)) e->line = false;
-    std::vector<dh::BlkMap> ml[3];
+    std::vector<dh::BlkMap> ml;
     if (e->line) {
         for (int m = 0; m < n; ++m) {
             dhara_ctx* c = e->mem[m];
@@ -967,9 +957,9 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
                 dhara_ensemble_destroy(e);
                 return DHARA_E_ALLOC;
             }
-            const int b = c->g.nz <= 16 ? 0 : c->g.nz <= 32 ? 1 : 2;
             const int nb = dh::line_blocks(c->g);
-            for (int i = 0; i < nb; ++i) ml[b].push_back(dh::BlkMap{m, i, nb});
+            for (int i = 0; i < nb; ++i) ml.push_back(dh::BlkMap{m, i, nb});
+            e->line_nz = std::max(e->line_nz, c->g.nz);
         }
     }
     // otherwise the one-kernel Jacobi PCG when every member asks for it (32-bit plane offsets)
@@ -1014,10 +1004,7 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
         if (!rc) rc = ealloc(e, &e->map_c1, mc1.size());
         if (!rc) rc = upload(e, e->map_c1, mc1);   // the first nb_c1 entries are live
     }
-    for (int b = 0; b < 3 && !rc; ++b) {
-        e->nb_l[b] = (int)ml[b].size();
-        if (e->nb_l[b] && !(rc = ealloc(e, &e->map_l[b], ml[b].size()))) rc = upload(e, e->map_l[b], ml[b]);
-    }
+    if (!rc && e->line && !(rc = ealloc(e, &e->map_l, ml.size()))) rc = upload(e, e->map_l, ml);
     e->aa_depth = e->mem[0]->p.picard_accel;
     std::vector<dh::BlkMap> ma;
     if (!rc && e->aa_depth > 0) {
@@ -1045,8 +1032,7 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
     }
     e->act.assign(n, -1);   // matches no active set: the first set_active records one
     if ((rc = init_cmap(e, e->cm3, e->map3, m3)) || (rc = init_cmap(e, e->cm2, e->map2, m2)) ||
-        (rc = init_cmap(e, e->cml[0], e->map_l[0], ml[0])) ||
-        (rc = init_cmap(e, e->cml[1], e->map_l[1], ml[1])) || (rc = init_cmap(e, e->cml[2], e->map_l[2], ml[2]))) {
+        (rc = init_cmap(e, e->cml, e->map_l, ml))) {
         dhara_ensemble_destroy(e);
         return rc;
     }

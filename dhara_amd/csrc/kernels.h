@@ -479,8 +479,8 @@ enum BatchKind { BK_VG = 0, BK_VG_PICARD, BK_SURF_PRE, BK_SURF_POST, BK_ASM_F64,
 void launch_batched(hipStream_t s, BatchKind kind, const void* args, const BlkMap* map, int nblocks,
                     const int* active);
 // Column-preconditioned form (untiled SpMV with z as input over map3; the column kernel over a map
-// of line_blocks(g) blocks per member, one launch per register-array size nzm = 16, 32, 64; init:
-// the start-up z = T^-1 r of a fresh residual).
+// of line_blocks(g) blocks per member, nz_max the planes of the tallest member; init: the start-up
+// z = T^-1 r of a fresh residual).
 void launch_batched_spmv_z(hipStream_t s, bool fp32, const void* kargs, const BlkMap* map, int nblocks,
                            const int* active, const int* it_base, int k);
 // Anderson pass of the active members (the host has decided), over a map of aa_blocks(g) blocks
@@ -488,7 +488,7 @@ void launch_batched_spmv_z(hipStream_t s, bool fp32, const void* kargs, const Bl
 void launch_batched_aa(hipStream_t s, int depth, const AaArgs* args, const BlkMap* map, int nblocks,
                        const int* active);
 int aa_blocks(const Geo& g);
-void launch_batched_line(hipStream_t s, bool fp32, bool init, int nzm, const void* kargs, const BlkMap* map,
+void launch_batched_line(hipStream_t s, bool fp32, bool init, int nz_max, const void* kargs, const BlkMap* map,
                          int nblocks, const int* active, const int* it_base, int k);
 void launch_batched_spmv3(hipStream_t s, bool fp32, const void* kargs, const BlkMap* map, int nblocks,
                           const int* active, const int* it_base, int k);

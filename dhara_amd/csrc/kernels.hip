@@ -974,7 +974,7 @@ __device__ __forceinline__ double jac_inv(double d)
 // Column (vertical line) preconditioner: z = T^-1 r with T the vertical tridiagonal part of the
 // 7-point operator -- diagonal D, coupling to the cell above / below -(wz/2)(K_k + K_k-+1), as
 // in the SpMV --, i.e. one independent tridiagonal system per column of cells, solved by the
-// Thomas algorithm with the column's forward factors in registers (NZM >= nz).  The flow
+// Thomas algorithm with the column's forward sweep in LDS.  The flow
 // operator's vertical couplings exceed the horizontal ones by (dx/dz)^2 (400 at dz = 5 cm);
 // Jacobi scaling leaves that stiffness to the Krylov iteration, the column solve removes it.
 // Thread = column: the plane-major layout makes every plane access coalesced.
@@ -986,14 +986,32 @@ __device__ __forceinline__ double jac_inv(double d)
 // (r, z) is accumulated as sum_k w_k y_k with w_k = r_k - a_k y_k-1 = den_k y_k (T = L diag(den)
 // L^T): the same value as sum_k r_k z_k, as a sum of positive terms.  The reciprocal of the
 // pivot is jac_inv, a fixed function of the operator, so every application is the same
-// linear map.  In FP64 the upper factors c'_k wait in z itself (written in the forward sweep,
-// overwritten by the back substitution) instead of registers: 2 x 32 doubles per thread would
-// leave 2 waves per SIMD, too few for the 2.5 waves of columns of a 400 x 400 surface.
-template <typename T, int NZM, bool INIT>
-__device__ __forceinline__ void b_line(Geo g, const T* __restrict__ K, const T* __restrict__ D, T* __restrict__ x,
-                                       T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ q,
-                                       T* __restrict__ z, SolveCtl sc, Blk bk)
+// linear map.
+//
+// A column's planes form a chain (elimination down, substitution up) and a thread owns a column,
+// so a surface of some 10^4 columns has one or two waves per SIMD to hide memory latency with:
+// the loads of A planes are in flight ahead of the plane in work, in registers.  y_k of every plane
+// waits in LDS, and so does c'_k in FP32; in FP64 c'_k waits in z itself (written in the forward
+// sweep, read back A planes ahead of the substitution, overwritten by it): 8 B per plane and thread
+// in both, two blocks per CU up to 40 planes.  With y in registers instead (arrays of 16, 32 or 64
+// planes, unrolled) each plane waited for its own loads, since a plane that may not exist ends the
+// unrolled block, and the batched form needed a launch per array size.  Working launches, registers
+// -> LDS: update FP64 333 x 187 x 24 30 -> 24 us (131 MB), 300 x 300 x 40 87 -> 62 us, 450 x 450 x 30
+// 126 -> 106 us, 800 x 800 x 30 316 -> 294 us (bytes); FP32 150 x 150 x 40 26 -> 13 us, 450 x 450 x 30
+// 55 -> 48 us, 1024 x 1024 x 30 232 -> 223 us, 400 x 400 x 30 34.6 -> 36.7 us (1.2 rounds of resident
+// blocks), 800 x 800 x 12 49 -> 52 us; start-up FP64 333 x 187 x 24 24 -> 17 us; 20 models of
+// 32..128 x 32..128 x 10..40 in FP64, all iterating: 95 us in three launches -> 50 us in one.
+template <typename T>
+struct LinePlane {
+    T r, q, p, x, K, D;
+};
+
+template <typename T, bool INIT>
+__device__ __forceinline__ void b_line(Geo g, const T* __restrict__ K, const T* __restrict__ D,
+                                           T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
+                                           const T* __restrict__ q, T* __restrict__ z, SolveCtl sc, Blk bk)
 {
+    extern __shared__ double line_lds[];
     double alpha_d = 0.0;
     double carry[2] = {0.0, 0.0};
     if constexpr (INIT) {
@@ -1005,99 +1023,121 @@ __device__ __forceinline__ void b_line(Geo g, const T* __restrict__ K, const T* 
     } else {
         if (!update_begin(sc, alpha_d, bk.id)) return;
     }
+    constexpr int A = INIT ? 8 : 4;   // planes ahead
+    constexpr bool kCpInZ = sizeof(T) == 8;
     const T alpha = (T)alpha_d;
     const T hz = (T)(0.5 * g.wz);
     const int nz = g.nz, nxy = g.nxy;
+    T* ysh = reinterpret_cast<T*>(line_lds) + threadIdx.x;   // y_k at ysh[k * kBlock]
+    T* csh = ysh + nz * kBlock;                              // c'_k (FP32)
     double acc[INIT ? 4 : 2] = {};
-    constexpr bool kCpInZ = sizeof(T) == 8;
-    // The start-up loads its planes in groups of G: the loads of a group are issued together and
-    // the group is then eliminated plane by plane, so a column pays one memory latency per group
-    // instead of one per plane (one column per thread leaves ~2.4 waves per SIMD on a 400 x 400
-    // surface, too few to hide a latency per plane); its FP64 back substitution reads the stored
-    // factors c'_k in groups the same way.  The update streams twice the arrays and runs at 0.7
-    // of the HBM peak plane by plane; grouped, its 48 plane streams per wave measured slower.
-    constexpr int G = INIT ? (sizeof(T) == 4 ? 8 : 4) : 1;
     for (int col = bk.id * kBlock + threadIdx.x; col < nxy; col += bk.n * kBlock) {
-        T y[NZM], cp[kCpInZ ? 1 : NZM];
-        T kprev = T(0), yprev = T(0), inv_prev = T(0);
-#pragma unroll
-        for (int k0 = 0; k0 < NZM; k0 += G) {
-            if (k0 < nz) {
-                T rb[G], qb[G], pb[G], xb[G], kb[G], db[G];
-#pragma unroll
-                for (int u = 0; u < G; ++u) {
-                    const int c = (k0 + u) * nxy + col;
-                    if (G > 1 && k0 + u < nz) {
-                        rb[u] = r[c];
-                        if constexpr (!INIT) {
-                            qb[u] = q[c];
-                            pb[u] = p[c];
-                            xb[u] = x[c];
-                        }
-                        kb[u] = K[c];
-                        db[u] = D[c];
-                    }
+        // c: the plane in work; ld: the next plane to load (it stays on the last plane once there:
+        // those loads are not used)
+        int c = col, ld = col, left = nz - 1;
+        LinePlane<T> buf[A];
+        auto fetch = [&](LinePlane<T>& b) {
+            b.r = r[ld];
+            if constexpr (!INIT) {
+                b.q = q[ld];
+                b.p = p[ld];
+                b.x = x[ld];
+            }
+            b.K = K[ld];
+            b.D = D[ld];
+            ld += left > 0 ? nxy : 0;
+            --left;
+        };
+        T kprev = T(0), yprev = T(0), inv_prev = T(0);   // (K above the first plane: its coupling is 0)
+        T *ys = ysh, *cs = csh;
+        auto plane = [&](const LinePlane<T>& b, bool top) {
+            T rc = b.r;
+            if constexpr (!INIT) {
+                rc -= alpha * b.q;
+                r[c] = rc;
+                x[c] = b.x + alpha * b.p;
+            }
+            T den = b.D, w = rc;
+            if (!top) {
+                const T a = -hz * (b.K + kprev);   // T[k][k-1] = T[k-1][k]
+                const T cpk = a * inv_prev;        // c'_{k-1}
+                if constexpr (kCpInZ) {
+                    z[c - nxy] = cpk;
+                } else {
+                    *cs = cpk;
+                    cs += kBlock;
                 }
+                den -= a * cpk;
+                w -= a * yprev;
+            }
+            const T inv = jac_inv(den);
+            const T yk = w * inv;
+            *ys = yk;
+            ys += kBlock;
+            acc[0] += (double)w * (double)yk;
+            acc[1] += (double)rc * (double)rc;
+            kprev = b.K;
+            asm volatile("" : "+v"(kprev));   // a copy: the slot's register is free for the next load
+            yprev = yk;
+            inv_prev = inv;
+            c += nxy;
+        };
+        LinePlane<T> b0;
+        fetch(b0);
 #pragma unroll
-                for (int u = 0; u < G; ++u) {
-                    const int k = k0 + u;
-                    if (k < nz) {
-                        const int c = k * nxy + col;
-                        // (G == 1: operands read where they are used, the plane-by-plane order)
-                        T rc = G > 1 ? rb[u] : r[c];
-                        if constexpr (!INIT) {
-                            rc -= alpha * (G > 1 ? qb[u] : q[c]);
-                            r[c] = rc;
-                            x[c] = (G > 1 ? xb[u] : x[c]) + alpha * (G > 1 ? pb[u] : p[c]);
-                        }
-                        const T kc = G > 1 ? kb[u] : K[c];
-                        T den = G > 1 ? db[u] : D[c], w = rc;
-                        if (k > 0) {
-                            const T a = -hz * (kc + kprev);   // T[k][k-1] = T[k-1][k]
-                            const T cpk = a * inv_prev;       // c'_{k-1}
-                            if constexpr (kCpInZ) z[c - nxy] = cpk;
-                            else cp[k - 1] = cpk;
-                            den -= a * cpk;
-                            w -= a * yprev;
-                        }
-                        const T inv = jac_inv(den);
-                        const T yk = w * inv;
-                        y[k] = yk;
-                        acc[0] += (double)w * (double)yk;
-                        acc[1] += (double)rc * (double)rc;
-                        kprev = kc;
-                        yprev = yk;
-                        inv_prev = inv;
-                    }
-                }
+        for (int u = 0; u < A; ++u) fetch(buf[u]);
+        plane(b0, true);
+        int k = 1;
+        for (; k + A <= nz; k += A) {
+#pragma unroll
+            for (int u = 0; u < A; ++u) {
+                plane(buf[u], false);
+                fetch(buf[u]);
+                __builtin_amdgcn_sched_barrier(0);   // else a later plane's r - alpha q is taken here, and waits
             }
         }
-        T zn = T(0);
 #pragma unroll
-        for (int k1 = NZM - 1; k1 >= 0; k1 -= G) {
-            if (k1 - G + 1 < nz) {
-                T cb[G];
-                if constexpr (kCpInZ && G > 1) {
+        for (int u = 0; u < A; ++u)
+            if (k + u < nz) plane(buf[u], false);
+        // back substitution
+        c -= nxy;
+        ys -= kBlock;
+        T zn = *ys;
+        z[c] = zn;
+        if constexpr (kCpInZ) {
+            T cb[A];
+            int lb = c, bl = nz - 1;   // planes above the one at lb
+            auto back = [&](T& b) {
+                lb -= bl > 0 ? nxy : 0;
+                --bl;
+                b = z[lb];
+            };
+            auto sub = [&](T cp) {
+                c -= nxy;
+                ys -= kBlock;
+                zn = *ys - cp * zn;
+                z[c] = zn;
+            };
 #pragma unroll
-                    for (int u = 0; u < G; ++u) {
-                        const int k = k1 - u;
-                        if (k < nz - 1) cb[u] = z[k * nxy + col];
-                    }
+            for (int u = 0; u < A; ++u) back(cb[u]);
+            int n = nz - 1;
+            for (; n >= A; n -= A) {
+#pragma unroll
+                for (int u = 0; u < A; ++u) {
+                    sub(cb[u]);
+                    back(cb[u]);
                 }
+            }
 #pragma unroll
-                for (int u = 0; u < G; ++u) {
-                    const int k = k1 - u;
-                    if (k < nz) {
-                        const int c = k * nxy + col;
-                        T zk = y[k];
-                        if (k < nz - 1) {
-                            if constexpr (kCpInZ) zk -= (G > 1 ? cb[u] : z[c]) * zn;
-                            else zk -= cp[k] * zn;
-                        }
-                        z[c] = zk;
-                        zn = zk;
-                    }
-                }
+            for (int u = 0; u < A; ++u)
+                if (u < n) sub(cb[u]);
+        } else {
+            for (int n = nz - 1; n > 0; --n) {
+                c -= nxy;
+                ys -= kBlock;
+                cs -= kBlock;
+                zn = *ys - *cs * zn;
+                z[c] = zn;
             }
         }
     }
@@ -1112,12 +1152,12 @@ __device__ __forceinline__ void b_line(Geo g, const T* __restrict__ K, const T* 
     }
 }
 
-template <typename T, int NZM, bool INIT>
+template <typename T, bool INIT>
 __global__ __launch_bounds__(kBlock) void k_line(Geo g, const T* __restrict__ K, const T* __restrict__ D,
-                                                 T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
-                                                 const T* __restrict__ q, T* __restrict__ z, SolveCtl sc)
+                                                     T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
+                                                     const T* __restrict__ q, T* __restrict__ z, SolveCtl sc)
 {
-    b_line<T, NZM, INIT>(g, K, D, x, r, p, q, z, sc, hw_blk());
+    b_line<T, INIT>(g, K, D, x, r, p, q, z, sc, hw_blk());
 }
 
 // SpMV kernel of the column-preconditioned PCG: p = z + beta p_old, q = A p, partial (p, q), on a
@@ -2025,7 +2065,7 @@ __global__ __launch_bounds__(kBlock) void kb_spmv_z(const KrylovArgs<T>* __restr
                                 Blk{e.id, e.n});
 }
 
-template <typename T, int NZM, bool INIT>
+template <typename T, bool INIT>
 __global__ __launch_bounds__(kBlock) void kb_line(const KrylovArgs<T>* __restrict__ args,
                                                   const BlkMap* __restrict__ map, const int* __restrict__ active,
                                                   const int* __restrict__ it_base, int k)
@@ -2035,7 +2075,7 @@ __global__ __launch_bounds__(kBlock) void kb_line(const KrylovArgs<T>* __restric
     const KrylovArgs<T>& a = args[e.m];
     SolveCtl sc = INIT ? a.init : a.upd;
     sc.it = INIT ? 0 : *it_base + k - a.seg0;
-    b_line<T, NZM, INIT>(a.g, a.K, a.D, a.x, a.res, a.p[(sc.it + 1) & 1], a.q, a.z, sc, Blk{e.id, e.n});
+    b_line<T, INIT>(a.g, a.K, a.D, a.x, a.res, a.p[(sc.it + 1) & 1], a.q, a.z, sc, Blk{e.id, e.n});
 }
 
 __global__ __launch_bounds__(kBlock) void kb_spmv2(const KrylovArgs<double>* __restrict__ args,
@@ -2818,6 +2858,9 @@ void launch_pcg3_spmv_z_f32(hipStream_t s, const Geo& g, const TileCfg& t, const
 
 bool line_supported(const Geo& g) { return g.nz >= 1 && g.nz <= kLineMaxNz; }
 
+// y (FP64) or y and c' (FP32) of a block's columns: 128 KB of the CU's 160 KB at kLineMaxNz planes.
+static size_t line_lds_bytes(int nz) { return (size_t)nz * kBlock * 8; }
+
 int line_blocks(const Geo& g) { return std::min((g.nxy + kBlock - 1) / kBlock, kMaxBlocks / 2); }
 
 template <typename T, bool INIT>
@@ -2825,9 +2868,8 @@ static void line_launch(hipStream_t s, const Geo& g, const T* K, const T* D, T* 
                         T* z, const SolveCtl& sc, const LaunchEv& ev)
 {
     const dim3 gr(line_blocks(g)), bl(kBlock);
-    if (g.nz <= 16) launch_ev(k_line<T, 16, INIT>, gr, bl, s, ev, g, K, D, x, r, p, q, z, sc);
-    else if (g.nz <= 32) launch_ev(k_line<T, 32, INIT>, gr, bl, s, ev, g, K, D, x, r, p, q, z, sc);
-    else launch_ev(k_line<T, 64, INIT>, gr, bl, s, ev, g, K, D, x, r, p, q, z, sc);
+    hipExtLaunchKernelGGL((k_line<T, INIT>), gr, bl, line_lds_bytes(g.nz), s, ev.start, ev.stop, 0, g, K, D, x, r, p,
+                          q, z, sc);
 }
 
 void launch_line_init_f64(hipStream_t s, const Geo& g, const double* K, const double* D, const double* r, double* z,
@@ -3005,25 +3047,19 @@ void launch_batched_spmv_z(hipStream_t s, bool fp32, const void* kargs, const Bl
                            map, active, it_base, k);
 }
 
-template <typename T, bool INIT>
-static void batched_line(hipStream_t s, int nzm, const void* kargs, const BlkMap* map, int nblocks,
-                         const int* active, const int* it_base, int k)
-{
-    const KrylovArgs<T>* a = (const KrylovArgs<T>*)kargs;
-    if (nzm <= 16) hipLaunchKernelGGL((kb_line<T, 16, INIT>), dim3(nblocks), dim3(kBlock), 0, s, a, map, active, it_base, k);
-    else if (nzm <= 32) hipLaunchKernelGGL((kb_line<T, 32, INIT>), dim3(nblocks), dim3(kBlock), 0, s, a, map, active, it_base, k);
-    else hipLaunchKernelGGL((kb_line<T, 64, INIT>), dim3(nblocks), dim3(kBlock), 0, s, a, map, active, it_base, k);
-}
-
-void launch_batched_line(hipStream_t s, bool fp32, bool init, int nzm, const void* kargs, const BlkMap* map,
+void launch_batched_line(hipStream_t s, bool fp32, bool init, int nz_max, const void* kargs, const BlkMap* map,
                          int nblocks, const int* active, const int* it_base, int k)
 {
+    const dim3 gr(nblocks), bl(kBlock);
+    const size_t lds = line_lds_bytes(nz_max);
     if (fp32) {
-        if (init) batched_line<float, true>(s, nzm, kargs, map, nblocks, active, it_base, k);
-        else batched_line<float, false>(s, nzm, kargs, map, nblocks, active, it_base, k);
+        const KrylovArgs<float>* a = (const KrylovArgs<float>*)kargs;
+        if (init) hipLaunchKernelGGL((kb_line<float, true>), gr, bl, lds, s, a, map, active, it_base, k);
+        else hipLaunchKernelGGL((kb_line<float, false>), gr, bl, lds, s, a, map, active, it_base, k);
     } else {
-        if (init) batched_line<double, true>(s, nzm, kargs, map, nblocks, active, it_base, k);
-        else batched_line<double, false>(s, nzm, kargs, map, nblocks, active, it_base, k);
+        const KrylovArgs<double>* a = (const KrylovArgs<double>*)kargs;
+        if (init) hipLaunchKernelGGL((kb_line<double, true>), gr, bl, lds, s, a, map, active, it_base, k);
+        else hipLaunchKernelGGL((kb_line<double, false>), gr, bl, lds, s, a, map, active, it_base, k);
     }
 }
 

@@ -4,8 +4,8 @@ dense solves in test_oracle_known_answers.py).
 
 Same method and stopping rule (||r|| <= 1e-12 ||b||): heads within the FP64 parity bound
 (1e-8 m) of the oracle, Krylov counts within one per solve, and several times fewer Krylov
-iterations than Jacobi on the thin-layer (dz = 5 cm) workloads.  Column lengths cover the three
-register-array sizes of the column kernel (nz <= 16, <= 32, <= 64); nz > 64 and Dirichlet rows
+iterations than Jacobi on the thin-layer (dz = 5 cm) workloads.  Column lengths cover the
+range of the column kernel (up to 64 planes); nz > 64 and Dirichlet rows
 fall back to Jacobi.
 """
 import numpy as np
