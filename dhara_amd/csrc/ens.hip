@@ -6,7 +6,7 @@
 //   * every kernel is launched once for all members: a block map sends physical block b to
 //     block map[b].id of model map[b].m, which reads that model's argument struct, so one
 //     launch covers ~sum N cells (>> 256 workgroups even when each member is small); the maps
-//     are compacted on the device to the members still iterating (use_map);
+//     are compacted on the device to the members still iterating (set_active);
 //   * members run in lockstep through the step -- surface pass, Picard iterations, Krylov
 //     solves, end of step, overland solve -- and a member that has converged drops out through
 //     its active flag (its blocks return at once); every member keeps its own Picard and
@@ -15,8 +15,12 @@
 //     captured once per size as a hipGraph and replayed while every member is active (eager
 //     launches over compacted maps otherwise); the kernels take the iteration index from a
 //     device counter that the batch's last node advances, so every replay is the same graph;
-//   * per-member reductions go through one kernel writing all members' sums, one copy to the
-//     host; the members' solver states sit in one array, one copy per batch.
+//   * per-member reductions go through one kernel that writes all members' sums to pinned host
+//     memory; the members' solver states sit in one array, which a batch's last node writes there;
+//   * what the host sends (active sets, changed argument images) goes through pinned staging and
+//     waits for nothing, so the host waits once per Krylov batch and once per reduction.  With a
+//     copy and a wait for each of them: 26.7 -> 24.9 ms (two steps of 20 models of 32..128 x 32..128 x
+//     10..40, FP64), 26.1 -> 22.3 ms (12 models, mixed: a refinement round changes the set twice).
 // Mixed precision here is FP32 PCG with FP64 iterative refinement that restarts the FP32
 // recurrence after each refinement: in lockstep rounds for the Jacobi forms, per member inside
 // the running batches for the column form (mixed_line_solve).  A member's overland solve is the
@@ -47,14 +51,19 @@ struct dhara_ensemble {
     dh::BlkMap *map3 = nullptr, *map2 = nullptr;
     int nb3 = 0, nb2 = 0;
     int* active = nullptr;        // device, M
-    int* h_active = nullptr;      // pinned
+    // Pinned staging of what the host sends between two waits for the stream: active sets (slots of
+    // M flags, read by k_activate) and argument images.  Every wait frees all of it; a full one waits.
+    static constexpr int kFlagSlots = 64;
+    int* h_flags = nullptr;
+    int flags_used = 0;
+    char* stage = nullptr;
+    size_t stage_size = 0, stage_used = 0;
     int* it_base = nullptr;
     dh::PcgState* st = nullptr;   // device, 2M: subsurface then overland
-    dh::PcgState* h_st = nullptr; // pinned
+    dh::PcgState* h_st = nullptr; // pinned, written by k_advance
     double** parts = nullptr;     // device, M (each member's partial buffer A)
     int *np3 = nullptr, *np2 = nullptr;
-    double* red = nullptr;        // device, M * kMaxSums
-    double* h_red = nullptr;      // pinned
+    double* h_red = nullptr;      // pinned, M * kMaxSums, written by k_reduce_models
     // argument arrays (device) and their host images
     dh::VgArgs* a_vg = nullptr;
     dh::SurfArgs* a_surf = nullptr;
@@ -109,22 +118,18 @@ struct dhara_ensemble {
     std::vector<dh::AaArgs> h_aa;
     // Block maps restricted to the active members: a batched launch over the full map spends a
     // block's dependent loads (map entry, active flag, solver state) on every block of an
-    // inactive member, which is most of the grid once most members have converged.  Each map
-    // is compacted on the device the first time it is used after the active set changed.
+    // inactive member, which is most of the grid once most members have converged.  k_activate
+    // makes all of them when the active set changes.
     struct CMap {
         const dh::BlkMap* full = nullptr;
         int n_full = 0;
         dh::BlkMap* cur = nullptr;          // device, n_full entries
-        int n_cur = 0;
-        int* seg = nullptr;                 // device, 3 M: start, count, offset per active member
-        int* h_seg = nullptr;               // pinned, 3 M
-        std::vector<int> start, count;      // host: member m's blocks are full[start[m] ..)
-        unsigned version = 0;               // active set the compaction was made for (0: none)
+        int n_cur = 0;                      // 0: the full map
+        std::vector<int> start, count;      // member m's blocks are full[start[m] ..)
+        int *d_start = nullptr, *d_count = nullptr;
     };
     CMap cm3, cm2, cml, cmaa;
     std::vector<int> act;                   // host copy of the active flags
-    unsigned act_version = 1;
-    std::vector<int*> pinned;
     // the last image uploaded to each argument array: an unchanged image is not sent again (the
     // arrays are read-only on the device), which saves a host synchronisation per launch group
     std::unordered_map<const void*, std::vector<unsigned char>> uploaded;
@@ -162,6 +167,15 @@ int upload(dhara_ensemble* e, T* dev, const std::vector<T>& host)
     return DHARA_OK;
 }
 
+// Waits for the stream; the staging memory is free again.
+int wait(dhara_ensemble* e)
+{
+    EHIP(e, hipStreamSynchronize(e->s));
+    e->flags_used = 0;
+    e->stage_used = 0;
+    return DHARA_OK;
+}
+
 // Upload of an argument array, skipped when the image equals the last one sent.
 template <typename T>
 int upload_args(dhara_ensemble* e, T* dev, const std::vector<T>& host)
@@ -169,23 +183,42 @@ int upload_args(dhara_ensemble* e, T* dev, const std::vector<T>& host)
     const size_t nb = host.size() * sizeof(T);
     std::vector<unsigned char>& last = e->uploaded[dev];
     if (last.size() == nb && std::memcmp(last.data(), host.data(), nb) == 0) return DHARA_OK;
-    int rc = upload(e, dev, host);
-    if (rc) return rc;
+    int rc;
+    if (nb > e->stage_size) {
+        if ((rc = upload(e, dev, host))) return rc;
+    } else {
+        if (e->stage_used + nb > e->stage_size && (rc = wait(e))) return rc;
+        char* at = e->stage + e->stage_used;
+        std::memcpy(at, host.data(), nb);
+        EHIP(e, hipMemcpyAsync(dev, at, nb, hipMemcpyHostToDevice, e->s));
+        e->stage_used += (nb + 63) / 64 * 64;
+    }
     last.assign(reinterpret_cast<const unsigned char*>(host.data()),
                 reinterpret_cast<const unsigned char*>(host.data()) + nb);
     return DHARA_OK;
 }
 
 // The active flags of the members for the launches that follow (unchanged flags are not sent
-// again).  When it sends them it synchronises the stream, which use_map relies on.
+// again) and the block maps restricted to them, in one launch that reads the flags from pinned
+// memory: the host neither copies nor waits.
 int set_active(dhara_ensemble* e, const std::vector<int>& on)
 {
     if (e->act == on) return DHARA_OK;
+    int rc;
+    if (e->flags_used == dhara_ensemble::kFlagSlots && (rc = wait(e))) return rc;
+    int* flags = e->h_flags + (size_t)e->flags_used++ * e->M;
+    std::copy(on.begin(), on.end(), flags);
+    dh::ActMaps maps{};
+    for (dhara_ensemble::CMap* cm : {&e->cm3, &e->cm2, &e->cml, &e->cmaa}) {
+        int tot = 0;
+        for (int m = 0; m < e->M; ++m)
+            if (on[m] && cm->n_full) tot += cm->count[m];
+        cm->n_cur = tot == cm->n_full ? 0 : tot;
+        if (cm->n_cur) maps.m[maps.n++] = dh::ActMap{cm->full, cm->d_start, cm->d_count, cm->cur};
+    }
     e->act = on;
-    ++e->act_version;
-    std::copy(on.begin(), on.end(), e->h_active);
-    EHIP(e, hipMemcpyAsync(e->active, e->h_active, e->M * sizeof(int), hipMemcpyHostToDevice, e->s));
-    EHIP(e, hipStreamSynchronize(e->s));
+    dh::launch_activate(e->s, flags, e->M, e->active, maps);
+    EHIP(e, hipGetLastError());
     return DHARA_OK;
 }
 
@@ -194,34 +227,9 @@ struct MapRef {
     int n;
 };
 
-// The block map `cm` restricted to the active members (the full map when all, or none, are, or
-// when the compaction could not be queued).
-// The stream has been synchronised since the last set_active (it synchronises), so the pinned
-// segment list of this map is free to rewrite when the active set has changed.
-MapRef use_map(dhara_ensemble* e, dhara_ensemble::CMap& cm)
-{
-    if (cm.n_full == 0) return {cm.full, 0};
-    if (cm.version != e->act_version) {
-        cm.version = e->act_version;
-        int nseg = 0, tot = 0;
-        for (int m = 0; m < e->M; ++m) {
-            if (!e->act[m] || cm.count[m] == 0) continue;
-            cm.h_seg[3 * nseg] = cm.start[m];
-            cm.h_seg[3 * nseg + 1] = cm.count[m];
-            cm.h_seg[3 * nseg + 2] = tot;
-            tot += cm.count[m];
-            ++nseg;
-        }
-        cm.n_cur = 0;   // the full map: always correct (the kernels test the active flags)
-        if (tot != 0 && tot != cm.n_full &&
-            hipMemcpyAsync(cm.seg, cm.h_seg, (size_t)3 * nseg * sizeof(int), hipMemcpyHostToDevice, e->s) ==
-                hipSuccess) {
-            dh::launch_compact_map(e->s, cm.full, cm.seg, nseg, tot, cm.cur);
-            if (hipGetLastError() == hipSuccess) cm.n_cur = tot;   // else keep launching the full map
-        }
-    }
-    return cm.n_cur ? MapRef{cm.cur, cm.n_cur} : MapRef{cm.full, cm.n_full};
-}
+// The block map `cm` restricted to the active members (the full map when all, or none, are: the
+// kernels test the active flags).
+MapRef use_map(const dhara_ensemble::CMap& cm) { return cm.n_cur ? MapRef{cm.cur, cm.n_cur} : MapRef{cm.full, cm.n_full}; }
 
 // Compacted maps: device buffers and the members' block ranges of a full map.
 int init_cmap(dhara_ensemble* e, dhara_ensemble::CMap& cm, const dh::BlkMap* full_dev,
@@ -237,43 +245,35 @@ int init_cmap(dhara_ensemble* e, dhara_ensemble::CMap& cm, const dh::BlkMap* ful
     }
     if (cm.n_full == 0) return DHARA_OK;
     int rc = ealloc(e, &cm.cur, full.size());
-    if (!rc) rc = ealloc(e, &cm.seg, (size_t)3 * e->M);
-    if (rc) return rc;
-    if (hipHostMalloc((void**)&cm.h_seg, (size_t)3 * e->M * sizeof(int)) != hipSuccess)
-        return eset(e, DHARA_E_ALLOC, "hipHostMalloc");
-    e->pinned.push_back(cm.h_seg);
-    return DHARA_OK;
+    if (!rc) rc = ealloc(e, &cm.d_start, e->M);
+    if (!rc) rc = ealloc(e, &cm.d_count, e->M);
+    if (!rc) rc = upload(e, cm.d_start, cm.start);
+    if (!rc) rc = upload(e, cm.d_count, cm.count);
+    return rc;
 }
 
-int read_states(dhara_ensemble* e)
-{
-    EHIP(e, hipMemcpyAsync(e->h_st, e->st, 2 * e->M * sizeof(dh::PcgState), hipMemcpyDeviceToHost, e->s));
-    EHIP(e, hipStreamSynchronize(e->s));
-    return DHARA_OK;
-}
-
+// The members' sums or maxima in e->h_red.
 int reduce(dhara_ensemble* e, bool two_d, int nv, bool take_max)
 {
-    dh::launch_reduce_models(e->s, e->M, e->parts, two_d ? e->np2 : e->np3, nv, take_max, e->red);
+    dh::launch_reduce_models(e->s, e->M, e->parts, two_d ? e->np2 : e->np3, nv, take_max, e->h_red);
     EHIP(e, hipGetLastError());
-    EHIP(e, hipMemcpyAsync(e->h_red, e->red, (size_t)e->M * nv * sizeof(double), hipMemcpyDeviceToHost, e->s));
-    EHIP(e, hipStreamSynchronize(e->s));
-    return DHARA_OK;
+    return wait(e);
 }
 
-// One batch of 1 << lg Krylov iterations for every member whose active flag is set.
+// One batch of 1 << lg Krylov iterations for every member whose active flag is set; leaves the
+// solver states in e->h_st.
 void krylov_batch(dhara_ensemble* e, bool two_d, int lg)
 {
     const int nb = 1 << lg;
     for (int k = 0; k < nb; ++k) {
         if (two_d) {
-            const MapRef r = use_map(e, e->cm2);
+            const MapRef r = use_map(e->cm2);
             dh::launch_batched_spmv2(e->s, e->a_k2, r.map, r.n, e->active, e->it_base, k);
             dh::launch_batched_update2(e->s, e->a_k2, r.map, r.n, e->active, e->it_base, k);
         } else if (e->line) {
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched_spmv_z(e->s, e->mixed, e->a_k3, r.map, r.n, e->active, e->it_base, k);
-            const MapRef l = use_map(e, e->cml);
+            const MapRef l = use_map(e->cml);
             dh::launch_batched_line(e->s, e->mixed, false, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, k);
         } else if (e->one) {
             dh::launch_batched_cg1(e->s, e->mixed, e->a_c1, e->map_c1, e->nb_c1, e->active, e->it_base, k);
@@ -282,7 +282,7 @@ void krylov_batch(dhara_ensemble* e, bool two_d, int lg)
             dh::launch_batched_update3(e->s, e->mixed, e->a_k3, e->map3, e->nb3, e->active, e->it_base, k);
         }
     }
-    dh::launch_advance(e->s, e->it_base, nb);
+    dh::launch_advance(e->s, e->it_base, nb, e->st, 2 * e->M, e->h_st);
 }
 
 int ensure_graph(dhara_ensemble* e, bool two_d, int lg)
@@ -322,7 +322,7 @@ int krylov_solve(dhara_ensemble* e, bool two_d, const std::vector<int>& on, int 
         EHIP(e, hipGetLastError());
     }
     if (!two_d && e->line) {   // z = T^-1 r of the fresh residual
-        const MapRef l = use_map(e, e->cml);
+        const MapRef l = use_map(e->cml);
         dh::launch_batched_line(e->s, e->mixed, true, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
         EHIP(e, hipGetLastError());
     }
@@ -342,7 +342,7 @@ int krylov_solve(dhara_ensemble* e, bool two_d, const std::vector<int>& on, int 
         }
         EHIP(e, hipGetLastError());
         launched += 1 << lg;
-        int rc = read_states(e);
+        int rc = wait(e);
         if (rc) return rc;
         bool all = true;
         int most = 0;
@@ -522,7 +522,7 @@ int mixed_line_solve(dhara_ensemble* e, const std::vector<int>& on, std::vector<
     if ((rc = upload_k3(e)) || (rc = set_active(e, solving))) return rc;
     EHIP(e, hipMemsetAsync(e->it_base, 0, sizeof(int), e->s));   // outside any captured graph
     {   // z = T^-1 r of the assembly's residual
-        const MapRef l = use_map(e, e->cml);
+        const MapRef l = use_map(e->cml);
         dh::launch_batched_line(e->s, true, true, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
     }
     EHIP(e, hipGetLastError());
@@ -541,7 +541,7 @@ int mixed_line_solve(dhara_ensemble* e, const std::vector<int>& on, std::vector<
         }
         EHIP(e, hipGetLastError());
         launched += 1 << lg;
-        if ((rc = read_states(e))) return rc;
+        if ((rc = wait(e))) return rc;
         std::vector<int> restart(M, 0), next(M, 0);
         bool any_next = false, any_restart = false;
         int most = 0;
@@ -588,10 +588,10 @@ int mixed_line_solve(dhara_ensemble* e, const std::vector<int>& on, std::vector<
             }
             if ((rc = upload_k3(e)) || (rc = upload_args(e, e->a_ref, e->h_ref)) || (rc = set_active(e, restart)))
                 return rc;
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched(e->s, dh::BK_REFINE_ADD, e->a_ref, r.map, r.n, e->active);
             dh::launch_batched(e->s, dh::BK_REFINE_RES, e->a_ref, r.map, r.n, e->active);
-            const MapRef l = use_map(e, e->cml);
+            const MapRef l = use_map(e->cml);
             dh::launch_batched_line(e->s, true, true, e->line_nz, e->a_k3, l.map, l.n, e->active, e->it_base, 0);
             EHIP(e, hipGetLastError());
             // a restarted segment is as long as the refinement segments before it
@@ -624,7 +624,7 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
     for (int m = 0; m < M; ++m) surf[m] = e->mem[m]->p.top_bc == DHARA_TOP_SURFACE;
     if ((rc = upload_args(e, e->a_surf, e->h_surf)) || (rc = set_active(e, surf))) return rc;
     {
-        const MapRef r = use_map(e, e->cm2);
+        const MapRef r = use_map(e->cm2);
         dh::launch_batched(e->s, dh::BK_SURF_PRE, e->a_surf, r.map, r.n, e->active);
     }
     for (int m = 0; m < M; ++m) {
@@ -647,7 +647,7 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         }
         if ((rc = upload_args(e, e->a_asm, e->h_asm)) || (rc = set_active(e, pic))) return rc;
         {
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched(e->s, e->mixed ? dh::BK_ASM_MIXED : dh::BK_ASM_F64, e->a_asm, r.map, r.n, e->active);
         }
         if ((rc = build_krylov(e, true))) return rc;
@@ -688,7 +688,7 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
             }
             if ((rc = upload_args(e, e->a_ref, e->h_ref)) || (rc = set_active(e, refine))) return rc;
             {
-                const MapRef r = use_map(e, e->cm3);
+                const MapRef r = use_map(e->cm3);
                 dh::launch_batched(e->s, dh::BK_REFINE_ADD, e->a_ref, r.map, r.n, e->active);
                 dh::launch_batched(e->s, dh::BK_REFINE_RES, e->a_ref, r.map, r.n, e->active);
             }
@@ -714,12 +714,12 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         if ((rc = upload_args(e, e->a_vg, e->h_vg))) return rc;
         if (any(full)) {
             if ((rc = set_active(e, full))) return rc;
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched(e->s, dh::BK_VG_PICARD, e->a_vg, r.map, r.n, e->active);
         }
         if (any(inc_only)) {
             if ((rc = set_active(e, inc_only))) return rc;
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched(e->s, dh::BK_PICARD_INC, e->a_vg, r.map, r.n, e->active);
         }
         if ((rc = reduce(e, false, 2, true))) return rc;
@@ -751,7 +751,7 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         for (int m = 0; m < M; ++m) final_vg[m] = inc_only[m] && !accel[m];
         if (any(final_vg)) {
             if ((rc = set_active(e, final_vg))) return rc;
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched(e->s, dh::BK_VG, e->a_vg, r.map, r.n, e->active);
         }
         if (any(accel)) {   // the Anderson pass: next iterate psi_m and theta, K, C at it
@@ -763,21 +763,21 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
                 ++c->aa_count;
             }
             if ((rc = upload_args(e, e->a_aa, e->h_aa)) || (rc = set_active(e, accel))) return rc;
-            const MapRef r = use_map(e, e->cmaa);
+            const MapRef r = use_map(e->cmaa);
             dh::launch_batched_aa(e->s, e->aa_depth, e->a_aa, r.map, r.n, e->active);
             EHIP(e, hipGetLastError());
         }
         if (any(relax)) {   // theta, K, C at the relaxed iterate psi_m
             for (int m = 0; m < M; ++m) e->h_vg[m] = vg_args(e->mem[m], e->mem[m]->psi_m, e->mem[m]->theta_m);
             if ((rc = upload_args(e, e->a_vg, e->h_vg)) || (rc = set_active(e, relax))) return rc;
-            const MapRef r = use_map(e, e->cm3);
+            const MapRef r = use_map(e->cm3);
             dh::launch_batched(e->s, dh::BK_VG, e->a_vg, r.map, r.n, e->active);
         }
     }
     // ponding update and end of step for every member
     if ((rc = set_active(e, surf))) return rc;
     {
-        const MapRef r = use_map(e, e->cm2);
+        const MapRef r = use_map(e->cm2);
         dh::launch_batched(e->s, dh::BK_SURF_POST, e->a_surf, r.map, r.n, e->active);
     }
     for (int m = 0; m < M; ++m) {
@@ -806,7 +806,7 @@ int subsurface_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
     }
     if ((rc = upload_args(e, e->a_end, e->h_end)) || (rc = set_active(e, all))) return rc;
     {
-        const MapRef r = use_map(e, e->cm3);
+        const MapRef r = use_map(e->cm3);
         dh::launch_batched(e->s, dh::BK_END, e->a_end, r.map, r.n, e->active);
     }
     if ((rc = reduce(e, false, 9, false))) return rc;
@@ -875,19 +875,21 @@ int overland_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
     if ((any_jac && ((rc = upload_args(e, e->a_ocg, e->h_ocg)) || (rc = upload_args(e, e->olf_jac, jac)))) ||
         (any_mg && ((rc = upload_args(e, e->a_omg, e->h_omg)) || (rc = upload_args(e, e->olf_mgm, mgm)))))
         return rc;
-    const MapRef r2 = use_map(e, e->cm2);
+    const MapRef r2 = use_map(e->cm2);
     dh::launch_batched(e->s, dh::BK_OLF_FACES, e->a_olf, r2.map, r2.n, e->active);
     dh::launch_batched(e->s, dh::BK_OLF_ASM, e->a_olf, r2.map, r2.n, e->active);
     if (any_mg) dh::launch_batched_olf_mgcg_block(e->s, e->a_omg, M, e->olf_mgm);
     if (any_jac) dh::launch_batched_olf_cg_block(e->s, e->a_ocg, M, e->olf_jac);
     EHIP(e, hipGetLastError());
-    // the lockstep solve reads every member's state after its batches; without it, read them here
+    // the lockstep solve leaves every member's state on the host; without it, they are sent here
     if (any_lock) {
         if ((rc = set_active(e, lock)) || (rc = krylov_solve(e, true, lock, e->mem[0]->p.olf_maxiter, 2)) ||
             (rc = set_active(e, on)))
             return rc;
-    } else if ((rc = read_states(e))) {
-        return rc;
+    } else {
+        dh::launch_advance(e->s, e->it_base, 0, e->st, 2 * M, e->h_st);
+        EHIP(e, hipGetLastError());
+        if ((rc = wait(e))) return rc;
     }
     for (int m = 0; m < M; ++m) {
         if (!on[m]) continue;
@@ -896,7 +898,7 @@ int overland_step(dhara_ensemble* e, std::vector<dhara_step_stats>& st)
         if (e->h_st[M + m].nan) st[m].nan_seen = 1;
     }
     {
-        const MapRef r = use_map(e, e->cm2);
+        const MapRef r = use_map(e->cm2);
         dh::launch_batched(e->s, dh::BK_OLF_POST, e->a_olf, r.map, r.n, e->active);
     }
     if ((rc = reduce(e, true, 2, false))) return rc;
@@ -988,7 +990,7 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
     if ((rc = ealloc(e, &e->map3, m3.size())) || (rc = ealloc(e, &e->map2, m2.size())) ||
         (rc = ealloc(e, &e->active, n)) || (rc = ealloc(e, &e->it_base, 1)) || (rc = ealloc(e, &e->st, 2 * n)) ||
         (rc = ealloc(e, &e->parts, n)) || (rc = ealloc(e, &e->np3, n)) || (rc = ealloc(e, &e->np2, n)) ||
-        (rc = ealloc(e, &e->red, (size_t)n * dh::kMaxSums)) || (rc = ealloc(e, &e->a_vg, n)) ||
+        (rc = ealloc(e, &e->a_vg, n)) ||
         (rc = ealloc(e, &e->a_surf, n)) || (rc = ealloc(e, &e->a_asm, n)) || (rc = ealloc(e, &e->a_ref, n)) ||
         (rc = ealloc(e, &e->a_end, n)) || (rc = ealloc(e, &e->a_olf, n)) || (rc = ealloc(e, &e->a_k2, n)) ||
         (rc = ealloc(e, &e->a_ocg, n)) || (rc = ealloc(e, &e->a_omg, n)) || (rc = ealloc(e, &e->olf_jac, n)) ||
@@ -1019,7 +1021,9 @@ int dhara_ensemble_create(int32_t n, dhara_ctx* const* members, dhara_ensemble**
         e->h_aa.resize(n);
     }
     if (rc) { dhara_ensemble_destroy(e); return rc; }
-    if (hipHostMalloc((void**)&e->h_active, n * sizeof(int)) != hipSuccess ||
+    e->stage_size = std::max<size_t>(size_t(1) << 20, (size_t)n * 8192);
+    if (hipHostMalloc((void**)&e->h_flags, (size_t)dhara_ensemble::kFlagSlots * n * sizeof(int)) != hipSuccess ||
+        hipHostMalloc((void**)&e->stage, e->stage_size) != hipSuccess ||
         hipHostMalloc((void**)&e->h_st, 2 * n * sizeof(dh::PcgState)) != hipSuccess ||
         hipHostMalloc((void**)&e->h_red, (size_t)n * dh::kMaxSums * sizeof(double)) != hipSuccess) {
         dhara_ensemble_destroy(e);
@@ -1201,10 +1205,10 @@ int dhara_ensemble_destroy(dhara_ensemble* e)
     if (e->s) (void)hipStreamSynchronize(e->s);
     drop_graphs(e, false);
     for (void* v : e->allocs) (void)hipFree(v);
-    if (e->h_active) (void)hipHostFree(e->h_active);
+    if (e->h_flags) (void)hipHostFree(e->h_flags);
+    if (e->stage) (void)hipHostFree(e->stage);
     if (e->h_st) (void)hipHostFree(e->h_st);
     if (e->h_red) (void)hipHostFree(e->h_red);
-    for (int* h : e->pinned) (void)hipHostFree(h);
     if (e->s) (void)hipStreamDestroy(e->s);
     delete e;
     return DHARA_OK;

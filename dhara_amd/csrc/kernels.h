@@ -498,10 +498,20 @@ void launch_batched_spmv2(hipStream_t s, const void* kargs, const BlkMap* map, i
                           const int* it_base, int k);
 void launch_batched_update2(hipStream_t s, const void* kargs, const BlkMap* map, int nblocks, const int* active,
                             const int* it_base, int k);
-void launch_advance(hipStream_t s, int* it_base, int by);
-// out[0 .. total) = the blocks of the nseg segments seg[3j] (start in full), seg[3j+1] (count),
-// seg[3j+2] (offset in out, increasing), i.e. a block map restricted to some members.
-void launch_compact_map(hipStream_t s, const BlkMap* full, const int* seg, int nseg, int total, BlkMap* out);
+// *it_base += by, and the nst solver states to out (pinned host memory).
+void launch_advance(hipStream_t s, int* it_base, int by, const PcgState* st, int nst, PcgState* out);
+// active[m] = flags[m] (pinned host memory) of M models, and for each of n block maps cur = the blocks
+// full[start[m] .. start[m] + count[m]) of the models whose flag is set, in the models' order.
+struct ActMap {
+    const BlkMap* full;
+    const int *start, *count;
+    BlkMap* cur;
+};
+struct ActMaps {
+    ActMap m[4];
+    int n;
+};
+void launch_activate(hipStream_t s, const int* flags, int M, int* active, const ActMaps& maps);
 // out[m*nv + v] = sum (or max) of row v of model m's partials part[m] (nparts[m] entries),
 // in block order; one block per model.
 void launch_reduce_models(hipStream_t s, int nmodels, const double* const* part, const int* nparts, int nv,

@@ -2103,9 +2103,48 @@ __global__ __launch_bounds__(kBlock) void kb_update2(const KrylovArgs<double>* _
     b_pcg_update<double>(a.g2.n, a.x, a.res, a.D, a.p[(sc.it + 1) & 1], a.q, sc, Blk{e.id, e.n});
 }
 
-__global__ void k_advance(int* it_base, int by)
+__global__ __launch_bounds__(kBlock) void k_advance(int* it_base, int by, const int* __restrict__ st, int words,
+                                                    int* __restrict__ out)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *it_base += by;
+    if (threadIdx.x == 0) *it_base += by;
+    for (int i = threadIdx.x; i < words; i += kBlock) out[i] = st[i];
+}
+
+// One launch when the set of active models changes, in place of a copy of the flags, a wait for it
+// and per map a copy of its segments and a compaction (about 3 us each and the gaps between them).
+// Every block reads all flags (a few lines over the bus) and takes the models m = blockIdx.x mod
+// gridDim.x; a model's place in a map is the sum of the counts before it.
+__global__ __launch_bounds__(kBlock) void k_activate(const int* __restrict__ flags, int M, int* __restrict__ active,
+                                                     ActMaps maps)
+{
+    __shared__ int sum[kBlock];
+    int base[4] = {};
+    for (int c0 = 0; c0 < M; c0 += kBlock) {
+        const int t = threadIdx.x, m = c0 + t, n = min(M - c0, kBlock);
+        const int on = m < M ? flags[m] : 0;
+        if (blockIdx.x == 0 && m < M) active[m] = on;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q >= maps.n) break;
+            const ActMap& a = maps.m[q];
+            const int cnt = on ? a.count[m] : 0;
+            int v = cnt;
+            __syncthreads();
+            sum[t] = v;
+            __syncthreads();
+            for (int d = 1; d < n; d <<= 1) {   // inclusive sums
+                const int w = t >= d ? sum[t - d] : 0;
+                __syncthreads();
+                sum[t] = v += w;
+                __syncthreads();
+            }
+            for (int j = (int)((blockIdx.x + gridDim.x - c0 % gridDim.x) % gridDim.x); j < n; j += gridDim.x) {
+                const int before = j ? sum[j - 1] : 0, len = sum[j] - before, from = len ? a.start[c0 + j] : 0;
+                for (int i = t; i < len; i += kBlock) a.cur[base[q] + before + i] = a.full[from + i];
+            }
+            base[q] += sum[n - 1];
+        }
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_reduce_models(const double* const* __restrict__ part,
@@ -3121,29 +3160,16 @@ void launch_batched_cg1(hipStream_t s, bool fp32, const void* args, const BlkMap
                            active, it_base, k);
 }
 
-void launch_advance(hipStream_t s, int* it_base, int by)
+void launch_advance(hipStream_t s, int* it_base, int by, const PcgState* st, int nst, PcgState* out)
 {
-    hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, it_base, by);
+    static_assert(sizeof(PcgState) % sizeof(int) == 0);
+    hipLaunchKernelGGL(k_advance, dim3(1), dim3(kBlock), 0, s, it_base, by, (const int*)st,
+                       nst * (int)(sizeof(PcgState) / sizeof(int)), (int*)out);
 }
 
-__global__ __launch_bounds__(kBlock) void k_compact_map(const BlkMap* __restrict__ full, const int* __restrict__ seg,
-                                                        int nseg, int total, BlkMap* __restrict__ out)
+void launch_activate(hipStream_t s, const int* flags, int M, int* active, const ActMaps& maps)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        int lo = 0, hi = nseg - 1;   // the last segment whose offset is <= i
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (seg[3 * mid + 2] <= i) lo = mid;
-            else hi = mid - 1;
-        }
-        out[i] = full[seg[3 * lo] + (i - seg[3 * lo + 2])];
-    }
-}
-
-void launch_compact_map(hipStream_t s, const BlkMap* full, const int* seg, int nseg, int total, BlkMap* out)
-{
-    const int blocks = std::min((total + kBlock - 1) / kBlock, 1024);
-    hipLaunchKernelGGL(k_compact_map, dim3(blocks), dim3(kBlock), 0, s, full, seg, nseg, total, out);
+    hipLaunchKernelGGL(k_activate, dim3(maps.n ? std::min(M, 128) : 1), dim3(kBlock), 0, s, flags, M, active, maps);
 }
 
 void launch_reduce_models(hipStream_t s, int nmodels, const double* const* part, const int* nparts, int nv,
