@@ -1501,20 +1501,11 @@ int dhara_scatter_group_field(dhara_ctx* c, int32_t f, const double* values, siz
 int dhara_init_state(dhara_ctx* c, int32_t mode)
 {
     if (!c) return DHARA_E_ARG;
-    const dh::Soil soil = soil_of(c);
-    if (mode == DHARA_INIT_FROM_THETA) {
-        dh::launch_vg_inverse(c->s, c->g, soil, c->theta_n, c->psi_n);
-    } else if (mode != DHARA_INIT_FROM_PSI) {
-        return set_err(c, DHARA_E_ARG, "bad init mode");
-    }
-    dh::VgArgs a = vg_args(c, c->psi_n, c->theta_n);
-    dh::launch_vg(c->s, a);
+    if (mode != DHARA_INIT_FROM_THETA && mode != DHARA_INIT_FROM_PSI) return set_err(c, DHARA_E_ARG, "bad init mode");
+    const dh::VgArgs v = vg_args(c, c->psi_n, c->theta_n);
+    dh::launch_init_state(c->s, {c->g, v.soil, c->psi_n, c->psi_m, c->x, c->theta_n, c->theta_m, c->theta_new, v.K, v.C,
+                                 v.K32}, mode == DHARA_INIT_FROM_THETA);
     LAUNCHCHK(c);
-    const size_t nb = (size_t)c->N * sizeof(double);
-    HIPCHK(c, hipMemcpyAsync(c->theta_m, c->theta_n, nb, hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(c, hipMemcpyAsync(c->theta_new, c->theta_n, nb, hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(c, hipMemcpyAsync(c->psi_m, c->psi_n, nb, hipMemcpyDeviceToDevice, c->s));
-    HIPCHK(c, hipMemcpyAsync(c->x, c->psi_n, nb, hipMemcpyDeviceToDevice, c->s));
     HIPCHK(c, hipStreamSynchronize(c->s));
     c->theta_m_current = true;
     c->initialized = true;

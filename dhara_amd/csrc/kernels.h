@@ -303,6 +303,15 @@ void launch_picard_next(hipStream_t s, const NextArgs& a, int depth, const Launc
 // Its first kernel for the rules on psi (ABS_PSI / REL_PSI): the increment of a.psi against a.psi_m
 // into a.part_out
 void launch_picard_inc(hipStream_t s, const VgArgs& a, const Gate& gate);
+// Initial state: psi_n (read, or written from theta_n first), theta_n and the copies theta_m,
+// theta_new, psi_m, x, and K, C (and K32) at psi_n.
+struct InitArgs {
+    Geo g;
+    Soil soil;
+    double *psi_n, *psi_m, *x, *theta_n, *theta_m, *theta_new, *K, *C;
+    float* K32;
+};
+void launch_init_state(hipStream_t s, const InitArgs& a, bool from_theta);
 void launch_vg_inverse(hipStream_t s, const Geo& g, const Soil& soil, const double* theta,
                        double* psi);
 void launch_row_flags(hipStream_t s, const Geo& g, const int* const bctype[6], uint8_t* flags);

@@ -82,6 +82,34 @@ __global__ __launch_bounds__(kBlock) void k_vg(VgArgs a)
     b_vg(a, hw_blk());
 }
 
+// A model's initial state in one launch: psi from theta (FROM_THETA) or as given, theta, K, C at it,
+// and the iteration's copies of both.  12 arrays at most, against an inverse pass, a vG pass and four
+// copies: 231 -> 168 us at 400 x 400 x 30 (bound by the FP64 operations of the two evaluations).
+template <bool FROM_THETA>
+__global__ __launch_bounds__(kBlock) void k_init_state(InitArgs a)
+{
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < a.g.n; c += gridDim.x * blockDim.x) {
+        const double al = cell_alpha(a.soil, c), nv = cell_n(a.soil, c);
+        double psi;
+        if constexpr (FROM_THETA) {
+            psi = vg_inverse(a.theta_n[c], al, nv, a.soil.ts, a.soil.tr);
+            a.psi_n[c] = psi;
+        } else {
+            psi = a.psi_n[c];
+        }
+        double th, K, C;
+        vg_eval(psi, a.soil.Ks[c], al, nv, a.soil.ts, a.soil.tr, th, K, C);
+        a.theta_n[c] = th;
+        a.theta_m[c] = th;
+        a.theta_new[c] = th;
+        a.psi_m[c] = psi;
+        a.x[c] = psi;
+        a.K[c] = K;
+        a.C[c] = C;
+        if (a.K32) a.K32[c] = (float)K;
+    }
+}
+
 // vanGenuchten on psi^{m+1} (src/subsurface.cu:754) fused with GetIterationDifference
 // (432-446), the max reduction (777) and ModifiedPicardUpdate (450-461).
 __device__ __forceinline__ void b_vg_picard(VgArgs a, Blk bk)
@@ -2592,6 +2620,13 @@ static void launch_ev(F kernel, dim3 gr, dim3 bl, hipStream_t s, const LaunchEv&
 void launch_vg(hipStream_t s, const VgArgs& a)
 {
     hipLaunchKernelGGL(k_vg, dim3(grid_for(a.g.n)), dim3(kBlock), 0, s, a);
+}
+
+void launch_init_state(hipStream_t s, const InitArgs& a, bool from_theta)
+{
+    const dim3 gr(grid_for(a.g.n)), bl(kBlock);
+    if (from_theta) hipLaunchKernelGGL(k_init_state<true>, gr, bl, 0, s, a);
+    else hipLaunchKernelGGL(k_init_state<false>, gr, bl, 0, s, a);
 }
 
 void launch_vg_picard(hipStream_t s, const VgArgs& a, const Gate& gate)
