@@ -69,6 +69,43 @@ dh::TileCfg default_tile(const dh::Geo& g)
     while (dh::tile_blocks(g, t) > dh::kMaxBlocks) ++t.kc;
     return t;
 }
+
+// Default tile of the column form's SpMV.  A chunk of planes reads z, p_old and K of a plane on either
+// side of it once more, and fills its pipeline anew, so whole columns are best once their tiles fill
+// the chip: 512-cell tiles from about 400 of them (fewest halo cells; 1024 x 1024 x 30 FP32 172 us,
+// 32 x 8 x 30 210; 450 x 450 x 30 FP64 72, 32 x 8 x 10 84), 64 x 4 below (400 x 400 x 30 FP32, 700 of
+// them: 28 us, 350 of 64 x 8: 30, 32 x 8 x 8: 36).  Fewer tiles than that are split into chunks of at
+// least 4 planes for about 850 blocks (333 x 187 x 24 FP64, 282 tiles: 24 / 12 / 8 / 6 / 4 planes 22.7 /
+// 19.5 / 18.6 / 19.9 / 21.2 us; 100 x 90 x 40 FP32, 46 tiles: 40 / 8 / 4 planes 21.9 / 9.4 / 8.0).
+// Rows that 64 columns would pad by an eighth more than 32 take 32 x 8.
+dh::TileCfg default_zin_tile(const dh::Geo& g)
+{
+    const int nx32 = (g.nx + 31) / 32, nx64 = (g.nx + 63) / 64, ny4 = (g.ny + 3) / 4, ny8 = (g.ny + 7) / 8;
+    const bool narrow = 2 * nx64 * 8 > nx32 * 9;
+    dh::TileCfg t = narrow ? dh::TileCfg{32, 8, g.nz} : dh::TileCfg{64, 8, g.nz};
+    int nt = narrow ? nx32 * ny8 : nx64 * ny8;
+    if (!narrow && nt < 400) {
+        t.ty = 4;
+        nt = nx64 * ny4;
+    }
+    if (nx32 * ny8 > dh::kMaxBlocks) return dh::TileCfg{0, 0, 0};   // as the other kernels' default
+    const int nkz = std::max(1, (850 + nt / 2) / nt);
+    t.kc = std::min(g.nz, std::max(4, (g.nz + nkz - 1) / nkz));
+    return t;
+}
+
+// Default tile of the one-kernel PCG's start-up, for about 1300 blocks: at 400 x 400 x 30 in FP64 650 /
+// 1300 / 1950 / 2600 blocks of 32 x 8 took 55 / 44 / 45 / 62 us (chunks as above).
+dh::TileCfg default_start_tile(const dh::Geo& g)
+{
+    dh::TileCfg t = default_tile(g);
+    if (!t.tx) return t;
+    const int nt = ((g.nx + 31) / 32) * ((g.ny + 7) / 8), nkz = std::max(1, std::min(g.nz, (1300 + nt / 2) / nt));
+    t.kc = (g.nz + nkz - 1) / nkz;
+    return t;
+}
+
+void use_tile(dhara_ctx* c, int e, const dh::TileCfg& t) { c->tile[e] = c->zin_tile[e] = c->start_tile[e] = t; }
 }
 
 namespace dhc {
@@ -531,9 +568,9 @@ int solve_fp64_cg1(dhara_ctx* c, dhara_step_stats* st)
         dh::SolveCtl k = sc;   // reads the assembly partials in part[0]
         k.nparts = aparts;
         k.part_out = c->part[1];
-        dh::launch_cg1_init_f64(c->s, c->g, c->tile[0], c->K, c->D, rb[0], pb[1], k);
+        dh::launch_cg1_init_f64(c->s, c->g, c->start_tile[0], c->K, c->D, rb[0], pb[1], k);
     }
-    const int init_parts = dh::cg1_init_blocks(c->g, c->tile[0]);
+    const int init_parts = dh::cg1_init_blocks(c->g, c->start_tile[0]);
     int rc = run_krylov1(c, c->st_sub, c->p.lin_maxiter, c->pcg_hint(), c->prof, 8.0,
                          [&](int it, const dh::LaunchEv& ev) {
                              dh::SolveCtl k = sc;
@@ -562,7 +599,7 @@ int solve_fp64_line(dhara_ctx* c, dhara_step_stats* st)
     LAUNCHCHK(c);
     double* const pp[2] = {c->pv[0], c->pv[1]};
     dh::SolveCtl sc = solve_ctl(c, c->st_sub, c->p.lin_maxiter, dh::grid_for(c->N), false, true);
-    const dh::TileCfg tc = c->tile[0];
+    const dh::TileCfg tc = c->zin_tile[0];
     const int spmv_parts = tc.tx ? dh::tile_blocks(c->g, tc) : dh::grid_for(c->N);
     const int lparts = dh::line_blocks(c->g);
     {
@@ -640,7 +677,7 @@ int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
     ra.part_out = c->part[0];
     ra.st = c->st_sub;
     const int maxit = c->p.inner_maxiter;
-    const dh::TileCfg tc = c->tile[1];
+    const dh::TileCfg tc = c->zin_tile[1];
     const int spmv_parts = tc.tx ? dh::tile_blocks(c->g, tc) : dh::grid_for(c->N);
     const int lparts = dh::line_blocks(c->g);
     dh::SolveCtl sc = solve_ctl(c, c->st_sub, maxit, dh::grid_for(c->N), true, true);
@@ -828,7 +865,7 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
     const int maxit = c->p.inner_maxiter;
     const dh::TileCfg tc = c->cg1_tile[1];
     const int nb = dh::cg1_blocks(c->g, tc);
-    const int init_parts = dh::cg1_init_blocks(c->g, c->tile[1]);
+    const int init_parts = dh::cg1_init_blocks(c->g, c->start_tile[1]);
     dh::SolveCtl sc = solve_ctl(c, c->st_sub, maxit, dh::grid_for(c->N), true, true);
     int it = 0, updates = 0, refine_parts = aparts;
     bool outer_conv = false;
@@ -840,7 +877,7 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
             k.segment_start = it > 0 ? 1 : 0;
             k.nparts = refine_parts;
             k.part_out = c->part[1];
-            dh::launch_cg1_init_f32(c->s, c->g, c->tile[1], c->K32, c->D32, rb[it & 1], pb[(it + 1) & 1], k);
+            dh::launch_cg1_init_f32(c->s, c->g, c->start_tile[1], c->K32, c->D32, rb[it & 1], pb[(it + 1) & 1], k);
         }
         const int seg = it;
         // after as many updates as the last solve took, this segment's start-up is likely to pass the
@@ -883,7 +920,7 @@ int solve_mixed_cg1(dhara_ctx* c, dhara_step_stats* st)
             k.first_sweep = 0;
             k.nparts = refine_parts;
             k.part_out = c->part[1];
-            dh::launch_cg1_init_f32(c->s, c->g, c->tile[1], c->K32, c->D32, rb[it_end & 1], pb[(it_end + 1) & 1],
+            dh::launch_cg1_init_f32(c->s, c->g, c->start_tile[1], c->K32, c->D32, rb[it_end & 1], pb[(it_end + 1) & 1],
                                     k);
             LAUNCHCHK(c);
             if ((rc = read_state(c, c->st_sub))) return rc;
@@ -1279,11 +1316,13 @@ int dhara_create(const dhara_grid* grid, const dhara_params* params, dhara_ctx**
     g2.cy = params->dt / (grid->dy * grid->dy);
     for (int e = 0; e < 2; ++e) {
         c->tile[e] = default_tile(g);
+        c->zin_tile[e] = default_zin_tile(g);
+        c->start_tile[e] = default_start_tile(g);
         c->cg1_tile[e] = dh::TileCfg{32, 8, dh::cg1_default_planes(g), 0};
         if (dh::cg1_blocks(g, c->cg1_tile[e]) > dh::kMaxBlocks) c->cg1_tile[e].grid = dh::kMaxBlocks;   // blocks loop
         const int tkind = (e == 0 && mixed_column(params)) ? 2 : 0;
         for (const TuneEntry& te : g_tune_table) {
-            if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, tkind}) c->tile[e] = te.cfg;
+            if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, tkind}) use_tile(c, e, te.cfg);
             if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, 1}) {
                 c->cg1_tile[e] = te.cfg;
                 c->cg1_set[e] = true;
@@ -1569,7 +1608,7 @@ int dhara_set_tile(dhara_ctx* c, int32_t elem_bytes, int32_t tx, int32_t ty, int
         if (!dh::tile_supported(t)) return set_err(c, DHARA_E_ARG, "unsupported tile shape");
         if (dh::tile_blocks(c->g, t) > dh::kMaxBlocks) return set_err(c, DHARA_E_ARG, "tile grid too large; raise kc");
     }
-    c->tile[elem_bytes == 8 ? 0 : 1] = t;
+    use_tile(c, elem_bytes == 8 ? 0 : 1, t);
     return DHARA_OK;
 }
 
@@ -1599,7 +1638,10 @@ int dhara_get_krylov_tile(const dhara_ctx* c, int32_t elem_bytes, int32_t* tx, i
 int dhara_get_tile(const dhara_ctx* c, int32_t elem_bytes, int32_t* tx, int32_t* ty, int32_t* kc)
 {
     if (!c || (elem_bytes != 8 && elem_bytes != 4) || !tx || !ty || !kc) return DHARA_E_ARG;
-    const dh::TileCfg& t = c->tile[elem_bytes == 8 ? 0 : 1];
+    // the SpMV's in the column form (in mixed precision the FP64 tile is the assembly's)
+    const int e = elem_bytes == 8 ? 0 : 1;
+    const bool zin = c->p.precond == DHARA_PRECOND_COLUMN && !(e == 0 && mixed_column(&c->p));
+    const dh::TileCfg& t = zin ? c->zin_tile[e] : c->tile[e];
     *tx = t.tx;
     *ty = t.ty;
     *kc = t.kc;
@@ -1712,7 +1754,7 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
                 if ((rc = consider(t))) return rc;
             }
         if ((rc = consider(dh::TileCfg{0, 0, 0}))) return rc;
-        c->tile[e] = best_cfg;
+        use_tile(c, e, best_cfg);
         best[e] = best_t;
         remember_tile(TuneKey{c->g.nx, c->g.ny, c->g.nz, e == 0 ? 8 : 4, (e == 0 && asm_tune) ? 2 : 0}, best_cfg);
     }

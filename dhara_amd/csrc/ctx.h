@@ -85,8 +85,11 @@ struct dhara_ctx {
     dhara_ctx() { std::fill(pcg_hints, pcg_hints + kHints, 8); }
     int& pcg_hint() { return pcg_hints[std::min(picard_it, kHints - 1)]; }
     std::vector<void*> allocs;
-    // SpMV tile shapes: [0] FP64 solves, [1] FP32 inner solves (tx = 0: untiled kernel)
-    dh::TileCfg tile[2] = {{32, 8, 0}, {32, 8, 0}};
+    // Tile shapes: [0] FP64, [1] FP32 (tx = 0: untiled kernels).  A tile that the caller or the autotuner
+    // chose is all three; the defaults differ.
+    dh::TileCfg tile[2] = {{32, 8, 0}, {32, 8, 0}};         // assembly, refinement, two-kernel SpMV
+    dh::TileCfg zin_tile[2] = {{32, 8, 0}, {32, 8, 0}};     // SpMV of the column form
+    dh::TileCfg start_tile[2] = {{32, 8, 0}, {32, 8, 0}};   // start-up of the one-kernel PCG
     // one-kernel PCG tiles: [0] FP64, [1] FP32; cg1_set: chosen by the caller or the autotuner
     dh::TileCfg cg1_tile[2] = {{32, 8, 0, 0}, {32, 8, 0, 0}};
     bool cg1_set[2] = {false, false};

@@ -1029,6 +1029,22 @@ __device__ __forceinline__ double jac_inv(double d)
 // 55 -> 48 us, 1024 x 1024 x 30 232 -> 223 us, 400 x 400 x 30 34.6 -> 36.7 us (1.2 rounds of resident
 // blocks), 800 x 800 x 12 49 -> 52 us; start-up FP64 333 x 187 x 24 24 -> 17 us; 20 models of
 // 32..128 x 32..128 x 10..40 in FP64, all iterating: 95 us in three launches -> 50 us in one.
+// A copy of a slot's value in a register of its own.  A loop that keeps the loads of the next planes in
+// flight reuses the slot's registers for the next load; a value that is still needed then must not
+// share them, or the new load goes elsewhere and a move at the end of the loop waits for it.
+__device__ __forceinline__ float take(float v)
+{
+    float r;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+__device__ __forceinline__ double take(double v)
+{
+    double r;
+    asm volatile("v_mov_b64 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
 template <typename T>
 struct LinePlane {
     T r, q, p, x, K, D;
@@ -1190,9 +1206,12 @@ __global__ __launch_bounds__(kBlock) void k_line(Geo g, const T* __restrict__ K,
 
 // SpMV kernel of the column-preconditioned PCG: p = z + beta p_old, q = A p, partial (p, q), on a
 // TX x TY tile of columns marching through kc planes with the p / K planes staged in LDS (one-cell
-// halo, double buffered, one barrier per plane).  Loads run ahead of their use so that a plane
-// does not wait for memory: the own column's raw z, p_old, K, D two planes ahead and the halo's
-// raw z, p_old, K one plane ahead are in flight while the current plane is computed.
+// halo, double buffered, one barrier per plane).  The loads of A planes, own column and halo, are in
+// flight in register slots that an unrolled loop goes round, without branches (a plane or halo that is
+// not there repeats a valid load); with slots moved down by one per plane the moves waited for the
+// fresh loads.  In the first iteration p_old is not read (z in its place, from cache).  At the same
+// tile this gave 38.9 -> 36.4 us at 400 x 400 x 30 and 211 -> 204 at 1024 x 1024 x 30 in FP32 (the halo's
+// requests bound it there), with the tiles of default_zin_tile 28 and 172 us (21 and 140 at copy rate).
 template <typename T, int TX, int TY>
 __global__ __launch_bounds__(TX * TY) void k_spmv_z(Geo g, const T* __restrict__ K, const T* __restrict__ D,
                                                     const T* __restrict__ z, const T* __restrict__ pold,
@@ -1222,65 +1241,53 @@ __global__ __launch_bounds__(TX * TY) void k_spmv_z(Geo g, const T* __restrict__
     else if (lid < 2 * TX + 2 * TY) { hx = TX; hy = lid - 2 * TX - TY; }
     const int hi = bx * TX + hx, hj = by * TY + hy;
     const bool has_halo = hx > -2 && hi >= 0 && hi < g.nx && hj >= 0 && hj < g.ny;
-    const int hcol = hj * g.nx + hi;
     const int nxy = g.nxy, nz = g.nz;
     const T wx = (T)g.wx, wy = (T)g.wy, wz = (T)g.wz, half = T(0.5);
     auto pv = [&](T zv, T pov) -> T { return first ? zv : zv + beta * pov; };
+    // the columns that a thread loads from: its own, and its halo's (any valid one without)
+    const int ccol = min(j, g.ny - 1) * g.nx + min(i, g.nx - 1);
+    const int hcol = has_halo ? hj * g.nx + hi : by * TY * g.nx + bx * TX;
+    const T* po = first ? z : pold;   // (z again: in cache, p_old is not used)
 
-    T pm = T(0), km = T(0), pc = T(0), kcur = T(0), dc = T(1), pn = T(0), kn = T(0), dn = T(1);
-    T z2 = T(0), p2 = T(0), k2 = T(0), d2 = T(1);
-    T hzc = T(0), hpc = T(0), hkc = T(0);
-    if (in) {
-        if (k0 > 0) {
-            const int c = (k0 - 1) * nxy + col;
-            pm = pv(z[c], pold[c]);
-            km = K[c];
-        }
-        if (k0 < k1) {
-            const int c = k0 * nxy + col;
-            pc = pv(z[c], pold[c]);
-            kcur = K[c];
-            dc = D[c];
-        }
-        if (k0 + 1 < nz) {
-            const int c = (k0 + 1) * nxy + col;
-            pn = pv(z[c], pold[c]);
-            kn = K[c];
-            dn = D[c];
-        }
-        if (k0 + 2 < nz) {
-            const int c = (k0 + 2) * nxy + col;
-            z2 = z[c]; p2 = pold[c]; k2 = K[c]; d2 = D[c];
-        }
+    constexpr int A = sizeof(T) == 4 ? 4 : 2;
+    struct Own { T z, p, K, D; } own[A];   // planes k + 1 .. k + A at step k
+    struct Halo { T z, p, K; } halo[A];    // planes k .. k + A - 1
+    const int lo = min(k1, nz - 1);        // last plane of the own column that is used
+    int fo = k0 + 1, fh = k0;              // next planes to load
+    auto fetch_own = [&](Own& o) {
+        const int c = min(fo, lo) * nxy + ccol;
+        ++fo;
+        o.z = z[c]; o.p = po[c]; o.K = K[c]; o.D = D[c];
+    };
+    auto fetch_halo = [&](Halo& h) {
+        const int c = min(fh, k1 - 1) * nxy + hcol;
+        ++fh;
+        h.z = z[c]; h.p = po[c]; h.K = K[c];
+    };
+    const int cm = max(k0 - 1, 0) * nxy + ccol, c0 = k0 * nxy + ccol;
+    const T zm = z[cm], zc = z[c0], qm = po[cm], qc = po[c0];
+    T km = K[cm], kcur = K[c0], dc = D[c0];
+#pragma unroll
+    for (int u = 0; u < A; ++u) {
+        fetch_halo(halo[u]);
+        fetch_own(own[u]);
     }
-    // the halo runs two planes ahead of its use too (one plane left the halo threads' loads
-    // exposed at every plane's barrier)
-    T hzn = T(0), hpn = T(0), hkn = T(0);
-    if (has_halo && k0 < k1) {
-        const int c = k0 * nxy + hcol;
-        hzc = z[c]; hpc = pold[c]; hkc = K[c];
-        if (k0 + 1 < k1) {
-            hzn = z[c + nxy]; hpn = pold[c + nxy]; hkn = K[c + nxy];
-        }
-    }
+    T pm = pv(zm, qm), pc = pv(zc, qc);
     double acc = 0.0;
-    for (int k = k0; k < k1; ++k) {
-        T z3 = T(0), p3 = T(0), k3 = T(0), d3 = T(1);
-        if (in && k + 3 < nz) {
-            const int c = (k + 3) * nxy + col;
-            z3 = z[c]; p3 = pold[c]; k3 = K[c]; d3 = D[c];
-        }
-        T hz2 = T(0), hp2 = T(0), hk2 = T(0);
-        if (has_halo && k + 2 < k1) {
-            const int c = (k + 2) * nxy + hcol;
-            hz2 = z[c]; hp2 = pold[c]; hk2 = K[c];
-        }
+    auto plane = [&](int k, Own& o, Halo& h, bool fetch) {
         const int buf = k & 1;
         sp[buf][ty + 1][tx + 1] = pc;
         sk[buf][ty + 1][tx + 1] = kcur;
         if (has_halo) {
-            sp[buf][hy + 1][hx + 1] = pv(hzc, hpc);
-            sk[buf][hy + 1][hx + 1] = hkc;
+            sp[buf][hy + 1][hx + 1] = pv(h.z, h.p);
+            sk[buf][hy + 1][hx + 1] = h.K;
+        }
+        T pn = pv(o.z, o.p);
+        asm volatile("" : "+v"(pn));   // computed here, not where it is used
+        const T kn = take(o.K), dn = take(o.D);
+        if (fetch) {
+            fetch_halo(h);
+            fetch_own(o);
         }
         __syncthreads();
         if (in) {
@@ -1298,11 +1305,18 @@ __global__ __launch_bounds__(TX * TY) void k_spmv_z(Geo g, const T* __restrict__
         }
         pm = pc; km = kcur;
         pc = pn; kcur = kn; dc = dn;
-        pn = pv(z2, p2); kn = k2; dn = d2;
-        z2 = z3; p2 = p3; k2 = k3; d2 = d3;
-        hzc = hzn; hpc = hpn; hkc = hkn;
-        hzn = hz2; hpn = hp2; hkn = hk2;
+    };
+    int k = k0;
+    for (; k + A <= k1; k += A) {
+#pragma unroll
+        for (int u = 0; u < A; ++u) {
+            plane(k + u, own[u], halo[u], true);
+            __builtin_amdgcn_sched_barrier(0);   // keeps the loads of a plane behind the uses of its slot
+        }
     }
+#pragma unroll
+    for (int u = 0; u < A; ++u)
+        if (k + u < k1) plane(k + u, own[u], halo[u], false);
     double v[1] = {acc};
     block_partials<1, false>(v, sc.part_out);
 }
