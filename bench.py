@@ -487,12 +487,12 @@ def main():
             kern.append((pr[f"{key}_ms"], kname, avg, pr[f"{key}_bytes"], nl))
     if pr["aa_launches"]:   # the Anderson Picard pass (FP64; bytes vary with its ring: the mean)
         nl = pr["aa_launches"]
-        kern.append((pr["aa_ms"], "aa_column", pr["aa_ms"] / nl * 1e-3, pr["aa_bytes"] / nl, nl))
+        kern.append((pr["aa_ms"], "picard_next", pr["aa_ms"] / nl * 1e-3, pr["aa_bytes"] / nl, nl))
     if kern:
         kern.sort(reverse=True)
         tot, kname, avg, byts, nl = kern[0]
         kprec = "f32" if pr["elem_bytes"] == 4 else "f64"
-        prec = "f64" if kname == "aa_column" else kprec
+        prec = "f64" if kname == "picard_next" else kprec
         # measured HBM bytes per launch (rocprof PMC, copy-calibrated) for the tile in use, if the
         # profile holds that tile
         traffic = None
@@ -506,14 +506,14 @@ def main():
             except Exception:
                 traffic = None
         out["roofline"] = {"bound": "hbm", "kernel": f"k_{kname}<{prec}>",
-                           "tile": None if kname == "aa_column" else r.get("tile"),
+                           "tile": None if kname == "picard_next" else r.get("tile"),
                            "achieved": byts / avg / 1e9,
                            "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": byts / avg / HBM_PEAK,
                            "traffic": traffic, "avg_us": avg * 1e6, "launches": nl,
                            "bytes_per_launch": byts}
         out["roofline"]["total_ms"] = tot
         out["roofline_other_kernels"] = [
-            {"kernel": f"k_{k[1]}<{'f64' if k[1] == 'aa_column' else kprec}>", "achieved": k[3] / k[2] / 1e9,
+            {"kernel": f"k_{k[1]}<{'f64' if k[1] == 'picard_next' else kprec}>", "achieved": k[3] / k[2] / 1e9,
              "frac": k[3] / k[2] / HBM_PEAK, "avg_us": k[2] * 1e6, "launches": k[4], "total_ms": k[0]}
             for k in kern[1:]]
     # CPU baseline: oracle on a bounded window, from the GPU FP64 state

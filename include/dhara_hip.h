@@ -70,8 +70,9 @@ extern "C" {
 /* Preconditioner of the overland CG (the reference's CUSP CG had none, src/overland.cu:410),
  * and the form of the solve.  The *_BLOCK forms solve a surface of at most 128 x 128 cells in
  * one workgroup and one launch (the form a batched ensemble uses for such members, so that a
- * member stepped alone can match it bit for bit; for a single model the grid-wide form is
- * faster); larger surfaces take the grid-wide form of the same preconditioner. */
+ * member stepped alone can match it bit for bit; for a single model the other forms are
+ * faster); larger surfaces take the grid-wide form of the same preconditioner.  Multigrid on a single
+ * model's surface of up to about 64 x 64 cells runs on chip in one workgroup, else grid-wide. */
 #define DHARA_OLF_PRECOND_JACOBI       0
 #define DHARA_OLF_PRECOND_MG           1   /* aggregation-multigrid V-cycle (same solution, far
                                               fewer iterations on ponded surfaces)            */
@@ -210,7 +211,7 @@ typedef struct dhara_kernel_profile {
     double  update_bytes;
     int32_t elem_bytes;         /* 8 (FP64) or 4 (FP32 inner solves) of the profiled solves  */
     int32_t reserved;
-    int64_t aa_launches;        /* Anderson Picard passes (k_aa_column) that ran              */
+    int64_t aa_launches;        /* Anderson Picard passes (k_picard_next) that ran            */
     double  aa_ms;              /* summed device time of those passes                         */
     double  aa_bytes;           /* summed algorithmic HBM bytes of those passes                */
 } dhara_kernel_profile;
@@ -298,7 +299,9 @@ int dhara_profile_read(dhara_ctx* ctx, dhara_kernel_profile* out);
 /* ---- tuning ------------------------------------------------------------------------------ */
 /* Tile shape of the LDS-tiled subsurface SpMV kernel for one precision (elem_bytes 8: FP64
  * solves, 4: FP32 inner solves).  tx = 0 selects the untiled one-cell-per-thread kernel.
- * Supported (tx, ty): (32,8) (64,4) (16,16) (32,4) (64,8); kc >= 1 planes per block. */
+ * Supported (tx, ty): (32,8) (64,4) (16,16) (32,4) (64,8); kc >= 1 planes per block.  A tile set here
+ * is also the assembly's (FP64) and the start-up's of the one-kernel PCG; without one, each kernel has
+ * a default of its own, and dhara_get_tile gives the SpMV's. */
 int dhara_set_tile(dhara_ctx* ctx, int32_t elem_bytes, int32_t tx, int32_t ty, int32_t kc);
 int dhara_get_tile(const dhara_ctx* ctx, int32_t elem_bytes, int32_t* tx, int32_t* ty, int32_t* kc);
 /* Tile of the one-kernel PCG (DHARA_KRYLOV_ONE_KERNEL): (tx, ty) in (32,8) (16,16) (32,16)
