@@ -593,7 +593,7 @@ void launch_olf_mgcg_block(hipStream_t s, const OlfMgArgs& a);
 void launch_batched_olf_mgcg_block(hipStream_t s, const OlfMgArgs* args, int nmodels, const int* active);
 
 // The same for surfaces that fit one workgroup's registers and LDS (mg_small: up to 64 x 64 cells and
-// shapes like it), single-reduction form; of h only the levels' sizes are used.
+// shapes like it); of h only the levels' sizes are used.
 bool mg_small(const MgHier& h);
 void launch_olf_mgcg_small(hipStream_t s, const OlfMgArgs& a);
 

@@ -730,9 +730,12 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_mg(int n, MgUpd u)
 // level-0 aggregate -- operator, residual, search direction, solution -- in registers for the whole
 // solve; the coarser levels' operators and right-hand sides and every level's planes are in LDS, so
 // after the first loads an iteration moves nothing but register spills.  The iteration is the
-// single-reduction form of the grid-wide solve: one V-cycle, A z and one block reduction, a chain of
-// ~40 barriers bound by LDS latency: 14 us on 64 x 48, where the grid-wide kernels took three
-// launches (26 us) and the set-up three more.
+// Hestenes-Stiefel one of the other one-workgroup forms, with (p, A p) summed directly: on flat deep
+// pools (face conductances from 1e-2 to 1e12 side by side) the single-reduction form's recurrence for
+// it loses every digit and comes out negative, and in one workgroup a second block reduction costs
+// one barrier, which that form spends on A z.  A chain of ~40 barriers an iteration bound by LDS
+// latency: 226 us a solve of 11 iterations on 64 x 48 cells (single-reduction form: 277), 261 on
+// 64 x 64 (327); the grid-wide kernels take three launches an iteration and three for the set-up.
 constexpr int kMgDeepAggs = 384;       // aggregates of levels 1 .. le - 1 together
 constexpr int kMgSmallPlanes = 7168;   // plane slots of all levels together
 constexpr int kMgOps = 16;             // operator values of a coarser aggregate
@@ -754,7 +757,7 @@ __device__ __forceinline__ void b_olf_mgcg_small(const OlfCgArgs& a, const MgHie
     __shared__ double sx[kMgSmallPlanes], sop[kMgOps * kMgDeepAggs], sb[kMgThreads + kMgDeepAggs];
     __shared__ MgExactLds ex;
     __shared__ MgSmallLevel lev[kMgMaxLevels];
-    __shared__ double red[4 * 16];
+    __shared__ double red[3 * 16], red_pq[16];   // one reduction's barrier frees the other's words
     const Geo2 g2 = a.g;
     const int le = h.le, tid = threadIdx.x;
     if (tid == 0) {
@@ -779,7 +782,7 @@ __device__ __forceinline__ void b_olf_mgcg_small(const OlfCgArgs& a, const MgHie
     for (int c = 0; c < 4; ++c) in.c[c] = in.c[c] && on0;
     const MgPlanes s0{sx + (J0 + 1) * (bx0 + 2) + I0 + 1, bx0 + 2, (bx0 + 2) * (by0 + 2)};
     MgAgg A;
-    double p[4] = {}, s[4] = {}, x[4], bb = 0.0;
+    double p[4] = {}, x[4], bb = 0.0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         A.d[c] = ld_if(in.c[c], a.D, g + off[c], 1.0);
@@ -925,11 +928,6 @@ __device__ __forceinline__ void b_olf_mgcg_small(const OlfCgArgs& a, const MgHie
             __syncthreads();
 #pragma unroll
             for (int c = 0; c < 4; ++c) A.x[c] = in.c[c] ? ex.ye[g + off[c]] : 0.0;
-            if (on0) {
-                put_red(A, s0);
-                s0.put(1, A.x[1]);
-                s0.put(2, A.x[2]);
-            }
             return;
         }
         {
@@ -991,62 +989,69 @@ __device__ __forceinline__ void b_olf_mgcg_small(const OlfCgArgs& a, const MgHie
             if (in.c[0]) A.x[0] += yc;
             if (in.c[3]) A.x[3] += yc;
         }
-        agg_up(A, s0, on0, true);
+        agg_up(A, s0, on0, false);
     };
-    double w[4] = {};
-    double sums[4];
-    auto cycle = [&]() {   // z = A.x = V-cycle(r), w = A z and the sums (r, z), (r, r), (w, z)
+    // z = A.x = V-cycle(r); (r, z), (r, r) and, at the start, (b, b)
+    double sums[3];
+    auto cycle = [&](double bb_c) {
         vcycle();
-        __syncthreads();
-        double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
-        if (on0) {
-            red_sums(A, s0, t0, t3);
-            black_sums(A, s0, t1, t2);
-        }
-        const double t[4] = {t0, t1, t2, t3};
-        sums[0] = sums[1] = sums[2] = 0.0;
+        sums[0] = sums[1] = 0.0;
+        sums[2] = bb_c;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            w[c] = in.c[c] ? A.d[c] * A.x[c] - t[c] : 0.0;
             if (!in.c[c]) continue;
             sums[0] += A.b[c] * A.x[c];
             sums[1] += A.b[c] * A.b[c];
-            sums[2] += w[c] * A.x[c];
         }
+        block_reduce<3, false, false>(sums, red);
     };
-    cycle();
-    sums[3] = bb;
-    block_reduce<4, false>(sums, red);
-    bb = sums[3];
+    cycle(bb);
+    bb = sums[2];
     const double tol2 = a.tol * a.tol * bb;
-    double gam_old = 0.0, pi_old = 0.0;
+    double rz = sums[0], rr = sums[1], beta = 0.0;
     int it = 0, conv = 0, nan = !isfinite(bb);
     for (;;) {
-        const double gam = sums[0], rr = sums[1], del = sums[2];
-        nan |= !isfinite(rr);
+        nan |= !(isfinite(rr) && isfinite(rz));
         conv = (rr <= tol2) ? 1 : 0;
         if (conv || nan || it >= a.maxit) break;
-        const double beta = it == 0 ? 0.0 : gam / gam_old;
-        const double pi = it == 0 ? del : del - beta * beta * pi_old;
-        const double alpha = gam / pi;
-        if (!(pi > 0.0) || !isfinite(alpha) || !isfinite(beta)) {
-            nan = 1;
-            conv = 0;
-            break;
-        }
-        gam_old = gam;
-        pi_old = pi;
+        // p, and A p through the planes (no wave still reads them: the reduction's barrier)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            s[c] = w[c] + beta * s[c];
-            A.b[c] -= alpha * s[c];
             p[c] = A.x[c] + beta * p[c];
-            x[c] += alpha * p[c];
+            A.x[c] = p[c];
         }
+        if (on0) {
+            put_red(A, s0);
+            s0.put(1, p[1]);
+            s0.put(2, p[2]);
+        }
+        __syncthreads();
+        double t[4] = {0.0, 0.0, 0.0, 0.0}, q[4], pq[1] = {0.0};
+        if (on0) {
+            red_sums(A, s0, t[0], t[3]);
+            black_sums(A, s0, t[1], t[2]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            q[c] = in.c[c] ? A.d[c] * p[c] - t[c] : 0.0;
+            pq[0] += p[c] * q[c];
+        }
+        block_reduce<1, false, false>(pq, red_pq);
+        const double alpha = rz / pq[0];
+        if (!(pq[0] != 0.0) || !isfinite(alpha)) {
+            nan = 1;
+            break;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            x[c] += alpha * p[c];
+            A.b[c] -= alpha * q[c];
+        }
+        cycle(0.0);
         ++it;
-        cycle();
-        sums[3] = 0.0;
-        block_reduce<4, false>(sums, red);
+        beta = sums[0] / rz;
+        rz = sums[0];
+        rr = sums[1];
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c)
@@ -1057,7 +1062,7 @@ __device__ __forceinline__ void b_olf_mgcg_small(const OlfCgArgs& a, const MgHie
         st->tol2 = tol2;
         st->iter = it;
         st->conv = conv && !nan;
-        st->rr = sums[1];
+        st->rr = rr;
         st->nan = nan;
         st->outer_conv = conv && !nan;
         st->done = 1;
