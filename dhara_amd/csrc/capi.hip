@@ -1131,61 +1131,56 @@ int do_overland_step(dhara_ctx* c, dhara_step_stats* st)
     double* const pp[2] = {c->p2[0], c->p2[1]};
     dh::SolveCtl sc = solve_ctl(c, c->st_olf, c->p.olf_maxiter, dh::grid_for(c->S), false, true);
     sc.lin_tol = c->p.olf_tol;
-    // a multigrid solve that fits one workgroup's registers and LDS (mg_small): the whole solve in one
-    // launch; the *_BLOCK forms on a surface of at most kOlfBlockCells cells: the ensemble's
-    // one-workgroup solve with the surface in memory (either preconditioner); multigrid on a surface with tiled levels: the
-    // single-reduction CG, one V-cycle per iteration
+    // One launch of one workgroup: a multigrid solve that fits its registers and LDS (mg_small); the
+    // *_BLOCK forms on a surface of at most kOlfBlockCells cells, the ensemble's solve with the surface
+    // in memory (either preconditioner), which also takes what is left without tiled levels: strips of
+    // one or two rows, whose cells are all on the ring.  Else grid-wide: the single-reduction multigrid
+    // CG, one V-cycle per iteration, or Jacobi-CG.
     const bool chip = op == DHARA_OLF_PRECOND_MG && dh::mg_small(c->mg);
-    const bool small = chip || ((op == DHARA_OLF_PRECOND_MG_BLOCK || op == DHARA_OLF_PRECOND_JACOBI_BLOCK) &&
-                                c->S <= dh::kOlfBlockCells);
-    const bool cg1 = mg && !small && dh::mg_coarse_level(c->mg) > 0;
-    if (mg && !small) {
-        // z0 = M^-1 r0; its kernel writes the partials the first CG kernel reads
-        dh::launch_mg_setup(c->s, c->g2, c->ke, c->kn, c->mg);
-        if (cg1) dh::launch_mg_vcycle_cg1_start(c->s, c->mg, c->st_olf, c->part[0], c->b2, c->w2);
-        else dh::launch_mg_vcycle(c->s, c->mg, c->st_olf, c->part[0], c->b2);
-        sc.nparts = dh::mg_partials(c->mg);
-    }
-    LAUNCHCHK(c);
+    const bool block = !chip && c->S <= dh::kOlfBlockCells &&
+                       (op == DHARA_OLF_PRECOND_MG_BLOCK || op == DHARA_OLF_PRECOND_JACOBI_BLOCK ||
+                        (mg && dh::mg_coarse_level(c->mg) == 0));
     int rc;
-    if (small) {   // the whole CG in one workgroup
-        if (chip) dh::launch_olf_mgcg_small(c->s, dh::OlfMgArgs{olf_cg_args(c, c->st_olf), c->mg});
-        else if (mg) dh::launch_olf_mgcg_block(c->s, dh::OlfMgArgs{olf_cg_args(c, c->st_olf), c->mg});
-        else dh::launch_olf_cg_block(c->s, olf_cg_args(c, c->st_olf));
+    if (chip || block) {
+        const dh::OlfCgArgs cg = olf_cg_args(c, c->st_olf);
+        if (chip) dh::launch_olf_mgcg_small(c->s, dh::OlfMgArgs{cg, c->mg});
+        else if (mg) dh::launch_olf_mgcg_block(c->s, dh::OlfMgArgs{cg, c->mg});
+        else dh::launch_olf_cg_block(c->s, cg);
         LAUNCHCHK(c);
         rc = read_state(c, c->st_olf);
+    } else if (mg) {
+        // z0 = M^-1 r0; its last kernel writes the partials the first CG kernel reads
+        dh::launch_mg_setup(c->s, c->g2, c->ke, c->kn, c->mg);
+        dh::launch_mg_vcycle_cg1_start(c->s, c->mg, c->st_olf, c->part[0], c->b2, c->w2);
+        LAUNCHCHK(c);
+        sc.nparts = dh::mg_partials(c->mg);
+        rc = run_krylov1(c, c->st_olf, c->p.olf_maxiter, c->olf_hint, false, 8.0,
+                         [&](int it, const dh::LaunchEv&) {
+                             dh::SolveCtl k = sc;
+                             k.it = it;
+                             double* const rb[2] = {c->r2, c->r2b};
+                             double* const sb[2] = {c->q2, c->s2b};
+                             const dh::MgCg1 v{k, c->H, c->p2[0], c->z2, c->w2, sb[it & 1], sb[(it + 1) & 1],
+                                               rb[it & 1], rb[(it + 1) & 1]};
+                             dh::launch_mg_vcycle_cg1(c->s, c->mg, c->st_olf, c->part[0], v);
+                         },
+                         [] { return false; });
     } else {
-        rc = cg1 ? run_krylov1(c, c->st_olf, c->p.olf_maxiter, c->olf_hint, false, 8.0,
-                                   [&](int it, const dh::LaunchEv&) {
-                                       dh::SolveCtl k = sc;
-                                       k.it = it;
-                                       double* const rb[2] = {c->r2, c->r2b};
-                                       double* const sb[2] = {c->q2, c->s2b};
-                                       const dh::MgCg1 v{k, c->H, c->p2[0], c->z2, c->w2, sb[it & 1], sb[(it + 1) & 1],
-                                                         rb[it & 1], rb[(it + 1) & 1]};
-                                       dh::launch_mg_vcycle_cg1(c->s, c->mg, c->st_olf, c->part[0], v);
-                                   },
-                                   [] { return false; })
-                     : run_krylov(
+        LAUNCHCHK(c);
+        rc = run_krylov(
             c, c->st_olf, c->p.olf_maxiter, c->olf_hint, false, 8.0,
-            [&](int it, const dh::LaunchEv& ev) {
+            [&](int it, const dh::LaunchEv&) {
                 dh::SolveCtl k = sc;
                 k.it = it;
-                dh::launch_pcg2_spmv(c->s, c->g2, c->ke, c->kn, c->D2, c->r2, pp, c->q2, k, mg ? c->z2 : nullptr);
+                dh::launch_pcg2_spmv(c->s, c->g2, c->ke, c->kn, c->D2, c->r2, pp, c->q2, k);
             },
-            [&](int it, const dh::LaunchEv& ev) {
+            [&](int it, const dh::LaunchEv&) {
                 dh::SolveCtl k = sc;
                 k.it = it;
                 k.part_in = c->part[1];
                 k.nparts = dh::grid_for(c->S);
                 k.part_out = c->part[0];
-                if (mg) {   // H += alpha p, r -= alpha q inside the V-cycle's first kernel (r2 / r2b alternate)
-                    double* const rb[2] = {c->r2, c->r2b};
-                    const dh::MgUpd u{k, c->H, pp[(it + 1) & 1], c->q2, rb[it & 1], rb[(it + 1) & 1]};
-                    dh::launch_mg_vcycle_upd(c->s, c->mg, c->st_olf, c->part[0], u);
-                } else {
-                    dh::launch_pcg_update_f64(c->s, c->S, c->H, c->r2, c->D2, pp[(it + 1) & 1], c->q2, k);
-                }
+                dh::launch_pcg_update_f64(c->s, c->S, c->H, c->r2, c->D2, pp[(it + 1) & 1], c->q2, k);
             });
     }
     if (rc) return rc;
@@ -1941,7 +1936,7 @@ int dhara_overland_precond(dhara_ctx* c, const double* r, double* z)
     dh::launch_mg_setup(c->s, c->g2, c->ke, c->kn, c->mg);
     const size_t nb = (size_t)c->S * sizeof(double);
     HIPCHK(c, hipMemcpyAsync(c->r2, r, nb, hipMemcpyHostToDevice, c->s));
-    dh::launch_mg_vcycle(c->s, c->mg, nullptr, nullptr, nullptr);
+    dh::launch_mg_vcycle(c->s, c->mg);
     LAUNCHCHK(c);
     HIPCHK(c, hipMemcpyAsync(z, c->z2, nb, hipMemcpyDeviceToHost, c->s));
     HIPCHK(c, hipStreamSynchronize(c->s));

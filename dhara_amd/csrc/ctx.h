@@ -47,7 +47,7 @@ struct dhara_ctx {
     dh::MgHier mg{};
     bool mg_ready = false;
     double* z2 = nullptr;
-    double* r2b = nullptr;   // second residual buffer: the multigrid-preconditioned CG alternates r2 / r2b
+    double* r2b = nullptr;   // second residual buffer: the single-reduction overland CG alternates r2 / r2b
     double *w2 = nullptr, *s2b = nullptr;   // single-reduction overland CG: A z, second A p buffer (with q2)
     // reductions: partial buffers A (written by assembly/update kernels) and B (SpMV kernels)
     double* part[2] = {nullptr, nullptr};

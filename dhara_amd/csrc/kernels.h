@@ -426,10 +426,8 @@ void launch_cast_f64(hipStream_t s, int n, const float* in, double* out);
 // Overland
 void launch_olf_faces(hipStream_t s, const OlfArgs& a);   // H = h + z and the face conductances
 void launch_olf_assemble(hipStream_t s, const OlfArgs& a);
-// z = NULL: Jacobi (p = r/D + beta p); otherwise p = z + beta p with z the preconditioned residual.
 void launch_pcg2_spmv(hipStream_t s, const Geo2& g, const double* ke, const double* kn,
-                      const double* D, const double* r, double* const p[2], double* q,
-                      const SolveCtl& sc, const double* z = nullptr);
+                      const double* D, const double* r, double* const p[2], double* q, const SolveCtl& sc);
 void launch_olf_post(hipStream_t s, const OlfArgs& a);
 
 // ---- batched launches over an ensemble of models (kernels.hip) ----------------------------
@@ -544,22 +542,10 @@ constexpr int kMgExactCells = 64;   // the V-cycle bottoms out on the first coar
 int mg_exact_level(const MgHier& h);   // that level
 int mg_levels(int nx, int ny, int dims[][2]);   // level sizes down to 1 x 1; returns the count
 int mg_coarse_level(const MgHier& h);           // first level handled by the single-block kernel
-int mg_partials(const MgHier& h);               // partial sums the V-cycle's last kernel writes
+int mg_partials(const MgHier& h);               // blocks of the V-cycle's last kernel (single-reduction form)
 // Level-0 weights from the face conductances and the Galerkin operators of all coarse levels.
 void launch_mg_setup(hipStream_t s, const Geo2& g, const double* ke, const double* kn, const MgHier& h);
-// y_0 = V-cycle(b_0); with `part`, partial sums [(b0, y0), (b0, b0), (bb_src, bb_src), (b0, b0)].
-// Every kernel returns at once when st->done is set (st may be NULL).
-void launch_mg_vcycle(hipStream_t s, const MgHier& h, const PcgState* st, double* part, const double* bb_src);
-// The overland CG's update fused into the V-cycle's first kernel: alpha from the SpMV partials
-// (sc), H += alpha p and r_new = r_old - alpha q (the tile's halo recomputes r_new from r_old
-// and q, so r_old and r_new must be different buffers), then the V-cycle of r_new.
-struct MgUpd {
-    SolveCtl sc;
-    double* x;
-    const double *p, *q, *r_old;
-    double* r_new;
-};
-void launch_mg_vcycle_upd(hipStream_t s, const MgHier& h, const PcgState* st, double* part, const MgUpd& u);
+void launch_mg_vcycle(hipStream_t s, const MgHier& h);   // y_0 = V-cycle(b_0)
 
 // Single-reduction (Chronopoulos-Gear) form of the multigrid-preconditioned overland CG, for
 // surfaces whose V-cycle has tiled levels (mg_coarse_level(h) > 0).  The V-cycle's last kernel

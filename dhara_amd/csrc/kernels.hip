@@ -1869,21 +1869,16 @@ __global__ __launch_bounds__(kBlock) void k_olf_assemble(OlfArgs a)
     b_olf_assemble(a, hw_blk());
 }
 
-// PRECZ: p = z + beta p with z the preconditioned residual (multigrid); else z = r / D.
-template <bool PRECZ>
-__device__ __forceinline__ void b_pcg2_spmv(Geo2 g, const double* __restrict__ ke,
-                                                      const double* __restrict__ kn,
-                                                      const double* __restrict__ D,
-                                                      const double* __restrict__ r,
-                                                      const double* __restrict__ pold,
-                                                      double* __restrict__ pnew, double* __restrict__ q,
-                                                      SolveCtl sc, const double* __restrict__ zp, Blk bk)
+__device__ __forceinline__ void b_pcg2_spmv(Geo2 g, const double* __restrict__ ke, const double* __restrict__ kn,
+                                            const double* __restrict__ D, const double* __restrict__ r,
+                                            const double* __restrict__ pold, double* __restrict__ pnew,
+                                            double* __restrict__ q, SolveCtl sc, Blk bk)
 {
     double beta;
     if (!pcg_begin(sc, beta, bk.id)) return;
     const bool first = (sc.it == 0);
     auto pf = [&](int c) -> double {
-        const double z = PRECZ ? zp[c] : r[c] / D[c];
+        const double z = r[c] / D[c];
         return first ? z : z + beta * pold[c];
     };
     double acc[1] = {0.0};
@@ -1897,16 +1892,12 @@ __device__ __forceinline__ void b_pcg2_spmv(Geo2 g, const double* __restrict__ k
     block_partials<1, false>(acc, sc.part_out, bk.id);
 }
 
-template <bool PRECZ>
 __global__ __launch_bounds__(kBlock) void k_pcg2_spmv(Geo2 g, const double* __restrict__ ke,
-                                                      const double* __restrict__ kn,
-                                                      const double* __restrict__ D,
-                                                      const double* __restrict__ r,
-                                                      const double* __restrict__ pold,
-                                                      double* __restrict__ pnew, double* __restrict__ q,
-                                                      SolveCtl sc, const double* __restrict__ zp)
+                                                      const double* __restrict__ kn, const double* __restrict__ D,
+                                                      const double* __restrict__ r, const double* __restrict__ pold,
+                                                      double* __restrict__ pnew, double* __restrict__ q, SolveCtl sc)
 {
-    b_pcg2_spmv<PRECZ>(g, ke, kn, D, r, pold, pnew, q, sc, zp, hw_blk());
+    b_pcg2_spmv(g, ke, kn, D, r, pold, pnew, q, sc, hw_blk());
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2129,7 +2120,7 @@ __global__ __launch_bounds__(kBlock) void kb_spmv2(const KrylovArgs<double>* __r
     const KrylovArgs<double>& a = args[e.m];
     SolveCtl sc = a.spmv;
     sc.it = *it_base + k;
-    b_pcg2_spmv<false>(a.g2, a.ke, a.kn, a.D, a.r, a.p[sc.it & 1], a.p[(sc.it + 1) & 1], a.q, sc, nullptr,
+    b_pcg2_spmv(a.g2, a.ke, a.kn, a.D, a.r, a.p[sc.it & 1], a.p[(sc.it + 1) & 1], a.q, sc,
                        Blk{e.id, e.n});
 }
 
@@ -3035,14 +3026,10 @@ void launch_olf_assemble(hipStream_t s, const OlfArgs& a)
 }
 
 void launch_pcg2_spmv(hipStream_t s, const Geo2& g, const double* ke, const double* kn,
-                      const double* D, const double* r, double* const p[2], double* q,
-                      const SolveCtl& sc, const double* z)
+                      const double* D, const double* r, double* const p[2], double* q, const SolveCtl& sc)
 {
-    const double* pold = p[sc.it & 1];
-    double* pnew = p[(sc.it + 1) & 1];
-    const dim3 gr(grid_for(g.n)), bl(kBlock);
-    if (z) hipLaunchKernelGGL(k_pcg2_spmv<true>, gr, bl, 0, s, g, ke, kn, D, r, pold, pnew, q, sc, z);
-    else hipLaunchKernelGGL(k_pcg2_spmv<false>, gr, bl, 0, s, g, ke, kn, D, r, pold, pnew, q, sc, z);
+    hipLaunchKernelGGL(k_pcg2_spmv, dim3(grid_for(g.n)), dim3(kBlock), 0, s, g, ke, kn, D, r, p[sc.it & 1],
+                       p[(sc.it + 1) & 1], q, sc);
 }
 
 void launch_olf_cg_block(hipStream_t s, const OlfCgArgs& a)

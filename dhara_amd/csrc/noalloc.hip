@@ -116,7 +116,7 @@ int dhara_overland_precond_noalloc(dhara_ctx* c, const double* r, double* z)
     dh::launch_olf_assemble(c->s, a);
     dh::launch_mg_setup(c->s, c->g2, c->ke, c->kn, h);
     HIPCHK(c, hipMemcpyAsync(c->r2, r, (size_t)c->S * sizeof(double), hipMemcpyDeviceToDevice, c->s));
-    dh::launch_mg_vcycle(c->s, h, nullptr, nullptr, nullptr);
+    dh::launch_mg_vcycle(c->s, h);
     LAUNCHCHK(c);
     HIPCHK(c, hipStreamSynchronize(c->s));
     return DHARA_OK;

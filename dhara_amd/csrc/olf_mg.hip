@@ -584,14 +584,13 @@ __device__ __forceinline__ void mg_exact_solve(const double (&m)[kMgInvRows], co
 }
 
 // The V-cycle from level lc down to le and back, in one block: reads b of level lc, writes y of
-// level lc (and on level 0 the CG partial sums).  A thread owns one aggregate of one of the levels
+// level lc.  A thread owns one aggregate of one of the levels
 // lc .. le - 1 (all operators are loaded at once at the start), so a phase is a barrier and at most
 // one aggregate's update; the residual sum of thread t's aggregate is cell t of the array of the
 // coarser levels' right-hand sides.  A chain of ~36 dependent phases of ~100 ns; with the operators in
 // LDS and the levels' cells dealt anew to the threads in every phase it took 26 us (50 x 50 down to
 // 7 x 7).
-__global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgState* st, double* part,
-                                                          const double* bb_src)
+__global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgState* st)
 {
     // a level of bx x by aggregates takes 4 (bx + 2) (by + 2) slots; a row of n aggregates is the worst
     __shared__ double sx[12 * kMgThreads + 24 * kMgMaxLevels];
@@ -672,26 +671,13 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarse(MgHier h, const PcgSta
         agg_up(a, s, on, true);
         __syncthreads();
     }
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
     if (lc == le) {
-        if (tid < ne) {
-            L.y[tid] = ex.ye[tid];
-            acc[0] = sb[tid] * ex.ye[tid];
-            acc[1] = sb[tid] * sb[tid];
-            if (bb_src) acc[2] = bb_src[tid] * bb_src[tid];
-        }
+        if (tid < ne) L.y[tid] = ex.ye[tid];
     } else if (lv == lc) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (!in.c[c]) continue;
-            L.y[g + off[c]] = a.x[c];
-            acc[0] += a.b[c] * a.x[c];
-            acc[1] += a.b[c] * a.b[c];
-            if (bb_src) acc[2] += bb_src[g + off[c]] * bb_src[g + off[c]];
-        }
+        for (int c = 0; c < 4; ++c)
+            if (in.c[c]) L.y[g + off[c]] = a.x[c];
     }
-    acc[3] = acc[1];
-    if (part) block_partials<4, false>(acc, part);
 }
 
 // The operators of the levels below the first one the single-block kernel handles (and level 0's
@@ -714,17 +700,6 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_setup_coarse(Geo2 g, const do
     mg_store_inverse(m, h.inv, n, n);
 }
 
-// The update of MgUpd as a kernel of its own (surfaces handled entirely by the coarse kernel).
-__global__ __launch_bounds__(kBlock) void k_pcg_update_mg(int n, MgUpd u)
-{
-    double alpha;
-    if (!update_begin(u.sc, alpha, blockIdx.x)) return;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-        u.x[c] = u.x[c] + alpha * u.p[c];
-        u.r_new[c] = u.r_old[c] - alpha * u.q[c];
-    }
-}
-
 // ---- the whole multigrid-preconditioned CG of a small surface in one workgroup, on chip ------
 // Surfaces whose level 0 has at most one aggregate per thread (64 x 64 cells).  A thread keeps its
 // level-0 aggregate -- operator, residual, search direction, solution -- in registers for the whole
@@ -737,7 +712,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_mg(int n, MgUpd u)
 // latency: 226 us a solve of 11 iterations on 64 x 48 cells (single-reduction form: 277), 261 on
 // 64 x 64 (327); the grid-wide kernels take three launches an iteration and three for the set-up.
 constexpr int kMgDeepAggs = 384;       // aggregates of levels 1 .. le - 1 together
-constexpr int kMgSmallPlanes = 7168;   // plane slots of all levels together
+constexpr int kMgSmallPlanes = 10240;  // plane slots of all levels together (a strip of 3 x 712 cells: 9,544)
 constexpr int kMgOps = 16;             // operator values of a coarser aggregate
 struct MgSmallLevel {
     int bx, by, x, op, b;   // aggregates; first plane slot, operator column, right-hand side entry
@@ -1299,11 +1274,7 @@ int mg_exact_level(const MgHier& h)
 
 int mg_coarse_level(const MgHier& h) { return mg_first_single_block(h); }
 
-int mg_partials(const MgHier& h)
-{
-    const int lc = mg_coarse_level(h);
-    return lc == 0 ? 1 : mg_tiles(h.lv[0]);
-}
+int mg_partials(const MgHier& h) { return mg_tiles(h.lv[0]); }
 
 void launch_mg_setup(hipStream_t s, const Geo2& g, const double* ke, const double* kn, const MgHier& h)
 {
@@ -1331,22 +1302,12 @@ static void mg_up0(hipStream_t s, const MgHier& h, int l, const PcgState* st)
                        h.lv[l + 1], h.lv[l].y, st, nullptr, nullptr, nullptr);
 }
 
-void launch_mg_vcycle(hipStream_t s, const MgHier& h, const PcgState* st, double* part, const double* bb_src)
+void launch_mg_vcycle(hipStream_t s, const MgHier& h)
 {
     const int lc = mg_coarse_level(h);
-    for (int l = 0; l < lc; ++l) mg_down0(s, h, l, st);
-    hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, h, st, lc == 0 ? part : nullptr,
-                       lc == 0 ? bb_src : nullptr);
-    for (int l = lc - 1; l >= 0; --l) mg_up0(s, h, l, st);
-}
-
-void launch_mg_vcycle_upd(hipStream_t s, const MgHier& h, const PcgState* st, double* part, const MgUpd& u)
-{
-    MgHier hh = h;
-    hh.lv[0].b = u.r_new;   // level 0 of this V-cycle: the updated residual
-    hipLaunchKernelGGL(k_pcg_update_mg, dim3(grid_for(h.lv[0].nx * h.lv[0].ny)), dim3(kBlock), 0, s,
-                       h.lv[0].nx * h.lv[0].ny, u);
-    launch_mg_vcycle(s, hh, st, part, nullptr);
+    for (int l = 0; l < lc; ++l) mg_down0(s, h, l, nullptr);
+    hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, h, (const PcgState*)nullptr);
+    for (int l = lc - 1; l >= 0; --l) mg_up0(s, h, l, nullptr);
 }
 
 // The V-cycle below level 0 (down kernels of levels 1 .. lc-1, the single-block kernel, up
@@ -1356,7 +1317,7 @@ static void mg_vcycle_cg1_rest(hipStream_t s, const MgHier& h, const PcgState* s
 {
     const int lc = mg_coarse_level(h);
     for (int l = 1; l < lc; ++l) mg_down0(s, h, l, st);
-    hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, h, st, nullptr, nullptr);
+    hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kMgThreads), 0, s, h, st);
     for (int l = lc - 1; l >= 1; --l) mg_up0(s, h, l, st);
     hipLaunchKernelGGL(k_mg_up<true>, dim3(mg_tiles(h.lv[0])), dim3(mg_tile_threads(kMgHaloA)), 0, s, h.lv[0], h.lv[1],
                        h.lv[0].y, st, part, bb_src, w);

@@ -1,6 +1,7 @@
 """The overland multigrid CG that runs on chip in one workgroup (surfaces whose level 0 has at most one
 2 x 2 aggregate per thread) against the oracle: the exact level alone, one and several smoothed
-levels, odd edges, the largest square it takes and a shape just beyond it (grid-wide form)."""
+levels, odd edges, the largest square it takes and a shape just beyond it (grid-wide form), strips up
+to the longest it takes and one of two rows that goes to the one-workgroup form in memory."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,8 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-8   # m: ponding and heads of every coupled parity case
 
 
-@pytest.mark.parametrize("nx,ny", [(8, 8), (9, 8), (16, 17), (33, 31), (47, 86), (64, 64), (65, 64), (3, 200)])
+@pytest.mark.parametrize("nx,ny", [(8, 8), (9, 8), (16, 17), (33, 31), (47, 86), (64, 64), (65, 64), (3, 200),
+                                   (3, 600), (470, 5), (6, 480), (3, 750), (2, 800)])
 @pytest.mark.parametrize("form", [_abi.OLF_PRECOND_MG])
 def test_small_surfaces_match_oracle(hip, orc, nx, ny, form):
     w = inputs.c2_coupled(nx=nx, ny=ny, nz=3, rain_mm_h=150.0)
