@@ -72,30 +72,38 @@ dh::TileCfg default_tile(const dh::Geo& g)
 
 // Default tile of the column form's SpMV.  A chunk of planes reads z, p_old and K of a plane on either
 // side of it once more, and fills its pipeline anew, so whole columns are best once their tiles fill
-// the chip: 512-cell tiles from about 400 of them (fewest halo cells; 1024 x 1024 x 30 FP32 172 us,
-// 32 x 8 x 30 210; 450 x 450 x 30 FP64 72, 32 x 8 x 10 84), 64 x 4 below (400 x 400 x 30 FP32, 700 of
-// them: 28 us, 350 of 64 x 8: 30, 32 x 8 x 8: 36).  Fewer tiles than that are split into chunks of at
-// least 4 planes for about 850 blocks (333 x 187 x 24 FP64, 282 tiles: 24 / 12 / 8 / 6 / 4 planes 22.7 /
-// 19.5 / 18.6 / 19.9 / 21.2 us; 100 x 90 x 40 FP32, 46 tiles: 40 / 8 / 4 planes 21.9 / 9.4 / 8.0).
-// Rows that 64 columns would pad by an eighth more than 32 take 32 x 8.
+// the chip: 64 x 8 from 400 of them (fewest halo cells; 1024 x 1024 x 30 FP32 172 us, 32 x 8 x 30 210),
+// 64 x 4 below (400 x 400 x 30 FP32, 700 of them: 28 us, 350 of 64 x 8: 30, 32 x 8 x 8: 36).  512 blocks
+// of 64 x 8 are resident at once (two a CU): up to there whole columns (450 x 450 x 30, 456 tiles, FP64 /
+// FP32 70 / 37 us, halves 75 / 39; 500 x 500 x 12, 504 tiles, 27 / 19, halves 33 / 25); a few more would
+// leave a second round nearly empty, so those are halved (512 x 560 x 30, 560 tiles, 97 / 49, whole
+// columns 101 / 53) until there are 567 (576 x 520 x 30, 585 tiles: 107 / 51, halves 102 / 52).  Smaller
+// surfaces are split into chunks of at least 4 planes for about 850 blocks of 256 (333 x 187 x 24 FP64,
+// 282 tiles: 24 / 12 / 8 / 6 / 4 planes 22.7 / 19.5 / 18.6 / 19.9 / 21.2 us; 100 x 90 x 40 FP32, 46 tiles:
+// 40 / 8 / 4 planes 21.9 / 9.4 / 8.0).  Rows that 64 columns would pad by an eighth more than 32 take
+// 32 x 8.
 dh::TileCfg default_zin_tile(const dh::Geo& g)
 {
     const int nx32 = (g.nx + 31) / 32, nx64 = (g.nx + 63) / 64, ny4 = (g.ny + 3) / 4, ny8 = (g.ny + 7) / 8;
     const bool narrow = 2 * nx64 * 8 > nx32 * 9;
     dh::TileCfg t = narrow ? dh::TileCfg{32, 8, g.nz} : dh::TileCfg{64, 8, g.nz};
     int nt = narrow ? nx32 * ny8 : nx64 * ny8;
+    const bool resident = !narrow && nt >= 400 && nt <= 512;
     if (!narrow && nt < 400) {
         t.ty = 4;
         nt = nx64 * ny4;
     }
     if (nx32 * ny8 > dh::kMaxBlocks) return dh::TileCfg{0, 0, 0};   // as the other kernels' default
-    const int nkz = std::max(1, (850 + nt / 2) / nt);
+    const int nkz = resident ? 1 : std::max(1, (850 + nt / 2) / nt);
     t.kc = std::min(g.nz, std::max(4, (g.nz + nkz - 1) / nkz));
     return t;
 }
 
-// Default tile of the one-kernel PCG's start-up, for about 1300 blocks: at 400 x 400 x 30 in FP64 650 /
-// 1300 / 1950 / 2600 blocks of 32 x 8 took 55 / 44 / 45 / 62 us (chunks as above).
+// Default tile of the one-kernel PCG's start-up, for about 1300 blocks of 32 x 8 (chunks as above):
+// 400 x 400 x 30 650 / 1300 / 1950 / 2600 blocks 56 / 45 / 45 / 61 us in FP64, 59 / 45 / 41 / 55 in FP32;
+// 333 x 187 x 24 528 / 1320 / 1584 / 2112 blocks 23 / 22 / 22 / 32 and 26 / 22 / 22 / 28; 64 x 48 x 20 12 /
+// 240 blocks (a plane each) 25 / 7.  Many planes on few tiles would want fewer, longer chunks:
+// 150 x 97 x 40 650 / 1300 / 2600 blocks 14 / 18 / 31 us.
 dh::TileCfg default_start_tile(const dh::Geo& g)
 {
     dh::TileCfg t = default_tile(g);

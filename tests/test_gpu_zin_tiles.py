@@ -31,3 +31,13 @@ def test_column_spmv_tiles(hip, orc, shape, tile):
         assert np.max(np.abs(g.download("PSI") - o.download("PSI"))) <= 1e-8
         assert sg["picard_iters"] == so["picard_iters"]
         assert abs(sg["lin_iters"] - so["lin_iters"]) <= sg["picard_iters"]
+
+
+def test_default_takes_whole_columns_while_they_are_resident(hip):
+    """64 x 8 tiles: 504 (resident at once) keep their columns whole, 560 (a second round nearly
+    empty) are halved."""
+    for nx, ny, kc in ((500, 500, 12), (512, 560, 6)):
+        m = hip.FlowModel(_abi.Grid(nx=nx, ny=ny, nz=12, nroot_groups=1, dx=1.0, dy=1.0, dz=0.05),
+                          _abi.default_params(precond=_abi.PRECOND_COLUMN))
+        assert m.get_tile(8) == (64, 8, kc)
+        m.close()
