@@ -1688,17 +1688,22 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
         dh::launch_cast_f32(c->s, c->N, c->D, c->D32);
         dh::launch_cast_f32(c->s, c->N, c->r, c->r32);
     }
-    // scratch solve state: it >= 1 reads (rz, rr) partials = 1, rz[0] = rz[1] = 1, tol2 = -1
+    // scratch solve state: it >= 1 reads partials = 1, rz[0] = rz[1] = 1, tol2 = -1.  All five of the
+    // one-kernel PCG's are set: a zero (w, u) would end the scratch solve and leave empty launches.
     dh::PcgState tune{};
     tune.rz[0] = tune.rz[1] = 1.0;
     tune.tol2 = -1.0;
+    constexpr int kRows = 5;
     dh::PcgState* st = nullptr;
     int rc = dalloc(c, &st, 1);
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(st, &tune, sizeof(tune), hipMemcpyHostToDevice, c->s));
-    std::vector<double> ones(2 * dh::kMaxBlocks, 1.0);
-    HIPCHK(c, hipMemcpyAsync(c->part[0], ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice, c->s));
-    HIPCHK(c, hipStreamSynchronize(c->s));
+    static_assert(kRows <= dh::kMaxSums);
+    const std::vector<double> ones(kRows * dh::kMaxBlocks, 1.0);
+    auto set_partials = [&]() -> int {
+        HIPCHK(c, hipMemcpyAsync(c->part[0], ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice, c->s));
+        return sync_stream(c);
+    };
     const int shapes[5][2] = {{32, 8}, {64, 4}, {16, 16}, {32, 4}, {64, 8}};
     std::vector<int> kcs = {c->g.nz, (c->g.nz + 1) / 2, (c->g.nz + 2) / 3, (c->g.nz + 3) / 4, 8, 4};
     const uint8_t* fl = has_dirichlet(c) ? c->flags : nullptr;
@@ -1708,6 +1713,7 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
     double best[2] = {0.0, 0.0};
     for (int e = 0; e < 2; ++e) {
         if (e == 1 && !mixed) continue;
+        if ((rc = set_partials())) return rc;   // (the assembly writes its own)
         float best_t = 1e30f;
         dh::TileCfg best_cfg{0, 0, 0};
         auto consider = [&](const dh::TileCfg& t) -> int {
@@ -1764,6 +1770,7 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
     // one-kernel PCG: tile shape x planes per chunk x grid cap, on scratch output buffers
     if (c->p.krylov == DHARA_KRYLOV_ONE_KERNEL && !fl && !zin) {
         HIPCHK(c, hipMemcpyAsync(st, &tune, sizeof(tune), hipMemcpyHostToDevice, c->s));
+        if ((rc = set_partials())) return rc;
         const size_t N = c->N;
         void *xs = nullptr, *rs = nullptr, *ps = nullptr;
         HIPCHK(c, hipMalloc(&xs, N * 8));

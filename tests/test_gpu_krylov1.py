@@ -138,3 +138,15 @@ def test_one_kernel_autotune_then_parity(hip, orc):
     g2 = model(hip, w, _abi.KRYLOV_ONE_KERNEL, precision=_abi.MIXED)
     assert g2.get_krylov_tile(4) == gm.get_krylov_tile(4)
     assert g2.get_krylov_tile(8) == gm.get_krylov_tile(8)
+
+
+@pytest.mark.parametrize("prec", [_abi.FP64, _abi.MIXED])
+def test_autotune_of_a_fresh_context_times_full_iterations(hip, prec):
+    """Before any step too, a timed launch is a whole iteration: no faster than its 8 arrays at 8 TB/s."""
+    w = inputs.c2_coupled(nx=400, ny=300, nz=30, precision=prec)
+    gm = model(hip, w, _abi.KRYLOV_ONE_KERNEL, precision=prec)
+    us = gm.autotune()
+    n = 400 * 300 * 30
+    print("autotune:", us, gm.get_krylov_tile(8), gm.get_krylov_tile(4), flush=True)
+    assert us[0] >= n * 8 * 8 / 8e6
+    assert prec == _abi.FP64 or us[1] >= n * 8 * 4 / 8e6
