@@ -32,8 +32,8 @@ namespace {
 
 struct TuneKey {
     int nx, ny, nz, elem;
-    int kind;   // 0: SpMV kernel of the two-kernel PCG, 1: one-kernel PCG, 2: assembly (FP64
-                // tile of the mixed column-preconditioned path, whose only FP64 tiled kernel it is)
+    int kind;   // 0: SpMV kernel of the two-kernel PCG, 1: one-kernel PCG, 2: assembly (where no
+                // SpMV runs on its tile, own_assembly), 3: SpMV of the column form
     bool operator==(const TuneKey& o) const
     {
         return nx == o.nx && ny == o.ny && nz == o.nz && elem == o.elem && kind == o.kind;
@@ -56,6 +56,13 @@ void remember_tile(const TuneKey& key, const dh::TileCfg& cfg)
 bool mixed_column(const dhara_params* p)
 {
     return p->precision == DHARA_MIXED && p->precond == DHARA_PRECOND_COLUMN;
+}
+
+// Forms whose `tile[0]` serves the assembly (and the refinement), no SpMV: mixed precision with the
+// column preconditioner and the one-kernel PCG.
+bool own_assembly(const dhara_params* p)
+{
+    return p->precond == DHARA_PRECOND_COLUMN ? p->precision == DHARA_MIXED : p->krylov == DHARA_KRYLOV_ONE_KERNEL;
 }
 
 // Default tile: 32 x 8 columns (128 B rows in FP32), planes per block chosen for ~2048 blocks.
@@ -1323,10 +1330,12 @@ int dhara_create(const dhara_grid* grid, const dhara_params* params, dhara_ctx**
         c->start_tile[e] = default_start_tile(g);
         c->cg1_tile[e] = dh::TileCfg{32, 8, dh::cg1_default_planes(g), 0};
         if (dh::cg1_blocks(g, c->cg1_tile[e]) > dh::kMaxBlocks) c->cg1_tile[e].grid = dh::kMaxBlocks;   // blocks loop
-        const int tkind = (e == 0 && mixed_column(params)) ? 2 : 0;
+        const int tkind = (e == 0 && own_assembly(params)) ? 2 : 0;
         for (const TuneEntry& te : g_tune_table) {
-            if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, tkind}) use_tile(c, e, te.cfg);
-            if (te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, 1}) {
+            const auto is = [&](int kind) { return te.key == TuneKey{g.nx, g.ny, g.nz, e == 0 ? 8 : 4, kind}; };
+            if (is(tkind)) c->tile[e] = te.cfg;
+            if (is(3)) c->zin_tile[e] = te.cfg;
+            if (is(1)) {
                 c->cg1_tile[e] = te.cfg;
                 c->cg1_set[e] = true;
             }
@@ -1709,11 +1718,14 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
     const uint8_t* fl = has_dirichlet(c) ? c->flags : nullptr;
     // the column-preconditioned PCG runs the SpMV kernel that reads z (= r here)
     const bool zin = c->p.precond == DHARA_PRECOND_COLUMN && !fl && dh::line_supported(c->g);
-    const bool asm_tune = zin && mixed;   // FP64 tile: time the assembly, its one user here
+    // A tile is timed on the kernel that runs on it, and no other kernel's tile changes.
+    const bool one = c->p.krylov == DHARA_KRYLOV_ONE_KERNEL && !fl && !zin;
+    const bool asm_tune = one || (zin && mixed);
     double best[2] = {0.0, 0.0};
     for (int e = 0; e < 2; ++e) {
-        if (e == 1 && !mixed) continue;
-        if ((rc = set_partials())) return rc;   // (the assembly writes its own)
+        if (e == 1 && (!mixed || one)) continue;   // (one: no FP32 kernel on this tile)
+        if ((rc = set_partials())) return rc;      // (the assembly writes its own)
+        dh::TileCfg& tile = zin && !(e == 0 && asm_tune) ? c->zin_tile[e] : c->tile[e];
         float best_t = 1e30f;
         dh::TileCfg best_cfg{0, 0, 0};
         auto consider = [&](const dh::TileCfg& t) -> int {
@@ -1729,7 +1741,7 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
                 // the assembly rewrites D, b, D32, r32, d32 and the free-drainage flux from the
                 // state, as the next Picard iteration does anyway
                 r2 = time_spmv<double>(c, [&](int) {
-                    dh::launch_assemble_tiled(c->s, asm_args(c, false), true, t);
+                    dh::launch_assemble_tiled(c->s, asm_args(c, false), mixed, t);
                 }, &us);
             } else if (e == 0) {
                 double* const pp[2] = {c->pv[0], c->pv[1]};
@@ -1756,6 +1768,7 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
             if (us < 0.97f * best_t || best_t >= 1e29f) { best_t = us; best_cfg = t; }
             return DHARA_OK;
         };
+        if ((rc = consider(tile))) return rc;   // the tile in use (the default's) first: it stays unless beaten
         for (const auto& sh : shapes)
             for (int kc : kcs) {
                 dh::TileCfg t{sh[0], sh[1], std::max(1, std::min(kc, c->g.nz))};
@@ -1763,12 +1776,13 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
                 if ((rc = consider(t))) return rc;
             }
         if ((rc = consider(dh::TileCfg{0, 0, 0}))) return rc;
-        use_tile(c, e, best_cfg);
+        tile = best_cfg;
         best[e] = best_t;
-        remember_tile(TuneKey{c->g.nx, c->g.ny, c->g.nz, e == 0 ? 8 : 4, (e == 0 && asm_tune) ? 2 : 0}, best_cfg);
+        const int kind = (e == 0 && asm_tune) ? 2 : zin ? 3 : 0;
+        remember_tile(TuneKey{c->g.nx, c->g.ny, c->g.nz, e == 0 ? 8 : 4, kind}, best_cfg);
     }
     // one-kernel PCG: tile shape x planes per chunk x grid cap, on scratch output buffers
-    if (c->p.krylov == DHARA_KRYLOV_ONE_KERNEL && !fl && !zin) {
+    if (one) {
         HIPCHK(c, hipMemcpyAsync(st, &tune, sizeof(tune), hipMemcpyHostToDevice, c->s));
         if ((rc = set_partials())) return rc;
         const size_t N = c->N;
@@ -1785,39 +1799,41 @@ int dhara_autotune(dhara_ctx* c, double* best_us)
             if (e == 1 && !mixed) continue;
             float best_t = 1e30f;
             dh::TileCfg best_cfg = c->cg1_tile[e];
+            std::vector<dh::TileCfg> cand{c->cg1_tile[e]};   // the tile in use (the default's) first
             for (const auto& sh : cshapes)
                 for (int kc : ckcs)
                     for (int gcap : grids) {
-                        dh::TileCfg t{sh[0], sh[1], std::max(1, kc), gcap};
-                        const int nt = dh::tile_blocks(c->g, t);
-                        if (gcap != 0 && gcap >= nt) continue;   // same launch as gcap = 0
-                        if (dh::cg1_blocks(c->g, t) > dh::kMaxBlocks) continue;
-                        dh::SolveCtl sc{};
-                        sc.maxit = 1 << 30;
-                        sc.part_in = c->part[0];
-                        sc.nparts = dh::grid_for(c->N);
-                        sc.part_out = c->part[1];
-                        sc.st = st;
-                        float us = 0.f;
-                        if (e == 0)
-                            rc2 = time_spmv<double>(c, [&](int it) {
-                                dh::SolveCtl k = sc;
-                                k.it = it;
-                                dh::launch_cg1_f64(c->s, c->g, t, c->K, c->D, c->r, (double*)rs, c->pv[0],
-                                                   (double*)ps, (double*)xs, k);
-                            }, &us);
-                        else
-                            rc2 = time_spmv<float>(c, [&](int it) {
-                                dh::SolveCtl k = sc;
-                                k.it = it;
-                                dh::launch_cg1_f32(c->s, c->g, t, c->K32, c->D32, c->r32, (float*)rs, c->p32[0],
-                                                   (float*)ps, (float*)xs, k);
-                            }, &us);
-                        if (rc2) break;
-                        // a later candidate must be 3 % faster: ties keep the first (whole columns, one
-                        // block per tile), so the choice is stable from run to run
-                        if (us < 0.97f * best_t || best_t >= 1e29f) { best_t = us; best_cfg = t; }
+                        const dh::TileCfg t{sh[0], sh[1], std::max(1, kc), gcap};
+                        if (gcap != 0 && gcap >= dh::tile_blocks(c->g, t)) continue;   // same launch as gcap = 0
+                        if (dh::cg1_blocks(c->g, t) <= dh::kMaxBlocks) cand.push_back(t);
                     }
+            for (const dh::TileCfg& t : cand) {
+                dh::SolveCtl sc{};
+                sc.maxit = 1 << 30;
+                sc.part_in = c->part[0];
+                sc.nparts = dh::grid_for(c->N);
+                sc.part_out = c->part[1];
+                sc.st = st;
+                float us = 0.f;
+                if (e == 0)
+                    rc2 = time_spmv<double>(c, [&](int it) {
+                        dh::SolveCtl k = sc;
+                        k.it = it;
+                        dh::launch_cg1_f64(c->s, c->g, t, c->K, c->D, c->r, (double*)rs, c->pv[0], (double*)ps,
+                                           (double*)xs, k);
+                    }, &us);
+                else
+                    rc2 = time_spmv<float>(c, [&](int it) {
+                        dh::SolveCtl k = sc;
+                        k.it = it;
+                        dh::launch_cg1_f32(c->s, c->g, t, c->K32, c->D32, c->r32, (float*)rs, c->p32[0], (float*)ps,
+                                           (float*)xs, k);
+                    }, &us);
+                if (rc2) break;
+                // a later candidate must be 3 % faster: ties keep the first, so the choice is stable
+                // from run to run
+                if (us < 0.97f * best_t || best_t >= 1e29f) { best_t = us; best_cfg = t; }
+            }
             c->cg1_tile[e] = best_cfg;
             c->cg1_set[e] = true;
             best[e] = best_t;

@@ -85,8 +85,8 @@ struct dhara_ctx {
     dhara_ctx() { std::fill(pcg_hints, pcg_hints + kHints, 8); }
     int& pcg_hint() { return pcg_hints[std::min(picard_it, kHints - 1)]; }
     std::vector<void*> allocs;
-    // Tile shapes: [0] FP64, [1] FP32 (tx = 0: untiled kernels).  A tile that the caller or the autotuner
-    // chose is all three; the defaults differ.
+    // Tile shapes: [0] FP64, [1] FP32 (tx = 0: untiled kernels).  A tile that the caller sets is all three;
+    // the defaults differ, and the autotuner sets the one that it timed.
     dh::TileCfg tile[2] = {{32, 8, 0}, {32, 8, 0}};         // assembly, refinement, two-kernel SpMV
     dh::TileCfg zin_tile[2] = {{32, 8, 0}, {32, 8, 0}};     // SpMV of the column form
     dh::TileCfg start_tile[2] = {{32, 8, 0}, {32, 8, 0}};   // start-up of the one-kernel PCG

@@ -150,3 +150,19 @@ def test_autotune_of_a_fresh_context_times_full_iterations(hip, prec):
     print("autotune:", us, gm.get_krylov_tile(8), gm.get_krylov_tile(4), flush=True)
     assert us[0] >= n * 8 * 8 / 8e6
     assert prec == _abi.FP64 or us[1] >= n * 8 * 4 / 8e6
+
+
+def test_autotune_keeps_the_defaults_that_it_does_not_beat(hip):
+    """A small surface's default splits its columns finer than any fixed candidate (whole, halves,
+    thirds: 7 planes of 20) and is faster by a third; and a tile timed in one form of the solver is
+    not taken over by another kernel in a later context of the same grid."""
+    w = inputs.c2_coupled(nx=64, ny=47, nz=20)
+    before = model(hip, w, _abi.KRYLOV_TWO_KERNEL).get_tile(8)
+    col = model(hip, w, _abi.KRYLOV_ONE_KERNEL, precond=_abi.PRECOND_COLUMN)
+    col.set_tile(8, 64, 8, 13)          # in use, so a candidate
+    col.autotune()
+    assert model(hip, w, _abi.KRYLOV_TWO_KERNEL).get_tile(8) == before
+    one = model(hip, w, _abi.KRYLOV_ONE_KERNEL)
+    one.step(1)
+    one.autotune()
+    assert one.get_krylov_tile(8)[2] < 7
