@@ -1149,9 +1149,11 @@ int dhara_ensemble_autotune(dhara_ensemble* e, double* best_us, int32_t* planes_
     EHIP(e, hipEventCreate(&e0));
     EHIP(e, hipEventCreate(&e1));
     const int old_div = e->kc_div;
-    float best = 1e30f;
-    int best_div = 1;
-    for (int div : {1, 2, 3}) {
+    // 0: the members' own tiles, which split a small ensemble's columns finer than any policy; they stay
+    // unless a policy is 3 % faster
+    float best = 1e30f, best_policy = 1e30f;
+    int keep = 0, best_div = 1;
+    for (int div : {0, 1, 2, 3}) {
         std::vector<dh::BlkMap> map;
         if ((rc = c1_map(e, div, map))) break;
         e->kc_div = div;
@@ -1182,16 +1184,17 @@ int dhara_ensemble_autotune(dhara_ensemble* e, double* best_us, int32_t* planes_
         EHIP(e, hipGetLastError());
         EHIP(e, hipEventElapsedTime(&ms, e0, e1));
         const float us = ms * 1e3f / 10.f;
-        if (us < 0.97f * best || best >= 1e29f) { best = us; best_div = div; }
+        if (us < 0.97f * best || best >= 1e29f) { best = us; keep = div; }
+        if (div > 0 && (us < 0.97f * best_policy || best_policy >= 1e29f)) { best_policy = us; best_div = div; }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     cleanup();
     if (rc) { e->kc_div = old_div; return rc; }
     // keep the winner: its tile map (the solves rebuild their arguments from the members)
-    e->kc_div = best_div;
+    e->kc_div = keep;
     std::vector<dh::BlkMap> map;
-    if ((rc = c1_map(e, best_div, map)) || (rc = upload(e, e->map_c1, map))) return rc;
+    if ((rc = c1_map(e, keep, map)) || (rc = upload(e, e->map_c1, map))) return rc;
     e->nb_c1 = (int)map.size();
     drop_graphs(e, true);   // their launches carry the old grid size: captured again at the next solve
     if (best_us) *best_us = best;
