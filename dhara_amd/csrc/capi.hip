@@ -730,7 +730,7 @@ int solve_mixed_line(dhara_ctx* c, dhara_step_stats* st)
     for (;;) {
         const int seg = it;
         rc = run_krylov_then(
-            c, c->st_sub, maxit, c->pcg_hint(), c->prof, 4.0,
+            c, c->st_sub, maxit, updates ? c->seg_hint : c->pcg_hint(), c->prof, 4.0,
             [&](int j, const dh::LaunchEv& ev) {
                 dh::SolveCtl k = sc;
                 k.it = j;
