@@ -1,6 +1,7 @@
-"""The Anderson pass's ring on the GPU against the oracle: depths 1 to the largest, a step long enough
-to wrap the ring, columns shorter and longer than the planes it keeps on chip, widths that are not a
-multiple of its 16 or 64 columns, surfaces on both sides of the rule between these two."""
+"""The Anderson pass's ring on the GPU against the oracle: depths 1 to the largest, each with a case whose
+steps wrap the ring (depth 5: 14 passes of the 45-plane case), columns shorter and longer than the
+planes it keeps on chip, widths that are not a multiple of its 16 or 64 columns, surfaces on both sides
+of the rule between these two."""
 import numpy as np
 import pytest
 
@@ -10,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shape,depth", [((9, 7, 5), 1), ((13, 11, 32), 2), ((16, 8, 33), 3), ((11, 7, 45), 4),
-                                         ((10, 13, 30), 5), ((129, 127, 3), 3), ((129, 128, 3), 3)])
+                                         ((10, 13, 30), 5), ((12, 9, 45), 5), ((129, 127, 3), 3), ((129, 128, 3), 3)])
 def test_ring_matches_oracle(hip, orc, shape, depth):
     w = inputs.c2_coupled(*shape)
     p = _abi.Params.from_buffer_copy(w.params)

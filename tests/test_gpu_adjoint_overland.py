@@ -1,5 +1,5 @@
 """Reverse overland solve in its two forms (one-workgroup multigrid CG; Jacobi-CG) over surfaces from
-one inner cell's neighbourhood to the largest that fits one workgroup and the first that does not: the
+3 x 2 inner cells to the largest square that fits one workgroup and the first size that does not: the
 gradients of a run with outlet discharge agree to the forward's and reverse's tolerances (1e-14, 1e-12)
 times the conditioning: 1e-6 of the largest entry, the bound of the oracle parity test."""
 import numpy as np
@@ -13,7 +13,7 @@ from test_oracle_adjoint import small_workload
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny", [(5, 4), (17, 9), (33, 64), (64, 64), (65, 40)])
+@pytest.mark.parametrize("nx,ny", [(5, 4), (17, 9), (33, 64), (64, 64), (65, 40), (65, 64)])
 def test_gradient_of_both_overland_forms(nx, ny):
     grads = []
     steps = 6

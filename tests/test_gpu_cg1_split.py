@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 HEAD_TOL = 1e-8   # m, as for every FP64 parity case (solves end at ||r|| <= 1e-12 ||b||)
 
 
-# (nx, ny, nz): one tile; 4 tiles of 7 planes (one plane a block); 66 tiles of 13 planes (6 chunks of
-# 3, the last of 1); 209 tiles (one chunk)
+# (nx, ny, nz): one tile; 4 tiles of 7 planes (one plane a block); 66 tiles of 13 planes (chunks of 3,
+# the last of 1); 209 tiles (one chunk)
 @pytest.mark.parametrize("shape", [(7, 5, 3), (33, 9, 7), (161, 88, 13), (333, 152, 4)])
 @pytest.mark.parametrize("prec", [_abi.FP64, _abi.MIXED])
 def test_default_split_matches_oracle(hip, orc, shape, prec):
@@ -38,7 +38,7 @@ def test_full_ensemble_matches_members_alone():
         m = dhara_amd.FlowModel(w.grid, _abi.Params.from_buffer_copy(w.params))
         w.apply(m)
         return m
-    ms = [make(s) for s in spec]   # 12 x 40 whole-column tiles: beyond the line
+    ms = [make(s) for s in spec]   # 464 whole-column tiles: beyond the line
     st = dhara_amd.Ensemble(ms).step(2)
     for i in (0, 11):
         alone = make(spec[i])
