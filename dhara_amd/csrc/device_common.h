@@ -81,8 +81,9 @@ __device__ __forceinline__ double vg_inverse(double theta, double alpha, double 
 // ---- reductions ---------------------------------------------------------------------------
 // No kernel communicates across blocks: a producer kernel writes one partial per block with a
 // plain store, and the consumer -- the next kernel, after the kernel boundary has made the
-// stores visible on every XCD, or the host -- sums the partials in block order.  Every
-// consuming block runs the same fixed-order sum, so all of them see identical totals and the
+// stores visible on every XCD; what the host reads is such a kernel's sum -- adds the partials in a
+// fixed order (a thread strides over them, then the block's reduction).  Every consuming block
+// runs the same sum, so all of them see identical totals and the
 // result does not depend on scheduling.  (A last-block-done reduction would need an
 // agent-scope release fence per block, i.e. an L2 writeback per block on a multi-XCD part.)
 __device__ __forceinline__ int lin_tid() { return threadIdx.x + threadIdx.y * blockDim.x; }

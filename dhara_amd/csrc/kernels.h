@@ -93,7 +93,7 @@ struct VgArgs {
     double am;
     int relax;               // Picard pass: 1 = write the relaxed update into psi_m (0: an
                              // Anderson pass follows and needs psi_m as it is)
-    double* part_out;        // Picard pass: [max increment, NaN flag] per block (host-reduced)
+    double* part_out;        // Picard pass: [max increment, NaN flag] per block
 };
 
 // Anderson-accelerated Picard update (k_picard_next).  The increment f = x - psi^m and relaxed
@@ -218,7 +218,7 @@ struct EndArgs {
     int carry_reference;
     const int* bctype[6];
     const double* bcq[6];
-    double* part_out;        // 9 sums per block (host-reduced)
+    double* part_out;        // 9 sums per block
 };
 
 struct OlfArgs {

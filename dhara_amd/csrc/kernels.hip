@@ -2,8 +2,8 @@
 // wave) solvers.  Every kernel is grid-stride over cells in the reference layout
 // (k*nx*ny + j*nx + i, k = 0 top) and keeps per-cell state in HBM as SoA arrays.
 //
-// Reductions: every kernel writes one partial per block; the next kernel (or the host) sums
-// them in block order (device_common.h).  The Krylov kernels read PcgState::done at entry and
+// Reductions: every kernel writes one partial per block; the next kernel sums them in a fixed order
+// (device_common.h).  The Krylov kernels read PcgState::done at entry and
 // return at once when the solve has finished, so the host can queue iterations in batches
 // without a round trip per iteration.
 #include <hip/hip_ext.h>
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kBlock) void k_vg_picard(VgArgs a, Gate gate)
 // The ring holds f and y themselves and not their differences: with a full ring of 3 a pass moves
 // 5 + 2 + 4 + 4 arrays (124 B per cell with K32) instead of 160 B, with the same differences.
 // Bytes bound it on large surfaces: 118 us a launch at 400 x 400 x 30 (672 MB / 130 us with the
-// differences stored), 750 us at 1024 x 1024 x 30 (909 us).  A surface of few columns is bound by the
+// differences stored), 775 us at 1024 x 1024 x 30 (909 us).  A surface of few columns is bound by the
 // chain of van Genuchten evaluations of a thread (about 1.7 us each, 515 dependent FP64 operations)
 // on the few CUs that its blocks reach: COLS = 16 columns per block spread it over four times the CUs
 // and four times the threads in pass 2; pass 1 keeps the four chunks, so the sums are the same
@@ -999,6 +999,22 @@ __device__ __forceinline__ double jac_inv(double d)
     return fma(y, fma(-d, y, 1.0), y);
 }
 
+// A copy of a slot's value in a register of its own.  A loop that keeps the loads of the next planes in
+// flight reuses the slot's registers for the next load; a value that is still needed then must not
+// share them, or the new load goes elsewhere and a move at the end of the loop waits for it.
+__device__ __forceinline__ float take(float v)
+{
+    float r;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+__device__ __forceinline__ double take(double v)
+{
+    double r;
+    asm volatile("v_mov_b64 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
 // Column (vertical line) preconditioner: z = T^-1 r with T the vertical tridiagonal part of the
 // 7-point operator -- diagonal D, coupling to the cell above / below -(wz/2)(K_k + K_k-+1), as
 // in the SpMV --, i.e. one independent tridiagonal system per column of cells, solved by the
@@ -1021,30 +1037,19 @@ __device__ __forceinline__ double jac_inv(double d)
 // the loads of A planes are in flight ahead of the plane in work, in registers.  y_k of every plane
 // waits in LDS, and so does c'_k in FP32; in FP64 c'_k waits in z itself (written in the forward
 // sweep, read back A planes ahead of the substitution, overwritten by it): 8 B per plane and thread
-// in both, two blocks per CU up to 40 planes.  With y in registers instead (arrays of 16, 32 or 64
-// planes, unrolled) each plane waited for its own loads, since a plane that may not exist ends the
-// unrolled block, and the batched form needed a launch per array size.  Working launches, registers
-// -> LDS: update FP64 333 x 187 x 24 30 -> 24 us (131 MB), 300 x 300 x 40 87 -> 62 us, 450 x 450 x 30
-// 126 -> 106 us, 800 x 800 x 30 316 -> 294 us (bytes); FP32 150 x 150 x 40 26 -> 13 us, 450 x 450 x 30
-// 55 -> 48 us, 1024 x 1024 x 30 232 -> 223 us, 400 x 400 x 30 34.6 -> 36.7 us (1.2 rounds of resident
-// blocks), 800 x 800 x 12 49 -> 52 us; start-up FP64 333 x 187 x 24 24 -> 17 us; 20 models of
-// 32..128 x 32..128 x 10..40 in FP64, all iterating: 95 us in three launches -> 50 us in one.
-// A copy of a slot's value in a register of its own.  A loop that keeps the loads of the next planes in
-// flight reuses the slot's registers for the next load; a value that is still needed then must not
-// share them, or the new load goes elsewhere and a move at the end of the loop waits for it.
-__device__ __forceinline__ float take(float v)
-{
-    float r;
-    asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
-    return r;
-}
-__device__ __forceinline__ double take(double v)
-{
-    double r;
-    asm volatile("v_mov_b64 %0, %1" : "=v"(r) : "v"(v));
-    return r;
-}
-
+// in both, two blocks per CU up to 39 planes (the reductions' LDS comes on top; with that folded into
+// the same array 40 planes fit twice and 300 x 300 x 40 took the same 57 us).  With y in registers
+// instead (arrays of 16, 32 or 64 planes, unrolled) each plane waited for its own loads, since a plane
+// that may not exist ends the unrolled block, and the batched form needed a launch per array size.
+// Working launches, registers -> LDS: update FP64 333 x 187 x 24 30 -> 24 us (131 MB), 300 x 300 x 40
+// 94 -> 57 us, 450 x 450 x 30 126 -> 106 us, 500 x 500 x 30 125 -> 107 us, 800 x 800 x 30 316 -> 294 us
+// (bytes); FP32 150 x 150 x 40 26 -> 13 us, 450 x 450 x 30 55 -> 48 us, 1024 x 1024 x 30 232 -> 223 us,
+// 400 x 400 x 30 37.0 -> 36.4 us (1.2 rounds of resident blocks), 800 x 800 x 12 51.7 -> 50.4 us; start-up
+// FP64 333 x 187 x 24 24 -> 17 us, 300 x 300 x 40 45 -> 39 us, FP32 800 x 800 x 12 44 -> 40 us, but
+// 400 x 400 x 30 26 -> 29 us (the 1.2 rounds).  In a batched launch the tallest member sets every
+// block's LDS: still less time than a launch per array size (20 models of 32..128 x 32..128 x 10..40 in
+// FP64, all iterating, 95 -> 50 us; 40 models of 12 planes and one of 64, all launches of six steps,
+// FP64 10.5 -> 7.9 ms, FP32 9.7 -> 7.9).
 template <typename T>
 struct LinePlane {
     T r, q, p, x, K, D;
